@@ -4,7 +4,8 @@
  * For the single-vector canonical kernel it sweeps workgroup size, workgroups
  * per CU, list_2_1 in LDS or L2, and the XCD-contiguous tile mapping; for the
  * block kernel (k > 1) it sweeps columns per lane, workgroup size, workgroups
- * per CU and the XCD mapping; the per-column kernel is always a candidate.  Each candidate is timed with HIP events over `reps` H·v calls on
+ * per CU and the XCD mapping; the per-column kernel is always a candidate, and
+ * the grand-canonical tiles where the sector has them.  Each candidate is timed with HIP events over `reps` H·v calls on
  * the caller's vectors (v0 accumulates: the caller re-initialises it), and
  * the fastest is left set on the engine.  A one-line report per candidate is
  * written to `report` when it is non-NULL.
@@ -39,7 +40,7 @@ int hphi_autotune(hphi_engine *e, int k, double *v0, const double *v1, int reps,
   if (!e || !v0 || !v1) return hphi_set_error("hphi_autotune: NULL argument");
   if (reps < 1) reps = 2;
   cand_t cands[96];
-  int n = 0, c2 = 0, blk = 0, lds_ok = 0, crank_ok = 0;
+  int n = 0, c2 = 0, blk = 0, lds_ok = 0, crank_ok = 0, gc = 0;
   memset(cands, 0, sizeof cands);
   if (k == 1 && hphi_engine_get_tune(e, "use_c2", &c2) == 0 && c2) {
     /* is list_2_1 allowed in LDS for this model? */
@@ -76,6 +77,11 @@ int hphi_autotune(hphi_engine *e, int k, double *v0, const double *v1, int reps,
       }
     }
   }
+  hphi_engine_get_tune(e, "gc_tile", &gc);
+  if (gc) { /* grand-canonical tiles: one shape; every later candidate turns them off */
+    cand_t *c = &cands[n++];
+    add(c, "gc_tile", 1), add(c, "use_blk", 1);
+  }
   if (k > 1 && hphi_engine_get_tune(e, "use_blk", &blk) == 0 && blk) {
     /* block kernel: columns per lane x workgroup size x workgroups per CU x XCD map */
     static char knob[16];
@@ -89,11 +95,13 @@ int hphi_autotune(hphi_engine *e, int k, double *v0, const double *v1, int reps,
           cand_t *c = &cands[n++];
           add(c, "use_blk", 1), add(c, "xcd_map", xcd), add(c, knob, cpls[a]);
           add(c, "blk_tpb", 256), add(c, "blk_wgs_per_cu", w);
+          if (gc) add(c, "gc_tile", 0);
         }
         if (cpls[a] <= 4) {
           cand_t *c = &cands[n++];
           add(c, "use_blk", 1), add(c, "xcd_map", xcd), add(c, knob, cpls[a]);
           add(c, "blk_tpb", 1024), add(c, "blk_wgs_per_cu", 1);
+          if (gc) add(c, "gc_tile", 0);
         }
       }
   }
@@ -101,6 +109,7 @@ int hphi_autotune(hphi_engine *e, int k, double *v0, const double *v1, int reps,
     for (int g = 2; g <= 16; g *= 2) {
       cand_t *c = &cands[n++];
       add(c, "use_c2", 0), add(c, "use_blk", 0), add(c, "xcd_map", xcd), add(c, "grid_per_cu", g);
+      if (gc) add(c, "gc_tile", 0);
     }
 
   double best = 1e300;

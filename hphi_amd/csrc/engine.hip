@@ -924,6 +924,7 @@ extern "C" void hphi_engine_destroy(hphi_engine *e) {
   (void)hipFree(e->d_blkpos);
   (void)hipFree(e->d_v1t);
   (void)hipFree(e->d_tofs);
+  (void)hipFree(e->d_gcterms);
   (void)hipFree(e->d_jb);
   (void)hipFree(e->d_diag);
   (void)hipFree(e->d_terms);
@@ -1008,6 +1009,9 @@ extern "C" int hphi_engine_tune(hphi_engine *e, const char *knob, int value) {
     e->grid_per_cu = value;
   } else if (k == "use_blk") {
     e->use_blk = value ? 1 : 0;
+  } else if (k == "gc_tile") {
+    if (value < -1 || value > 1) return hphi_set_error("gc_tile must be -1, 0 or 1");
+    e->gc_tile = value;
   } else if (k == "lb_mfma") {
     e->lb_mfma = value ? 1 : 0;
   } else if (k == "blk_tpb") {
@@ -1044,6 +1048,8 @@ extern "C" int hphi_engine_get_tune(const hphi_engine *e, const char *knob, int 
   else if (k == "use_c2") *value = e->use_c2 && e->c2_ok;
   else if (k == "grid_per_cu") *value = e->grid_per_cu;
   else if (k == "use_blk") *value = e->use_blk && hphi_blk_ok(e);
+  else if (k == "gc_tile") *value = hphi_gc_wanted(e, 1) || hphi_gc_wanted(e, 2) || hphi_gc_wanted(e, 4) ||
+                                    hphi_gc_wanted(e, 8) || hphi_gc_wanted(e, 16);
   else if (k == "lb_mfma") *value = e->lb_mfma;
   else if (k == "blk_tpb" || k == "blk_wgs_per_cu" || k.rfind("blk_cpl", 0) == 0) {
     int kk = k.rfind("blk_cpl", 0) == 0 ? atoi(k.c_str() + 7) : 16;
@@ -1145,6 +1151,7 @@ int hphi_build_diag(hphi_engine *e) {
                        (int)e->h_dterms.size(), e->d_diag, e->stream))
     return -1;
   HIPCHK(hipStreamSynchronize(e->stream));
+  if (hphi_gc_plan_build(e)) return -1;
   e->diag_ready = true;
   return 0;
 }
@@ -1212,7 +1219,14 @@ int hphi_hv_launch(hphi_engine *e, int k, double *v0, const double *v1) {
   return hphi_hv_launch_ex(e, k, v0, v1, 0);
 }
 
-static int hv_launch_args(hphi_engine *e, int k, HvArgs &A, double2 *prdct_out);
+static int hv_launch_args(hphi_engine *e, int k, HvArgs &A, double2 *prdct_out, int gather = 0);
+
+// V0 = H V1 (overwrite) by the gather kernels, for callers that need their order of summation
+int hphi_hv_launch_gather(hphi_engine *e, int k, double *v0, const double *v1) {
+  HvArgs A = hphi_hv_args(e, k, v0, v1);
+  A.overwrite = 1;
+  return hv_launch_args(e, k, A, (double2 *)e->d_prdct, 1);
+}
 
 int hphi_hv_launch_ex(hphi_engine *e, int k, double *v0, const double *v1, int overwrite) {
   HvArgs A = hphi_hv_args(e, k, v0, v1);
@@ -1222,11 +1236,15 @@ int hphi_hv_launch_ex(hphi_engine *e, int k, double *v0, const double *v1, int o
 
 // which kernel a launch for k columns uses, and its workgroups (each writes k
 // partial sums of prdct)
-enum { HV_PATH_CANON, HV_PATH_BLK, HV_PATH_GENERIC };
-static int hv_path(const hphi_engine *e, int k, int *grid) {
+enum { HV_PATH_CANON, HV_PATH_GC, HV_PATH_BLK, HV_PATH_GENERIC };
+static int hv_path(const hphi_engine *e, int k, int *grid, int gather = 0) {
   if (k == 1 && e->c2_ok && e->use_c2) {
     *grid = canon_grid(e);
     return HV_PATH_CANON;
+  }
+  if (!gather && hphi_gc_wanted(e, k)) {
+    *grid = hphi_gc_partials(e, k);
+    return HV_PATH_GC;
   }
   if (k > 1 && e->use_blk && hphi_blk_ok(e)) {
     *grid = hphi_blk_grid(e, k);
@@ -1239,9 +1257,9 @@ static int hv_path(const hphi_engine *e, int k, int *grid) {
 // launch of prepared arguments: the canonical single-vector kernel, the block
 // kernel, or the generic kernel; then the partials in A.partial are reduced
 // into prdct_out[0..k)
-static int hv_launch_args(hphi_engine *e, int k, HvArgs &A, double2 *prdct_out) {
+static int hv_launch_args(hphi_engine *e, int k, HvArgs &A, double2 *prdct_out, int gather) {
   int g = 0;
-  const int path = hv_path(e, k, &g);
+  const int path = hv_path(e, k, &g, gather);
   if (path == HV_PATH_CANON) {
     // canonical Spin: the high-half terms in a second pass over a tile-major
     // copy of v1 (only with the engine's own partial-sum buffer, which holds
@@ -1259,6 +1277,8 @@ static int hv_launch_args(hphi_engine *e, int k, HvArgs &A, double2 *prdct_out) 
       if (hphi_hv_launch_high(e, A, A.partial + g, &g2)) return -1;
       g += g2;
     }
+  } else if (path == HV_PATH_GC) {
+    if (hphi_hv_launch_gc(e, A, k, &g)) return -1;
   } else if (path == HV_PATH_BLK) {
     int gb = 0;
     if (hphi_hv_launch_blk(e, A, k, &gb)) return -1;

@@ -136,6 +136,29 @@ struct HiPlan {
   uint64_t wgp[HI_MAXC + 1], base[HI_MAXC + 1];
 };
 
+// Grand-canonical H·v in LDS tiles (hv_gc.hip): a pass applies the terms whose
+// flips lie inside its bit set S to the tiles of 2^|S| states.
+struct GcTerm {
+  double cre, cim;
+  uint32_t flow, fe, flip;  // flip in the tile's element index: thread part, element part; in the state
+  uint32_t tmask, tval;     // predicate (tval: the value, or 1 when an even parity passes)
+  uint32_t sgn, sgi, es;    // sign masks of the real and imaginary part; their parities per element
+  int parity, src;
+};
+#define GC_E 8       // elements per thread of k_hv_gc
+#define GC_CASES 15  // parity terms by the element bits of predicate and flip: both m (0..7), or none and f (7 + f)
+#define GC_MAXPASS 8
+struct GcPass {
+  int at = 0, nloc = 0, nother = 0, nrem = 0;  // first term; terms in the tile, those of no case; terms gathered
+  uint32_t count[2][GC_CASES] = {};             // parity terms without and with a sign, by case
+  int nob = 0, nrun = 0;                 // state bits outside S, and the runs they form
+  uint32_t sb[16] = {}, omask[17] = {}, oshl[17] = {}, xe[GC_E] = {};
+};
+struct GcPlan {
+  int npass = 0;
+  GcPass pass[GC_MAXPASS];
+};
+
 struct hphi_engine {
   int model = 0, nsite = 0, nup = 0, ndown = 0, nbits = 0, nlow = 0;
   uint64_t dim = 0, sdim = 0, size21 = 0, size22 = 0, irght = 0, ilft = 0, ihfbit = 0;
@@ -185,6 +208,10 @@ struct hphi_engine {
   double2 *d_v1t = nullptr;      // tile-major copy of v1, hi_plan.base[ncls] elements
   ulonglong2 *d_tofs = nullptr;  // per block: its first tile-major element, and the stride between its tiles
   HiPlan hi_plan{};
+  // grand-canonical H·v in LDS tiles: -1 by size, 0 off, 1 also with a hand-set block shape
+  int gc_tile = -1;
+  GcPlan gc_plan[5];  // block sizes 1, 2, 4, 8, 16
+  GcTerm *d_gcterms = nullptr;
 };
 
 extern "C" int hphi_set_error(const char *fmt, ...);
@@ -192,6 +219,7 @@ int hphi_build_tables(hphi_engine *e);
 int hphi_build_diag(hphi_engine *e);
 int hphi_hv_launch(hphi_engine *e, int k, double *v0, const double *v1);
 int hphi_hv_launch_ex(hphi_engine *e, int k, double *v0, const double *v1, int overwrite);
+int hphi_hv_launch_gather(hphi_engine *e, int k, double *v0, const double *v1);
 int hphi_fetch_prdct(hphi_engine *e, int k, double *prdct);
 int hphi_hv_grid(const hphi_engine *e, int k);
 int hphi_canon_config(hphi_engine *e);
@@ -213,6 +241,10 @@ int hphi_hi_wanted(const hphi_engine *e);
 int hphi_hi_split_on(hphi_engine *e);
 // launches the high-half pass: accumulates into A.v0, partials at partial[0..*grid)
 int hphi_hv_launch_high(hphi_engine *e, const HvArgs &A, double2 *partial, int *grid);
+int hphi_gc_wanted(const hphi_engine *e, int k);
+int hphi_gc_plan_build(hphi_engine *e);
+int hphi_gc_partials(const hphi_engine *e, int k);  // workgroups of all passes of one H·v
+int hphi_hv_launch_gc(hphi_engine *e, const HvArgs &A, int k, int *grid);
 int hphi_blk_ok(const hphi_engine *e);
 int hphi_blk_cpl_ok(int k, int cpl);
 void hphi_blk_shape(const hphi_engine *e, int k, int *cpl, int *tpb, int *wgs_per_cu);

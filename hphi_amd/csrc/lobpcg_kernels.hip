@@ -583,9 +583,13 @@ extern "C" int hphi_lb_store(hphi_lb_ws *ws, uint64_t dim, const double *x, cons
   return 0;
 }
 
-// W = H w (overwrite) for a block of k columns, no prdct read-back
+// W = H w (overwrite) for a block of k columns, no prdct read-back.  By the
+// gather kernels: the subspace matrices hold entries that are rounding alone,
+// whose phases set those of the Ritz vectors, so another order of summation in
+// W would give every returned vector another phase (equally valid, but a
+// restart or a saved file would no longer repeat an earlier run).
 extern "C" int hphi_lb_hv(hphi_engine *e, int k, double *W, const double *w) {
-  return hphi_hv_launch_ex(e, k, W, w, 1);
+  return hphi_hv_launch_gather(e, k, W, w);
 }
 
 extern "C" const double *hphi_lb_diag(hphi_engine *e) { return e->d_diag; }
