@@ -345,27 +345,51 @@ __global__ __launch_bounds__(HV_TPB) void k_hv(const HvArgs A) {
   wg_reduce_store<K>(pre, pim, A.partial);
 }
 
-// deterministic final reduction: out[v] = sum_w partial[w*K + v] in fixed order
-__global__ __launch_bounds__(256) void k_reduce_partials(const double2 *partial, int nblk, int K,
-                                                         double2 *out) {
-  __shared__ double2 s[256];
-  for (int v = 0; v < K; v++) {
-    double re = 0.0, im = 0.0;
-    for (int w = threadIdx.x; w < nblk; w += 256) {
-      re += partial[(uint64_t)w * K + v].x;
-      im += partial[(uint64_t)w * K + v].y;
-    }
-    s[threadIdx.x] = make_double2(re, im);
-    __syncthreads();
-    for (int st = 128; st > 0; st >>= 1) {
-      if (threadIdx.x < st) {
-        s[threadIdx.x].x += s[threadIdx.x + st].x;
-        s[threadIdx.x].y += s[threadIdx.x + st].y;
+// deterministic final reduction: out[v] = sum_w partial[w*K + v] in fixed
+// order, one workgroup per column v.  Latency-bound: with one workgroup of 256
+// threads for all columns it took 110 us after the 8x4 H·v (67,072 partials)
+// and 82 us after a k = 8 block of 12,288 workgroups; eight loads in flight on
+// 1024 threads per column take 33 and 23 us (256 threads up to 2,048 partials:
+// a quarter of the waves to start and join, 0.3 us less on a 50-workgroup call).
+#define RP_U 8
+template <int RP_TPB>
+__global__ __launch_bounds__(RP_TPB) void k_reduce_partials(const double2 *__restrict__ partial, int nblk, int K,
+                                                            double2 *out) {
+  const int v = blockIdx.x;
+  double2 a[RP_U];
+#pragma unroll
+  for (int u = 0; u < RP_U; u++) a[u] = make_double2(0.0, 0.0);
+  for (int w = threadIdx.x; w < nblk; w += RP_TPB * RP_U) {
+#pragma unroll
+    for (int u = 0; u < RP_U; u++) {
+      const int q = w + u * RP_TPB;
+      if (q < nblk) {
+        const double2 p = partial[(uint64_t)q * K + v];
+        a[u].x += p.x;
+        a[u].y += p.y;
       }
-      __syncthreads();
     }
-    if (threadIdx.x == 0) out[v] = s[0];
-    __syncthreads();
+  }
+#pragma unroll
+  for (int u = 1; u < RP_U; u++) {
+    a[0].x += a[u].x;
+    a[0].y += a[u].y;
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    a[0].x += __shfl_xor(a[0].x, off, 64);
+    a[0].y += __shfl_xor(a[0].y, off, 64);
+  }
+  __shared__ double2 s[RP_TPB / 64];
+  if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = a[0];
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double2 r = s[0];
+    for (int w = 1; w < RP_TPB / 64; w++) {
+      r.x += s[w].x;
+      r.y += s[w].y;
+    }
+    out[v] = r;
   }
 }
 
@@ -1302,8 +1326,12 @@ static int hv_launch_args(hphi_engine *e, int k, HvArgs &A, double2 *prdct_out, 
     }
 #undef LAUNCH
   }
-  hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(256), 0, e->stream, (const double2 *)A.partial, g, k,
-                     prdct_out);
+  if (g <= 2048)
+    hipLaunchKernelGGL(k_reduce_partials<256>, dim3(k), dim3(256), 0, e->stream, (const double2 *)A.partial, g, k,
+                       prdct_out);
+  else
+    hipLaunchKernelGGL(k_reduce_partials<1024>, dim3(k), dim3(1024), 0, e->stream, (const double2 *)A.partial, g, k,
+                       prdct_out);
   HIPCHK(hipGetLastError());
   return 0;
 }

@@ -12,6 +12,7 @@
 #include <algorithm>
 #include <cstring>
 
+#include "block_layout.h"
 #include "engine_internal.h"
 #include "hphi_amd.h"
 
@@ -545,39 +546,17 @@ extern "C" int hphi_lb_update(hphi_lb_ws *ws, uint64_t dim, const double *w, dou
   return lb_finish(ws, g, 2 * k, norms2);
 }
 
-// x[j][c] = src[c*dim + j] (k vectors one after another -> state-major block)
-__global__ __launch_bounds__(256) void k_lb_load(const double2 *src, double2 *x, uint64_t dim, int k) {
-  const uint64_t n = dim * (uint64_t)k;
-  for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256) {
-    const uint64_t c = i / dim, j = i % dim;
-    x[j * k + c] = src[i];
-  }
-}
-
-// dst[c*dim + j] = sx_c x[j][c]: the normalised columns, one vector after another
-__global__ __launch_bounds__(256) void k_lb_store(const double2 *x, double2 *dst, uint64_t dim, int k, LbCols cf) {
-  const uint64_t n = dim * (uint64_t)k;
-  for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256) {
-    const uint64_t c = i / dim, j = i % dim;
-    const double2 a = x[j * k + c];
-    const double f = cf.a[c];
-    dst[i] = make_double2(f * a.x, f * a.y);
-  }
-}
-
 extern "C" int hphi_lb_load(hphi_lb_ws *ws, uint64_t dim, const double *src, double *x) {
-  hipLaunchKernelGGL(k_lb_load, dim3(lb_grid(dim * ws->k)), dim3(256), 0, ws->stream, (const double2 *)src,
-                     (double2 *)x, dim, ws->k);
+  block_layout<true>((const double2 *)src, (double2 *)x, dim, ws->k, nullptr, BlScale{}, ws->stream);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(ws->stream));
   return 0;
 }
 
 extern "C" int hphi_lb_store(hphi_lb_ws *ws, uint64_t dim, const double *x, const double *sx, double *dst) {
-  LbCols cf;
-  for (int c = 0; c < 16; c++) cf.a[c] = c < ws->k ? sx[c] : 0.0, cf.b[c] = 0.0;
-  hipLaunchKernelGGL(k_lb_store, dim3(lb_grid(dim * ws->k)), dim3(256), 0, ws->stream, (const double2 *)x,
-                     (double2 *)dst, dim, ws->k, cf);
+  BlScale cf;
+  for (int c = 0; c < 16; c++) cf.f[c] = c < ws->k ? sx[c] : 0.0;
+  block_layout<false>((const double2 *)x, (double2 *)dst, dim, ws->k, nullptr, cf, ws->stream);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(ws->stream));
   return 0;

@@ -18,6 +18,7 @@
 #include <cmath>
 #include <cstring>
 
+#include "block_layout.h"
 #include "engine_internal.h"
 #include "hphi_amd.h"
 
@@ -138,12 +139,34 @@ __global__ __launch_bounds__(TQ_TPB) void k_tpq_fused(double2 *v1, const double2
   }
 }
 
+// One workgroup's sums of the m columns of partial[nblk][m] (m a power of two,
+// at most 128) into sh[0..m), in fixed order.  Latency-bound: one thread per
+// column took 297 us for 1024 x 128 sums; TQ_FIN threads with eight loads in
+// flight each take 55 us (1 MB through one CU).
+#define TQ_FIN 1024
+__device__ __forceinline__ void tq_colsums(const double *__restrict__ partial, int nblk, int m, double *sh) {
+  const int q = threadIdx.x % m, ns = TQ_FIN / m;
+  double a[8] = {};
+  for (int b = threadIdx.x / m; b < nblk; b += 8 * ns) {
+#pragma unroll
+    for (int u = 0; u < 8; u++)
+      if (b + u * ns < nblk) a[u] += partial[(uint64_t)(b + u * ns) * m + q];
+  }
+  sh[threadIdx.x] = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
+  __syncthreads();
+  for (int st = TQ_FIN / 2; st >= m; st >>= 1) {
+    if (threadIdx.x < st) sh[threadIdx.x] += sh[threadIdx.x + st];
+    __syncthreads();
+  }
+}
+
 // state layout (doubles): [0..16) |w_s|^2, [16..32) 1/|w_s|, [32] step counter
-__global__ void k_tpq_start(const double *partial, int nblk, int k, double *state) {
+__global__ __launch_bounds__(TQ_FIN) void k_tpq_start(const double *partial, int nblk, int k, double *state) {
+  __shared__ double sh[TQ_FIN];
+  tq_colsums(partial, nblk, k, sh);
   const int c = threadIdx.x;
   if (c < k) {
-    double n = 0.0;
-    for (int b = 0; b < nblk; b++) n += partial[(uint64_t)b * k + c];
+    const double n = sh[c];
     state[c] = n;
     state[16 + c] = 1.0 / sqrt(n);
   }
@@ -151,16 +174,15 @@ __global__ void k_tpq_start(const double *partial, int nblk, int k, double *stat
 }
 
 // one block: output row of step s, next scale
-__global__ void k_tpq_finalize(const double *partial, int nblk, int k, const double2 *prdct, double *state,
-                               double lv, double Ns, int obs_kind, int nsite, double sz_const, double *out,
-                               int max_steps, int row0) {
+__global__ __launch_bounds__(TQ_FIN) void k_tpq_finalize(const double *partial, int nblk, int k, const double2 *prdct,
+                                                         double *state, double lv, double Ns, int obs_kind, int nsite,
+                                                         double sz_const, double *out, int max_steps, int row0) {
+  __shared__ double sh[TQ_FIN];
   const int c = threadIdx.x;
   const int s = (int)state[32];
-  __syncthreads();
+  tq_colsums(partial, nblk, k * TQ_NRED, sh);
   if (c < k) {
-    double r[TQ_NRED] = {};
-    for (int b = 0; b < nblk; b++)
-      for (int q = 0; q < TQ_NRED; q++) r[q] += partial[((uint64_t)b * k + c) * TQ_NRED + q];
+    const double *r = sh + c * TQ_NRED;
     const double n = state[c];
     const double E = prdct[c].x / n;
     const double var = r[0] / n;
@@ -275,30 +297,22 @@ static int tpq_enqueue_step(hphi_engine *e, const TpqPlan &P) {
                      dim, P.k, P.sj, P.sc, (const double *)P.state, P.lv, 1.0 / P.Ns, P.obs_kind, e->nsite,
                      hphi_model_gc(e->model) ? (const uint64_t *)nullptr : (const uint64_t *)e->d_list1,
                      P.part);
-  hipLaunchKernelGGL(k_tpq_finalize, dim3(1), dim3(64), 0, e->stream, (const double *)P.part, P.g, P.k,
+  hipLaunchKernelGGL(k_tpq_finalize, dim3(1), dim3(TQ_FIN), 0, e->stream, (const double *)P.part, P.g, P.k,
                      (const double2 *)(P.layout == 1 ? e->d_prdct : e->d_coef), P.state, P.lv, P.Ns, P.obs_kind,
                      e->nsite, P.sz_const, P.out, P.steps, P.row0);
   HIPCHK(hipGetLastError());
   return 0;
 }
 
-// w_c <- W0 column c (vector-major input, element c*dim + j) in the run's layout
-__global__ void k_tpq_load(double2 *v, const double2 *W0, uint64_t dim, int k, uint64_t sj, uint64_t sc) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= dim * (uint64_t)k) return;
-  const uint64_t c = i / dim, j = i % dim;
-  v[j * sj + c * sc] = W0[i];
-}
-
-// W_end column c = w_c / |w_c|, the normalised vector of the last step
-__global__ void k_tpq_store(double2 *W_end, const double2 *v, uint64_t dim, int k, uint64_t sj, uint64_t sc,
-                            const double *state) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= dim * (uint64_t)k) return;
-  const uint64_t c = i / dim, j = i % dim;
-  const double2 a = v[j * sj + c * sc];
-  const double f = state[16 + c];
-  W_end[i] = make_double2(a.x * f, a.y * f);
+// W_end column c = w_c / |w_c| where the run keeps its vectors one after another
+__global__ __launch_bounds__(256) void k_tpq_store(double2 *W_end, const double2 *v, uint64_t dim,
+                                                   const double *state) {
+  const double f = state[16 + blockIdx.y];
+  const uint64_t c0 = (uint64_t)blockIdx.y * dim;
+  for (uint64_t j = (uint64_t)blockIdx.x * 256 + threadIdx.x; j < dim; j += (uint64_t)gridDim.x * 256) {
+    const double2 a = v[c0 + j];
+    W_end[c0 + j] = make_double2(a.x * f, a.y * f);
+  }
 }
 
 // the step counter of a resumed run (the first enqueued step is step0 - 1)
@@ -364,15 +378,19 @@ static int tpq_run(hphi_engine *e, const hphi_tpq_params *p, const double *W0, i
     }
     uint64_t n = dim * (uint64_t)k;
     const unsigned gn = (unsigned)((n + 255) / 256);
-    if (W0)
-      hipLaunchKernelGGL(k_tpq_load, dim3(gn), dim3(256), 0, e->stream, (double2 *)P.V1, (const double2 *)W0, dim, k,
-                         P.sj, P.sc);
-    else
+    if (W0 && P.layout == 1) {
+      block_layout<true>((const double2 *)W0, (double2 *)P.V1, dim, k, nullptr, BlScale{}, e->stream);
+    } else if (W0) {
+      if (hipMemcpyAsync(P.V1, W0, vbytes, hipMemcpyDeviceToDevice, e->stream) != hipSuccess) {
+        rc = hphi_set_error("hphi_tpq: copy of the start vectors failed");
+        break;
+      }
+    } else
       hipLaunchKernelGGL(k_tpq_init, dim3(gn), dim3(256), 0, e->stream, (double2 *)P.V1, dim, k, P.sj, P.sc, p->seed,
                          p->init_kind);
     hipLaunchKernelGGL(k_tpq_colnorm, dim3(P.g), dim3(TQ_TPB), 0, e->stream, (const double2 *)P.V1, dim, k, P.sj,
                        P.sc, P.part);
-    hipLaunchKernelGGL(k_tpq_start, dim3(1), dim3(64), 0, e->stream, (const double *)P.part, P.g, k, P.state);
+    hipLaunchKernelGGL(k_tpq_start, dim3(1), dim3(TQ_FIN), 0, e->stream, (const double *)P.part, P.g, k, P.state);
     if (step0 > 0) {  // resumed: the given vector is step step0 - 1's, its row is not kept
       hipLaunchKernelGGL(k_tpq_set_step, dim3(1), dim3(1), 0, e->stream, P.state, (double)(step0 - 1));
       P.row0 = step0;
@@ -384,8 +402,12 @@ static int tpq_run(hphi_engine *e, const hphi_tpq_params *p, const double *W0, i
     // taken right before that step, whose fused pass moves on to the next vector
     const int s_first = step0 > 0 ? step0 - 1 : 0, last = p->steps - 1;
     auto store = [&]() {
-      hipLaunchKernelGGL(k_tpq_store, dim3(gn), dim3(256), 0, e->stream, (double2 *)W_end, (const double2 *)P.V1, dim,
-                         k, P.sj, P.sc, (const double *)P.state);
+      if (P.layout == 1)
+        block_layout<false>((const double2 *)P.V1, (double2 *)W_end, dim, k, (const double *)P.state + 16, BlScale{},
+                            e->stream);
+      else
+        hipLaunchKernelGGL(k_tpq_store, dim3((unsigned)std::min<uint64_t>((dim + 255) / 256, 4096), k), dim3(256), 0,
+                           e->stream, (double2 *)W_end, (const double2 *)P.V1, dim, (const double *)P.state);
     };
     if (W_end && s_first == last) store();
     if ((rc = tpq_enqueue_step(e, P))) break;  // the first step eagerly (also loads the code objects)
@@ -467,11 +489,12 @@ __global__ __launch_bounds__(256) void k_ct_acc(double2 *A, const double2 *Cv, u
 
 // norms of the k columns from k_tpq_colnorm partials: state[c] = |A_c|,
 // state[16 + c] = 1 / |A_c|
-__global__ void k_ct_norms(const double *partial, int nblk, int k, double *state) {
+__global__ __launch_bounds__(TQ_FIN) void k_ct_norms(const double *partial, int nblk, int k, double *state) {
+  __shared__ double sh[TQ_FIN];
+  tq_colsums(partial, nblk, k, sh);
   const int c = threadIdx.x;
   if (c < k) {
-    double n = 0.0;
-    for (int b = 0; b < nblk; b++) n += partial[(uint64_t)b * k + c];
+    const double n = sh[c];
     state[c] = sqrt(n);
     state[16 + c] = 1.0 / sqrt(n);
   }
@@ -534,23 +557,17 @@ __global__ __launch_bounds__(TQ_TPB) void k_ct_moments(const double2 *P, const d
   }
 }
 
-// W_end column c (element c*dim + j) = P[j][c]
-__global__ void k_ct_store(double2 *W_end, const double2 *P, uint64_t dim, int k) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= dim * (uint64_t)k) return;
-  const uint64_t c = i / dim, j = i % dim;
-  W_end[i] = P[j * (uint64_t)k + c];
-}
-
 // row s of sample c (the mTPQ row layout): inv_temp (s additions of dtau), E, <H^2>, the
 // norm before normalisation (step 0: the start vector's), the moments
-__global__ void k_ct_finalize(const double *partial, int nblk, int k, const double2 *prdct, const double *state,
-                              int s, double dtau, int obs_kind, int nsite, double sz_const, double *out, int row0) {
+__global__ __launch_bounds__(TQ_FIN) void k_ct_finalize(const double *partial, int nblk, int k, const double2 *prdct,
+                                                        const double *state, int s, double dtau, int obs_kind,
+                                                        int nsite, double sz_const, double *out, int row0) {
+  __shared__ double sh[TQ_FIN];
+  if (s < row0) return;
+  tq_colsums(partial, nblk, k * TQ_NRED, sh);
   const int c = threadIdx.x;
-  if (c >= k || s < row0) return;
-  double r[TQ_NRED] = {};
-  for (int b = 0; b < nblk; b++)
-    for (int q = 0; q < TQ_NRED; q++) r[q] += partial[((uint64_t)b * k + c) * TQ_NRED + q];
+  if (c >= k) return;
+  const double *r = sh + c * TQ_NRED;
   double *o = out + ((uint64_t)(s - row0) * k + c) * TQ_NOUT;
   double it = 0.0;  // inv_temp += delta_tau once per step (CalcByCanonicalTPQ.c:227)
   for (int i = 0; i < s; i++) it += dtau;
@@ -628,8 +645,7 @@ static int ctpq_run(hphi_engine *e, const hphi_ctpq_params *p, const double *W0,
     if (hipEventRecord(ev0, e->stream) != hipSuccess) { rc = hphi_set_error("event record failed"); break; }
     // step 0: start vector (MakeIniVec), normalised, measured (CalcByCanonicalTPQ.c:140-175)
     if (W0)
-      hipLaunchKernelGGL(k_tpq_load, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, e->stream, A,
-                         (const double2 *)W0, dim, k, (uint64_t)k, (uint64_t)1);
+      block_layout<true>((const double2 *)W0, A, dim, k, nullptr, BlScale{}, e->stream);
     else
       hipLaunchKernelGGL(k_tpq_init, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, e->stream, A, dim, k,
                          (uint64_t)k, (uint64_t)1, p->seed, p->init_kind);
@@ -651,14 +667,14 @@ static int ctpq_run(hphi_engine *e, const hphi_ctpq_params *p, const double *W0,
       // normalise A into P (global_norm; step 0: global_1st_norm)
       hipLaunchKernelGGL(k_tpq_colnorm, dim3(g), dim3(TQ_TPB), 0, e->stream, (const double2 *)A, dim, k, (uint64_t)k,
                          (uint64_t)1, part);
-      hipLaunchKernelGGL(k_ct_norms, dim3(1), dim3(64), 0, e->stream, (const double *)part, g, k, state);
+      hipLaunchKernelGGL(k_ct_norms, dim3(1), dim3(TQ_FIN), 0, e->stream, (const double *)part, g, k, state);
       hipLaunchKernelGGL(k_ct_scale, dim3(gs), dim3(256), 0, e->stream, P, (const double2 *)A, dim, k,
                          (const double *)state);
       // measure: Hp = H P (its prdct is E), <H^2> and the moments (expec_energy_flct)
       if (hphi_hv_launch_ex(e, k, (double *)Hp, (const double *)P, 1)) { rc = -1; break; }
       hipLaunchKernelGGL(k_ct_moments, dim3(g), dim3(TQ_TPB), 0, e->stream, (const double2 *)P, (const double2 *)Hp,
                          dim, k, obs_kind, e->nsite, list1, part);
-      hipLaunchKernelGGL(k_ct_finalize, dim3(1), dim3(64), 0, e->stream, (const double *)part, g, k,
+      hipLaunchKernelGGL(k_ct_finalize, dim3(1), dim3(TQ_FIN), 0, e->stream, (const double *)part, g, k,
                          (const double2 *)e->d_prdct, (const double *)state, s, dtau, obs_kind, e->nsite, sz_const,
                          out, step0);
       if (hipGetLastError() != hipSuccess) { rc = hphi_set_error("hphi_ctpq: launch failed"); break; }
@@ -671,8 +687,9 @@ static int ctpq_run(hphi_engine *e, const hphi_ctpq_params *p, const double *W0,
     float ms = 0.f;
     (void)hipEventElapsedTime(&ms, ev0, ev1);
     if (W_end) {  // P holds the last step's normalised vectors, state-major
-      hipLaunchKernelGGL(k_ct_store, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, e->stream, (double2 *)W_end,
-                         (const double2 *)P, dim, k);
+      BlScale one;
+      for (double &f : one.f) f = 1.0;
+      block_layout<false>((const double2 *)P, (double2 *)W_end, dim, k, nullptr, one, e->stream);
       if (hipGetLastError() != hipSuccess || hipStreamSynchronize(e->stream) != hipSuccess) {
         rc = hphi_set_error("hphi_ctpq: copy of the final vectors failed");
         break;
