@@ -68,6 +68,14 @@ struct DTerm {
   double V;
 };
 
+// runs of one kind in a diagonal's terms, after the skip leading constants (sum
+// d0): the term compiler lists at most five kinds, each together
+#define DIAG_RUNS 8
+struct DRuns {
+  double d0;
+  int skip, n, kind[DIAG_RUNS], len[DIAG_RUNS];
+};
+
 struct SzParams {
   int hubbard, nlow, nhigh, nup, ndn;
   int nlu, nld, nhu, nhd;  // Hubbard: up/down positions in the low / high half
@@ -231,9 +239,9 @@ int hphi_ensure_binom_table();
 uint64_t hphi_term_nnz(const hphi_engine *e);
 SzParams hphi_sz_params(const hphi_engine *e);
 int hphi_launch_tables(const SzParams &P, uint64_t sdim, uint64_t size21, uint64_t *jb, uint32_t *l21, uint64_t *l22, uint64_t *list1, hipStream_t st);
-// diag[j * stride + col] for j < dim
-int hphi_launch_diag(uint64_t dim, const uint64_t *list1, int gc, const DTerm *dterms, int nd, double *diag,
-                     hipStream_t st, int stride = 1, int col = 0);
+// diag[j * stride + col] for the states j of h's sector, dterms its diagonal terms on the device
+int hphi_launch_diag(const hphi_engine &h, const uint64_t *list1, const DTerm *dterms, double *diag, hipStream_t st,
+                     int stride = 1, int col = 0);
 int hphi_hv_launch_canon(hphi_engine *e, const HvArgs &A, int g, int skip_high = 0);
 // canonical Spin: is the high-half pass usable and wanted for this engine (host check only)
 int hphi_hi_wanted(const hphi_engine *e);

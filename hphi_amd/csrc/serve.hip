@@ -945,7 +945,7 @@ static int column_start(hphi_server *s, Slab *b, int c, Job *j) {
   HIPCHK(hipMemcpyAsync(b->coef, stage(s, b->coef_host.data(), cb), cb, hipMemcpyHostToDevice, s->stream));
   DTerm *dt = b->dterms + (size_t)c * std::max<size_t>(nd, 1);
   if (db) HIPCHK(hipMemcpyAsync(dt, stage(s, h.h_dterms.data(), db), db, hipMemcpyHostToDevice, s->stream));
-  if (hphi_launch_diag(h.dim, b->list1, 0, dt, (int)nd, b->diag, s->stream, SL_K, c)) return -1;
+  if (hphi_launch_diag(h, b->list1, dt, b->diag, s->stream, SL_K, c)) return -1;
   const unsigned g = (unsigned)((h.dim + 255) / 256);
   hipLaunchKernelGGL(k_sl_start, dim3(g), dim3(256), 0, s->stream, b->R, b->Q, c, h.dim, j->seed, s->d_js, j->slot);
   HIPCHK(hipGetLastError());
