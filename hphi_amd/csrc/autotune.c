@@ -1,8 +1,8 @@
 /*
  * Launch-shape autotuner for the H·v kernels (host C over the hphi_amd C ABI).
  *
- * For the single-vector canonical kernel it sweeps workgroup size, workgroups
- * per CU, list_2_1 in LDS or L2, and the XCD-contiguous tile mapping; for the
+ * For the single-vector canonical kernels it sweeps blocks per wave of the one by
+ * classes, and of the other workgroup size, workgroups per CU, list_2_1 in LDS or L2, and the XCD-contiguous tile mapping; for the
  * block kernel (k > 1) it sweeps columns per lane, workgroup size, workgroups
  * per CU and the XCD mapping; the per-column kernel is always a candidate, and
  * the grand-canonical tiles where the sector has them.  Each candidate is timed with HIP events over `reps` H·v calls on
@@ -19,8 +19,8 @@ int hphi_set_error(const char *fmt, ...);
 
 typedef struct {
   int n;
-  const char *knob[6];
-  int val[6];
+  const char *knob[7];
+  int val[7];
 } cand_t;
 
 static void add(cand_t *c, const char *knob, int val) {
@@ -40,9 +40,14 @@ int hphi_autotune(hphi_engine *e, int k, double *v0, const double *v1, int reps,
   if (!e || !v0 || !v1) return hphi_set_error("hphi_autotune: NULL argument");
   if (reps < 1) reps = 2;
   cand_t cands[96];
-  int n = 0, c2 = 0, blk = 0, lds_ok = 0, crank_ok = 0, gc = 0;
+  int n = 0, c2 = 0, blk = 0, lds_ok = 0, crank_ok = 0, gc = 0, cls = 0;
   memset(cands, 0, sizeof cands);
   if (k == 1 && hphi_engine_get_tune(e, "use_c2", &c2) == 0 && c2) {
+    hphi_engine_get_tune(e, "cls", &cls);
+    for (int cb = 1; cls && cb <= 4; cb *= 2) { /* by classes; every later candidate turns it off */
+      cand_t *c = &cands[n++];
+      add(c, "cls", 1), add(c, "cls_blocks", cb), add(c, "use_c2", 1), add(c, "c2_crank", 1);
+    }
     /* is list_2_1 allowed in LDS for this model? */
     int saved = 0;
     hphi_engine_get_tune(e, "lds21", &saved);
@@ -58,6 +63,7 @@ int hphi_autotune(hphi_engine *e, int k, double *v0, const double *v1, int reps,
           cand_t *c = &cands[n++];
           add(c, "use_c2", 1), add(c, "xcd_map", xcd), add(c, "tpb", tpbs[a]);
           add(c, "wgs_per_cu", 1), add(c, "lds21", 1), add(c, "c2_crank", 0);
+          if (cls) add(c, "cls", 0);
         }
       }
       for (int a = 0; a < 3; a++)
@@ -66,6 +72,7 @@ int hphi_autotune(hphi_engine *e, int k, double *v0, const double *v1, int reps,
             cand_t *c = &cands[n++];
             add(c, "use_c2", 1), add(c, "xcd_map", xcd), add(c, "tpb", tpbs[a]);
             add(c, "wgs_per_cu", w), add(c, "lds21", 0), add(c, "c2_crank", 0);
+            if (cls) add(c, "cls", 0);
           }
       if (crank_ok) { /* spin rank tables: large grids of small workgroups */
         const int ws[4] = {14, 21, 40, 48};
@@ -73,6 +80,7 @@ int hphi_autotune(hphi_engine *e, int k, double *v0, const double *v1, int reps,
           cand_t *c = &cands[n++];
           add(c, "use_c2", 1), add(c, "xcd_map", xcd), add(c, "tpb", 256);
           add(c, "wgs_per_cu", ws[a]), add(c, "c2_crank", 1);
+          if (cls) add(c, "cls", 0);
         }
       }
     }

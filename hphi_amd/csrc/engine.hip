@@ -980,6 +980,7 @@ extern "C" void hphi_engine_destroy(hphi_engine *e) {
   (void)hipFree(e->d_v1t);
   (void)hipFree(e->d_tofs);
   (void)hipFree(e->d_gcterms);
+  (void)hipFree(e->d_cls);
   (void)hipFree(e->d_jb);
   (void)hipFree(e->d_diag);
   (void)hipFree(e->d_terms);
@@ -1019,6 +1020,8 @@ extern "C" uint64_t hphi_engine_device_bytes(const hphi_engine *e) { return e ? 
 extern "C" int hphi_engine_tune(hphi_engine *e, const char *knob, int value) {
   if (!e || !knob) return hphi_set_error("hphi_engine_tune: NULL argument");
   std::string k(knob);
+  if (k == "tpb" || k == "wgs_per_cu" || k == "lds21" || k == "c2_crank" || k == "c2_unroll" || k == "xcd_map")
+    e->c2_tuned = 1;
   if (k == "tpb") {
     if (value != 256 && value != 512 && value != 1024) return hphi_set_error("tpb must be 256, 512 or 1024");
     e->c2_tpb = value;
@@ -1064,6 +1067,15 @@ extern "C" int hphi_engine_tune(hphi_engine *e, const char *knob, int value) {
     e->grid_per_cu = value;
   } else if (k == "use_blk") {
     e->use_blk = value ? 1 : 0;
+  } else if (k == "cls") {
+    if (value < -1 || value > 1) return hphi_set_error("cls must be -1, 0 or 1");
+    e->cls = value;
+  } else if (k == "cls_blocks") {
+    if (value != 0 && value != 1 && value != 2 && value != 4) return hphi_set_error("cls_blocks must be 0, 1, 2 or 4");
+    e->cls_blocks = value;
+  } else if (k == "cls_wgs_per_cu") {
+    if (value < 1 || value > 256) return hphi_set_error("cls_wgs_per_cu out of range");
+    e->cls_wgs_per_cu = value;
   } else if (k == "gc_tile") {
     if (value < -1 || value > 1) return hphi_set_error("gc_tile must be -1, 0 or 1");
     e->gc_tile = value;
@@ -1103,6 +1115,9 @@ extern "C" int hphi_engine_get_tune(const hphi_engine *e, const char *knob, int 
   else if (k == "use_c2") *value = e->use_c2 && e->c2_ok;
   else if (k == "grid_per_cu") *value = e->grid_per_cu;
   else if (k == "use_blk") *value = e->use_blk && hphi_blk_ok(e);
+  else if (k == "cls") *value = hphi_cls_wanted(e);
+  else if (k == "cls_blocks") *value = hphi_cls_blocks(e);
+  else if (k == "cls_wgs_per_cu") *value = e->cls_wgs_per_cu;
   else if (k == "gc_tile") *value = hphi_gc_wanted(e, 1) || hphi_gc_wanted(e, 2) || hphi_gc_wanted(e, 4) ||
                                     hphi_gc_wanted(e, 8) || hphi_gc_wanted(e, 16);
   else if (k == "lb_mfma") *value = e->lb_mfma;
@@ -1187,6 +1202,7 @@ int hphi_build_tables(hphi_engine *e) {
     return hphi_set_error("basis count %llu differs from idim_max %llu", (unsigned long long)total,
                           (unsigned long long)e->dim);
   e->tables_ready = true;
+  if (hphi_cls_build(e)) return -1;
   // plan of the high-half pass now, outside any H·v launch (it copies list_2_2 to the host)
   if (hphi_hi_split_on(e) < 0) return -1;
   return 0;
@@ -1306,7 +1322,7 @@ int hphi_hv_launch_ex(hphi_engine *e, int k, double *v0, const double *v1, int o
 enum { HV_PATH_CANON, HV_PATH_GC, HV_PATH_BLK, HV_PATH_GENERIC };
 static int hv_path(const hphi_engine *e, int k, int *grid, int gather = 0) {
   if (k == 1 && e->c2_ok && e->use_c2) {
-    *grid = canon_grid(e);
+    *grid = hphi_cls_wanted(e) ? hphi_cls_grid(e) : canon_grid(e);
     return HV_PATH_CANON;
   }
   if (!gather && hphi_gc_wanted(e, k)) {
@@ -1337,8 +1353,12 @@ static int hv_launch_args(hphi_engine *e, int k, HvArgs &A, double2 *prdct_out, 
       A.v1t = e->d_v1t;
       A.tofs = e->d_tofs;
     }
-    if (split) g = canon_grid(e, e->hi_p1_wgs_per_cu);  // the first pass without the high terms
-    if (hphi_hv_launch_canon(e, A, g, split)) return -1;
+    if (hphi_cls_wanted(e)) {
+      if (hphi_hv_launch_cls(e, A, g, split)) return -1;
+    } else {
+      if (split) g = canon_grid(e, e->hi_p1_wgs_per_cu);  // the first pass without the high terms
+      if (hphi_hv_launch_canon(e, A, g, split)) return -1;
+    }
     if (split) {
       int g2 = 0;
       if (hphi_hv_launch_high(e, A, A.partial + g, &g2)) return -1;

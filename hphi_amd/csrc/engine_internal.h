@@ -144,6 +144,26 @@ struct HiPlan {
   uint64_t wgp[HI_MAXC + 1], base[HI_MAXC + 1];
 };
 
+// Canonical H·v by classes (hv_class.hip)
+struct ClsTerm {
+  double cre, cim;
+  uint32_t flip, tmask, tval, sgn;
+  uint32_t tlo;            // the low half's part of tval
+  int parity, never, lo;   // parity predicate (else value); padding; index of a mixed term's low-half flip
+};
+#define CL_TPB 256
+#define CL_MAXC 96
+#define CL_MAXLO 64               // distinct low-half flips of the mixed terms
+struct ClsArgs {
+  int ncls, n_low, n_high, n_mixed, nt, nlo, skip;
+  int n_lowp, n_mixp;  // of the low and mixed terms, those with a parity predicate (first)
+  uint32_t units;
+  uint32_t start[CL_MAXC], nblk[CL_MAXC], size[CL_MAXC], ntile[CL_MAXC], upre[CL_MAXC + 1];
+  uint32_t lo[CL_MAXLO];
+  const ClsTerm *terms;
+  const uint32_t *bstart, *bxh, *tgt;  // per block in class order; tgt [block][high and mixed terms]
+};
+
 // Grand-canonical H·v in LDS tiles (hv_gc.hip): a pass applies the terms whose
 // flips lie inside its bit set S to the tiles of 2^|S| states.
 struct GcTerm {
@@ -216,6 +236,12 @@ struct hphi_engine {
   double2 *d_v1t = nullptr;      // tile-major copy of v1, hi_plan.base[ncls] elements
   ulonglong2 *d_tofs = nullptr;  // per block: its first tile-major element, and the stride between its tiles
   HiPlan hi_plan{};
+  // canonical H·v by classes: -1 unless a shape of k_hv_canon is set, 0 off, 1 on where the sector allows it
+  int cls = -1, cls_blocks = 0;
+  int cls_wgs_per_cu = 256;  // 8x4 J1-J2: 77.3 ms at 64, 75.1 at 256; 7x4: 3.67, 3.37; no effect below
+  int c2_tuned = 0;  // a shape of k_hv_canon was set by hand
+  void *d_cls = nullptr;
+  ClsArgs cls_args{};
   // grand-canonical H·v in LDS tiles: -1 by size, 0 off, 1 also with a hand-set block shape
   int gc_tile = -1;
   GcPlan gc_plan[5];  // block sizes 1, 2, 4, 8, 16
@@ -249,6 +275,11 @@ int hphi_hi_wanted(const hphi_engine *e);
 int hphi_hi_split_on(hphi_engine *e);
 // launches the high-half pass: accumulates into A.v0, partials at partial[0..*grid)
 int hphi_hv_launch_high(hphi_engine *e, const HvArgs &A, double2 *partial, int *grid);
+int hphi_cls_build(hphi_engine *e);
+int hphi_cls_wanted(const hphi_engine *e);
+int hphi_cls_blocks(const hphi_engine *e);
+int hphi_cls_grid(const hphi_engine *e);
+int hphi_hv_launch_cls(hphi_engine *e, const HvArgs &H, int g, int skip_high);
 int hphi_gc_wanted(const hphi_engine *e, int k);
 int hphi_gc_plan_build(hphi_engine *e);
 int hphi_gc_partials(const hphi_engine *e, int k);  // workgroups of all passes of one H·v

@@ -1,0 +1,520 @@
+// Gather-form H·v of canonical sectors (Spin, Hubbard), a tile of low-half ranks
+// for several blocks at once.
+//
+// A state is (block = its high-half bits, rank of its low-half bits among
+// those of its class), at index start[block] + rank; blocks of one class (equal
+// particle numbers in the high half) have the same low halves in the same
+// order.  k_hv_canon decodes every state of its own: predicate, rank lookup and
+// 64-bit address of every term, some 28 vector instructions per term and state,
+// which is half its time on sectors whose vectors stay in the caches.  Here
+// a wave takes 64 consecutive ranks of one class and CB blocks of that class:
+//  * low-half terms: predicate and target rank are the same in every block, so
+//    they are computed once; the gather's address is the block's scalar base
+//    plus the rank's 32-bit offset, with no vector arithmetic per block;
+//  * high-half terms: the target block's base comes from a table of every
+//    block and term (no base: the term does not act there); the offset is the
+//    state's own rank;
+//  * mixed terms: the base from the same table, the target rank from LDS, where
+//    each lane keeps one rank per low-half flip that occurs (16 for the 48 mixed
+//    terms of the 8x4 sector).
+// Same sums in the same order as k_hv_canon (value predicates after parity
+// ones within a group).  Microseconds per H·v, k_hv_canon / this kernel:
+//   16-site J1-J2 chain (12,870 states)  15.6 / 10.8    6x4 J1-J2 (2.7e6)    292 / 151
+//   20-site ladder (184,756)             20.9 / 16.8    12-site Hubbard      55.3 / 34.4
+//   23-site chain (1.35e6)               90.2 / 50.5    7x4 J1-J2 (4.0e7)    5657 / 3380
+//   4x4 Hubbard (1.7e8)                14,350 / 12,880  8x4 J1-J2 (6.0e8, with the
+//   high-half pass)                    90,000 / 75,400
+// The small ones are a chain of latencies, the middle ones were bound by that
+// arithmetic and are now by the L1's 64 bytes per cycle and L2; on 8x4 each of
+// the two halves of the terms misses L2 for 200 GB, 5.5 TB/s with the streams.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <map>
+#include <vector>
+
+#include "engine_internal.h"
+
+#define HIPCHK(x)                                                                  \
+  do {                                                                             \
+    hipError_t e_ = (x);                                                           \
+    if (e_ != hipSuccess) return hphi_set_error("%s failed: %s", #x, hipGetErrorString(e_)); \
+  } while (0)
+
+typedef const uint32_t __attribute__((address_space(4))) *CU32;
+typedef const ClsTerm __attribute__((address_space(4))) *CClsTerm;
+
+#define CL_U 8  // gathers in flight per lane: CL_U / CB terms per batch (4 and 16 within 3 % or slower)
+#define CL_NONE 0xffffffffu  // the term does not act in this block
+
+// 16 x the rank of low-half value y within its class (byte offset of its amplitude)
+template <int RK>
+__device__ __forceinline__ uint32_t cl_rank16(const uint16_t *t, uint32_t y) {
+  if (RK == 3)
+    return ((uint32_t)t[y & 255u] + (uint32_t)t[256u + 25u * (y >> 8) + 5u * (uint32_t)__popc(y & 0x55u) +
+                                                 (uint32_t)__popc(y & 0xAAu)]) << 4;
+  return ((uint32_t)t[y & 255u] + (uint32_t)t[256u + 9u * (y >> 8) + (uint32_t)__popc(y & 255u)]) << 4;
+}
+
+__device__ __forceinline__ double2 cl_at(const double2 *base, uint32_t off) {
+  return *(const double2 *)((const char *)base + off);
+}
+
+template <bool REALC>
+__device__ __forceinline__ void cl_mac(double2 &a, double cr, double ci, double2 g) {
+  a.x += cr * g.x;
+  a.y += cr * g.y;
+  if (!REALC) {
+    a.x -= ci * g.y;
+    a.y += ci * g.x;
+  }
+}
+
+__device__ __forceinline__ ClsTerm cl_term(CClsTerm p) {
+  ClsTerm t;
+  t.cre = p->cre;
+  t.cim = p->cim;
+  t.flip = p->flip;
+  t.tmask = p->tmask;
+  t.tval = p->tval;
+  t.sgn = p->sgn;
+  t.lo = p->lo;
+  t.tlo = p->tlo;
+  t.parity = t.never = 0;
+  return t;
+}
+
+// n low-half terms of one predicate kind (PAR: the parity of the masked bits is
+// odd; else the masked bits have a value) on CB blocks
+template <int CB, bool PAR, bool REALC, int RK>
+__device__ __forceinline__ void cl_low(CClsTerm TL, int n, uint32_t ia, const double2 *v1, const uint32_t *base,
+                                       const uint16_t *s21, double2 *acc) {
+  constexpr int U = CL_U / CB;
+#pragma unroll 1
+  for (int t = 0; t < n; t += U) {
+    double2 g[U][CB];
+    uint32_t off[U];
+    bool act[U];
+#pragma unroll
+    for (int q = 0; q < U; q++) {
+      const ClsTerm T = cl_term(TL + t + q);
+      act[q] = PAR ? (__popc(ia & T.tmask) & 1) != 0 : (ia & T.tmask) == T.tval;
+      off[q] = cl_rank16<RK>(s21, ia ^ T.flip);
+    }
+#pragma unroll
+    for (int q = 0; q < U; q++) {
+#pragma unroll
+      for (int b = 0; b < CB; b++) g[q][b] = make_double2(0.0, 0.0);
+      if (act[q]) {
+#pragma unroll
+        for (int b = 0; b < CB; b++) g[q][b] = cl_at(v1 + base[b], off[q]);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < U; q++) {
+      const ClsTerm T = cl_term(TL + t + q);
+      const bool neg = RK == 3 && (__popc(ia & T.sgn) & 1);
+      const double cr = neg ? -T.cre : T.cre, ci = neg ? -T.cim : T.cim;
+#pragma unroll
+      for (int b = 0; b < CB; b++) cl_mac<REALC>(acc[b], cr, ci, g[q][b]);
+    }
+  }
+}
+
+// n mixed terms of one predicate kind: the low half's part of the predicate per
+// lane, the high half's per block; tgt: the terms' first column of the table
+template <int CB, bool PAR, bool REALC, int RK>
+__device__ __forceinline__ void cl_mixed(CClsTerm TM, int n, uint32_t ia, const double2 *v1, const uint32_t *xh,
+                                         CU32 tgt, const uint32_t *row, const uint32_t *sla, double2 *acc) {
+  constexpr int U = CL_U / CB;
+#pragma unroll 1
+  for (int t = 0; t < n; t += U) {
+    double2 g[U][CB];
+    uint32_t off[U], lp[U], to[U][CB];
+#pragma unroll
+    for (int b = 0; b < CB; b++)
+#pragma unroll
+      for (int q = 0; q < U; q++) to[q][b] = tgt[row[b] + t + q];
+#pragma unroll
+    for (int q = 0; q < U; q++) {
+      const ClsTerm T = cl_term(TM + t + q);
+      off[q] = sla[T.lo * CL_TPB + threadIdx.x];
+      lp[q] = PAR ? (uint32_t)__popc(ia & T.tmask) & 1u : ((ia & T.tmask) == T.tlo ? 1u : 0u);
+    }
+#pragma unroll
+    for (int q = 0; q < U; q++) {
+      const ClsTerm T = cl_term(TM + t + q);
+#pragma unroll
+      for (int b = 0; b < CB; b++) {
+        // scalar: what lp must be in this block (2: never)
+        const uint32_t ok = PAR ? ((uint32_t)__popc(xh[b] & T.tmask) & 1u) ^ 1u : 1u;
+        const uint32_t want = to[q][b] == CL_NONE ? 2u : ok;
+        g[q][b] = make_double2(0.0, 0.0);
+        if (lp[q] == want) g[q][b] = cl_at(v1 + to[q][b], off[q]);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < U; q++) {
+      const ClsTerm T = cl_term(TM + t + q);
+      const uint32_t ls = RK == 3 ? (uint32_t)__popc(ia & T.sgn) : 0u;
+#pragma unroll
+      for (int b = 0; b < CB; b++) {
+        const bool neg = RK == 3 && ((ls + (uint32_t)__popc(xh[b] & T.sgn)) & 1u);
+        cl_mac<REALC>(acc[b], neg ? -T.cre : T.cre, neg ? -T.cim : T.cim, g[q][b]);
+      }
+    }
+  }
+}
+
+template <int CB, bool REALC, int RK>
+__global__ __launch_bounds__(CL_TPB) void k_hv_cls(const HvArgs A, const ClsArgs C) {
+  constexpr int U = CL_U / CB;  // terms per batch
+  constexpr bool SGN = RK == 3;
+  constexpr int NT = RK == 3 ? HRANK_N : CRANK_N;
+  __shared__ uint16_t s21[NT];
+  extern __shared__ uint32_t sla[];  // [nlo][CL_TPB]: offsets of the low-half flips of the mixed terms
+  const uint32_t tid = threadIdx.x;
+  for (uint32_t i = tid; i < NT / 4; i += CL_TPB) ((uint2 *)s21)[i] = ((const uint2 *)A.crank)[i];
+  __syncthreads();
+  const uint32_t lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const CU32 bstart = (CU32)C.bstart, bxh = (CU32)C.bxh, tgt = (CU32)C.tgt;
+  const CClsTerm TL = (CClsTerm)C.terms, TH = TL + C.n_low, TM = TH + C.n_high;
+  const double2 *v1 = (const double2 *)A.v1;
+  double2 *v0 = (double2 *)A.v0;
+  // an XCD takes a contiguous range of units
+  const uint32_t xcd = blockIdx.x & 7u, slot = (blockIdx.x >> 3) * (CL_TPB / 64) + wave;
+  const uint32_t nslot = (gridDim.x >> 3) * (CL_TPB / 64);
+  const uint32_t U1 = (uint32_t)((uint64_t)C.units * (xcd + 1) / 8);
+  double pre = 0.0, pim = 0.0;
+  for (uint32_t u = (uint32_t)((uint64_t)C.units * xcd / 8) + slot; u < U1; u += nslot) {
+    int c = 0, hi = C.ncls;  // upre[c] <= u < upre[hi]
+    while (hi - c > 1) {
+      const int mid = (c + hi) >> 1;
+      if (C.upre[mid] <= u) c = mid;
+      else hi = mid;
+    }
+    const uint32_t loc = u - C.upre[c], ntile = C.ntile[c], size = C.size[c];
+    const uint32_t grp = loc / ntile, tile = loc % ntile;
+    const uint32_t p0 = C.start[c] + grp * CB, nb = C.start[c] + C.nblk[c] - p0;  // blocks from here on
+    const uint32_t r = tile * 64u + lane;
+    if (r >= size) continue;
+    const uint32_t own_off = r << 4;
+    uint32_t base[CB], xh[CB], row[CB];
+    double2 acc[CB];
+#pragma unroll
+    for (int b = 0; b < CB; b++) {
+      const uint32_t p = p0 + (b < (int)nb ? b : 0);  // past the class's last block: the first again, not stored
+      base[b] = bstart[p];
+      xh[b] = bxh[p];
+      row[b] = p * (uint32_t)C.nt;
+    }
+    const uint32_t ia = (uint32_t)A.list1[base[0] + r] & (uint32_t)A.irght;
+#pragma unroll
+    for (int b = 0; b < CB; b++) acc[b] = cl_at(v1 + base[b], own_off);
+    if (A.v1t) {  // tile-major copy for the high-half pass
+#pragma unroll
+      for (int b = 0; b < CB; b++)
+        if (b < (int)nb) {
+          const ulonglong2 ts = A.tofs[xh[b] >> A.nlow];
+          A.v1t[ts.x + (uint64_t)(r / HI_RT) * ts.y + r % HI_RT] = acc[b];
+        }
+    }
+#pragma unroll
+    for (int b = 0; b < CB; b++) {
+      const double d = *(const double *)((const char *)(A.diag + base[b]) + (r << 3));
+      acc[b].x *= d;
+      acc[b].y *= d;
+    }
+    // ---- low-half terms: one predicate and one target rank for all blocks
+    cl_low<CB, true, REALC, RK>(TL, C.n_lowp, ia, v1, base, s21, acc);
+    cl_low<CB, false, REALC, RK>(TL + C.n_lowp, C.n_low - C.n_lowp, ia, v1, base, s21, acc);
+    // ---- high-half terms: the same rank of another block
+    for (int t = C.skip; t < C.n_high; t += U) {
+      double2 g[U][CB];
+      uint32_t to[U][CB];
+#pragma unroll
+      for (int b = 0; b < CB; b++)
+#pragma unroll
+        for (int q = 0; q < U; q++) to[q][b] = tgt[row[b] + t + q];
+#pragma unroll
+      for (int q = 0; q < U; q++)
+#pragma unroll
+        for (int b = 0; b < CB; b++) {
+          g[q][b] = make_double2(0.0, 0.0);
+          if (to[q][b] != CL_NONE) g[q][b] = cl_at(v1 + to[q][b], own_off);
+        }
+#pragma unroll
+      for (int q = 0; q < U; q++) {
+        const ClsTerm T = cl_term(TH + t + q);
+#pragma unroll
+        for (int b = 0; b < CB; b++) {
+          const bool neg = SGN && (__popc(xh[b] & T.sgn) & 1);
+          cl_mac<REALC>(acc[b], neg ? -T.cre : T.cre, neg ? -T.cim : T.cim, g[q][b]);
+        }
+      }
+    }
+    // ---- mixed terms: another rank of another block
+    for (int q = 0; q < C.nlo; q++) sla[q * CL_TPB + tid] = cl_rank16<RK>(s21, ia ^ C.lo[q]);
+    cl_mixed<CB, true, REALC, RK>(TM, C.n_mixp, ia, v1, xh, tgt + C.n_high, row, sla, acc);
+    cl_mixed<CB, false, REALC, RK>(TM + C.n_mixp, C.n_mixed - C.n_mixp, ia, v1, xh, tgt + C.n_high + C.n_mixp, row, sla,
+                                   acc);
+#pragma unroll
+    for (int b = 0; b < CB; b++) {
+      if (b < (int)nb) {
+        const double2 a = cl_at(v1 + base[b], own_off);
+        double2 *out = (double2 *)((char *)(v0 + base[b]) + own_off);
+        double2 o = make_double2(A.c1 * acc[b].x, A.c1 * acc[b].y);
+        if (!A.overwrite) {
+          const double2 p = *out;
+          o.x += A.c0 * p.x;
+          o.y += A.c0 * p.y;
+        }
+        *out = o;
+        pre += a.x * acc[b].x + a.y * acc[b].y;
+        pim += a.x * acc[b].y - a.y * acc[b].x;
+      }
+    }
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    pre += __shfl_xor(pre, off, 64);
+    pim += __shfl_xor(pim, off, 64);
+  }
+  __shared__ double2 red[CL_TPB / 64];
+  if (lane == 0) red[wave] = make_double2(pre, pim);
+  __syncthreads();
+  if (tid == 0) {
+    double2 s = red[0];
+    for (int w = 1; w < CL_TPB / 64; w++) {
+      s.x += red[w].x;
+      s.y += red[w].y;
+    }
+    A.partial[blockIdx.x] = s;
+  }
+}
+
+// tgt[p][t]: the first index of the block that high or mixed term t reads from
+// block p, or CL_NONE where the high half fails its predicate or has no target
+__global__ __launch_bounds__(256) void k_cls_targets(const uint32_t *bxh, const uint64_t *l22, uint32_t np, int nlow,
+                                                     const ClsTerm *terms, int n_low, int nt, int n_high, uint32_t irght,
+                                                     uint32_t *tgt) {
+  const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (uint64_t)np * nt) return;
+  const uint32_t p = (uint32_t)(i / nt), t = (uint32_t)(i % nt);
+  const ClsTerm T = terms[n_low + t];
+  const uint32_t xh = bxh[p], hm = T.tmask & ~irght;
+  bool ok;
+  if (T.never) ok = false;
+  else if (T.parity) ok = (int)t >= n_high || (__popc(xh & hm) & 1);  // a mixed one: either value, the low half decides
+  else ok = (xh & hm) == (T.tval & ~irght);
+  const uint64_t s = ok ? l22[((xh ^ T.flip) & ~irght) >> nlow] : 0;
+  tgt[i] = s ? (uint32_t)(s - 1) : CL_NONE;
+}
+
+// ---------------------------------------------------------------- host ----
+
+// the particle numbers a term changes, per species; false: not known from its masks
+static bool conserves(const GTerm &t, uint64_t up) {
+  if (t.kind != P_EQ) {  // two bits that differ, both flipped: of one species
+    const int nb = __builtin_popcountll(t.tmask), nu = __builtin_popcountll(t.tmask & up);
+    return t.kind == P_DIFF && nb == 2 && t.flip == t.tmask && (nu == 0 || nu == 2);
+  }
+  if (t.flip & ~t.tmask) return false;
+  const uint64_t y = t.tval ^ t.flip;
+  return __builtin_popcountll(t.tval & up) == __builtin_popcountll(y & up) &&
+         __builtin_popcountll(t.tval & ~up) == __builtin_popcountll(y & ~up);
+}
+
+// Can this engine's H·v go by classes (host check; the plan is built with the tables)?
+static bool cls_possible(const hphi_engine *e) {
+  const int nhigh = e->nbits - e->nlow;
+  if (!e->c2_ok || !e->c2_crank_ok || e->nlow > 16 || nhigh < 1 || nhigh > 16 || e->dim >= CL_NONE) return false;
+  const uint64_t up = e->model == HPHI_MODEL_HUBBARD ? 0x5555555555555555ull : ~0ull;
+  for (const GTerm &t : e->h_terms_dev)
+    if (!(t.kind == P_EQ && t.tmask == 0 && t.tval != 0) && !conserves(t, up)) return false;
+  return true;
+}
+
+// Blocks per wave.  Few states: one, for more waves (12,870 states: 10.8 us with
+// one, 13.1 with two, 18.1 with four; 184,756: 16.8, 17.5, 22.3).  Where the
+// vectors sit in the caches and arithmetic counts: two for Spin (1.35e6: 56.9,
+// 50.5, 56.4; 2.7e6: 168, 151, 169), four for Hubbard, whose rank lookup costs
+// more (8.5e5: 43.0, 37.8, 34.4; 1.7e8: 14,005, 13,378, 12,885).  Spin vectors
+// beyond the caches: one, whose rank tiles follow closest on each other in a
+// block (4.0e7: 3,380, 3,688, 3,711; 6.0e8: 75,400, 78,213, 80,848).
+int hphi_cls_blocks(const hphi_engine *e) {
+  if (e->cls_blocks > 0) return e->cls_blocks;
+  const uint64_t d = e->dim;
+  if (e->model == HPHI_MODEL_HUBBARD) return d < ((uint64_t)1 << 17) ? 1 : d < ((uint64_t)1 << 19) ? 2 : 4;
+  return d < ((uint64_t)1 << 18) || d >= ((uint64_t)1 << 24) ? 1 : 2;
+}
+
+// a shape of k_hv_canon set by hand keeps that kernel
+int hphi_cls_wanted(const hphi_engine *e) {
+  if (!e->d_cls || !e->use_c2 || !e->c2_crank || e->cls == 0) return 0;
+  return e->cls == 1 || !e->c2_tuned;
+}
+
+// Blocks by class, their first indices and high halves, the terms in three
+// groups (padded with terms that never act) and the target table: one device
+// allocation.  Sectors or terms the layout does not fit keep k_hv_canon.
+int hphi_cls_build(hphi_engine *e) {
+  if (e->d_cls || e->cls == 0 || !cls_possible(e)) return 0;
+  const int nhigh = e->nbits - e->nlow;
+  const bool hub = e->model == HPHI_MODEL_HUBBARD;
+  const SzParams S = hphi_sz_params(e);
+  const uint64_t even = 0x5555555555555555ull;
+  auto C = [](int n, int k) -> uint64_t {
+    if (k < 0 || k > n) return 0;
+    uint64_t r = 1;
+    for (int i = 1; i <= k; i++) r = r * (uint64_t)(n - k + i) / (uint64_t)i;
+    return r;
+  };
+  uint64_t cu[33], cd[33];  // low-half values by the particles left for them
+  for (int k = 0; k <= 32; k++) {
+    cu[k] = hub ? C(S.nlu, k) : C(e->nlow, k);
+    cd[k] = hub ? C(S.nld, k) : 1;
+  }
+  struct Cls {
+    uint64_t size;
+    std::vector<uint32_t> xh, at;
+  };
+  std::map<uint32_t, Cls> cls;
+  uint64_t pos = 0;
+  for (uint32_t ib = 0; ib < (1u << nhigh); ib++) {
+    const uint64_t x = (uint64_t)ib << e->nlow;
+    const int u = hub ? __builtin_popcountll(x & even) : __builtin_popcountll(x);
+    const int d = hub ? __builtin_popcountll(x & ~even) : 0;
+    if (u > e->nup || (hub && d > e->ndown) || e->nup - u > 32 || (hub && e->ndown - d > 32)) continue;
+    const uint64_t n = cu[e->nup - u] * (hub ? cd[e->ndown - d] : 1);
+    if (!n) continue;
+    Cls &k = cls[(uint32_t)(u * 64 + d)];
+    k.size = n;
+    k.xh.push_back((uint32_t)x);
+    k.at.push_back((uint32_t)pos);
+    pos += n;
+  }
+  if (pos != e->dim || cls.size() > CL_MAXC) return 0;
+  std::vector<uint32_t> at, xh;
+  ClsArgs &A = e->cls_args;
+  A = ClsArgs{};
+  for (const auto &k : cls) {
+    A.start[A.ncls] = (uint32_t)at.size();
+    A.nblk[A.ncls] = (uint32_t)k.second.at.size();
+    A.size[A.ncls] = (uint32_t)k.second.size;
+    A.ntile[A.ncls] = (uint32_t)((k.second.size + 63) / 64);
+    A.ncls++;
+    at.insert(at.end(), k.second.at.begin(), k.second.at.end());
+    xh.insert(xh.end(), k.second.xh.begin(), k.second.xh.end());
+  }
+  // terms by group: pure low, pure high, the others
+  std::vector<ClsTerm> grp[5];  // low by parity, low by value, high, mixed by parity, mixed by value
+  std::vector<uint32_t> lo;
+  for (const GTerm &t : e->h_terms_dev) {
+    if (t.kind == P_EQ && t.tmask == 0 && t.tval != 0) continue;
+    const uint64_t all = t.flip | t.tmask | t.sgn, hm = ~e->irght;
+    ClsTerm c{};
+    c.cre = t.cre;
+    c.cim = t.cim;
+    c.flip = (uint32_t)t.flip;
+    c.tmask = (uint32_t)t.tmask;
+    c.tval = (uint32_t)t.tval;
+    c.tlo = (uint32_t)(t.tval & e->irght);
+    c.sgn = (uint32_t)t.sgn;
+    c.parity = t.kind == P_DIFF;
+    const int g = (all & hm) == 0 ? 0 : (all & e->irght) == 0 ? 1 : 2;
+    if (g == 2) {
+      const uint32_t f = (uint32_t)(t.flip & e->irght);
+      size_t q = std::find(lo.begin(), lo.end(), f) - lo.begin();
+      if (q == lo.size()) lo.push_back(f);
+      c.lo = (int)q;
+    }
+    grp[g == 1 ? 2 : g == 0 ? (c.parity ? 0 : 1) : (c.parity ? 3 : 4)].push_back(c);
+  }
+  if (lo.size() > CL_MAXLO) return 0;
+  ClsTerm never{};  // an empty mask has neither odd parity nor this value
+  never.tval = never.tlo = 1;
+  never.never = 1;
+  for (auto &g : grp)
+    while (g.size() % 8) g.push_back(never);
+  A.n_lowp = (int)grp[0].size();
+  A.n_low = A.n_lowp + (int)grp[1].size();
+  A.n_high = (int)grp[2].size();
+  A.n_mixp = (int)grp[3].size();
+  A.n_mixed = A.n_mixp + (int)grp[4].size();
+  A.nt = A.n_high + A.n_mixed;
+  A.nlo = (int)lo.size();
+  std::copy(lo.begin(), lo.end(), A.lo);
+  std::vector<ClsTerm> terms;
+  for (auto &g : grp) terms.insert(terms.end(), g.begin(), g.end());
+  const size_t np = at.size(), tb = sizeof(ClsTerm) * std::max<size_t>(terms.size(), 1);
+  const size_t bytes = tb + 4 * (2 * np + np * (size_t)A.nt);
+  char *p = nullptr;
+  if (hipMalloc((void **)&p, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;  // no room: k_hv_canon serves this engine
+  }
+  e->d_cls = p;
+  e->bytes += bytes;
+  A.terms = (const ClsTerm *)p;
+  A.bstart = (const uint32_t *)(p + tb);
+  A.bxh = A.bstart + np;
+  uint32_t *tgt = (uint32_t *)(A.bxh + np);
+  A.tgt = tgt;
+  std::vector<char> up(tb + 8 * np);
+  std::copy(terms.begin(), terms.end(), (ClsTerm *)up.data());
+  std::copy(at.begin(), at.end(), (uint32_t *)(up.data() + tb));
+  std::copy(xh.begin(), xh.end(), (uint32_t *)(up.data() + tb) + np);
+  HIPCHK(hipMemcpy(p, up.data(), up.size(), hipMemcpyHostToDevice));
+  const uint64_t n = (uint64_t)np * A.nt;
+  if (n)
+    hipLaunchKernelGGL(k_cls_targets, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, e->stream, A.bxh, e->d_l22,
+                       (uint32_t)np, e->nlow, A.terms, A.n_low, A.nt, A.n_high, (uint32_t)e->irght, tgt);
+  HIPCHK(hipGetLastError());
+  return 0;
+}
+
+// units (a rank tile of a group of blocks) of the launch, and its workgroups
+static void cls_units(const hphi_engine *e, ClsArgs &A, int cb) {
+  uint32_t u = 0;
+  for (int c = 0; c < A.ncls; c++) {
+    A.upre[c] = u;
+    u += (A.nblk[c] + cb - 1) / cb * A.ntile[c];
+  }
+  A.upre[A.ncls] = u;
+  A.units = u;
+}
+
+int hphi_cls_grid(const hphi_engine *e) {
+  ClsArgs A = e->cls_args;
+  cls_units(e, A, hphi_cls_blocks(e));
+  const uint64_t want = (A.units + CL_TPB / 64 - 1) / (CL_TPB / 64);
+  uint64_t g = std::min<uint64_t>(want, (uint64_t)e->cls_wgs_per_cu * std::max(e->num_cu, 1));
+  g = std::max<uint64_t>((g + 7) / 8 * 8, 8);
+  return (int)std::min<uint64_t>(g, HV_MAX_GRID);
+}
+
+template <int CB>
+static int cls_launch(hphi_engine *e, const HvArgs &H, const ClsArgs &A, int g) {
+  const size_t lds = sizeof(uint32_t) * CL_TPB * std::max(A.nlo, 1);
+  const bool hub = e->model == HPHI_MODEL_HUBBARD;
+#define CL_GO(R, K) hipLaunchKernelGGL((k_hv_cls<CB, R, K>), dim3(g), dim3(CL_TPB), lds, e->stream, H, A)
+  if (e->c2_realc) {
+    if (hub) CL_GO(true, 3);
+    else CL_GO(true, 2);
+  } else {
+    if (hub) CL_GO(false, 3);
+    else CL_GO(false, 2);
+  }
+#undef CL_GO
+  HIPCHK(hipGetLastError());
+  return 0;
+}
+
+int hphi_hv_launch_cls(hphi_engine *e, const HvArgs &H, int g, int skip_high) {
+  ClsArgs A = e->cls_args;
+  const int cb = hphi_cls_blocks(e);
+  cls_units(e, A, cb);
+  if (skip_high) A.skip = A.n_high;  // the high terms have a pass of their own
+  return cb == 4 ? cls_launch<4>(e, H, A, g) : cb == 2 ? cls_launch<2>(e, H, A, g) : cls_launch<1>(e, H, A, g);
+}
