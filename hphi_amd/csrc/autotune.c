@@ -94,6 +94,11 @@ int hphi_autotune(hphi_engine *e, int k, double *v0, const double *v1, int reps,
     /* block kernel: columns per lane x workgroup size x workgroups per CU x XCD map */
     static char knob[16];
     snprintf(knob, sizeof knob, "blk_cpl%d", k);
+    hphi_engine_get_tune(e, "cls", &cls);
+    for (int cb = 1; cls && cb <= 4; cb *= 2) {
+      cand_t *c = &cands[n++];
+      add(c, "cls", 1), add(c, "cls_blocks", cb), add(c, "use_blk", 1), add(c, "c2_crank", 1);
+    }
     int cpls[3] = {1, 4, k}, ncpl = k > 4 ? 3 : 2;
     if (k <= 4) cpls[1] = k;
     for (int xcd = 1; xcd >= 0; xcd--)
@@ -104,12 +109,14 @@ int hphi_autotune(hphi_engine *e, int k, double *v0, const double *v1, int reps,
           add(c, "use_blk", 1), add(c, "xcd_map", xcd), add(c, knob, cpls[a]);
           add(c, "blk_tpb", 256), add(c, "blk_wgs_per_cu", w);
           if (gc) add(c, "gc_tile", 0);
+          if (cls) add(c, "cls", 0);
         }
         if (cpls[a] <= 4) {
           cand_t *c = &cands[n++];
           add(c, "use_blk", 1), add(c, "xcd_map", xcd), add(c, knob, cpls[a]);
           add(c, "blk_tpb", 1024), add(c, "blk_wgs_per_cu", 1);
           if (gc) add(c, "gc_tile", 0);
+          if (cls) add(c, "cls", 0);
         }
       }
   }

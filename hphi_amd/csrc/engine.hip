@@ -918,31 +918,28 @@ extern "C" int hphi_engine_create(const hphi_model_desc *d, hphi_engine **out) {
   if (hipGetDevice(&e->device) != hipSuccess) e->device = 0;
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, e->device) == hipSuccess) e->num_cu = prop.multiProcessorCount;
-  size_t tb = std::max<size_t>(e->h_terms_dev.size(), 1) * sizeof(GTerm);
-  size_t db = std::max<size_t>(e->h_dterms.size(), 1) * sizeof(DTerm);
-  if (hipMalloc(&e->d_terms, tb) != hipSuccess || hipMalloc(&e->d_dterms, db) != hipSuccess) {
+  hphi_canon_config(e);
+  // terms, diagonal terms and rank tables: one allocation, one copy (a copy is 13 us)
+  const size_t tb = e->h_terms_dev.size() * sizeof(GTerm), db = e->h_dterms.size() * sizeof(DTerm);
+  const size_t ob = (tb + 255) / 256 * 256, oc = ob + (db + 255) / 256 * 256;
+  const bool hub = e->model == HPHI_MODEL_HUBBARD;
+  const size_t cb = e->c2_crank_ok ? sizeof(uint16_t) * (hub ? HRANK_N : CRANK_N) : 0;
+  std::vector<char> up(oc + cb);
+  if (tb) memcpy(up.data(), e->h_terms_dev.data(), tb);
+  if (db) memcpy(up.data() + ob, e->h_dterms.data(), db);
+  if (cb && hub) hphi_hrank_tables((uint16_t *)(up.data() + oc));
+  else if (cb) hphi_crank_tables((uint16_t *)(up.data() + oc));
+  char *dev = nullptr;
+  if (hipMalloc((void **)&dev, std::max<size_t>(up.size(), 1)) != hipSuccess ||
+      (!up.empty() && hipMemcpy(dev, up.data(), up.size(), hipMemcpyHostToDevice) != hipSuccess)) {
+    (void)hipFree(dev);
     hphi_engine_destroy(e);
     return hphi_set_error("hipMalloc(terms) failed");
   }
-  if (!e->h_terms_dev.empty())
-    (void)hipMemcpy(e->d_terms, e->h_terms_dev.data(), e->h_terms_dev.size() * sizeof(GTerm), hipMemcpyHostToDevice);
-  if (!e->h_dterms.empty())
-    (void)hipMemcpy(e->d_dterms, e->h_dterms.data(), e->h_dterms.size() * sizeof(DTerm), hipMemcpyHostToDevice);
-  e->bytes += tb + db;
-  hphi_canon_config(e);
-  if (e->c2_crank_ok) {
-    const bool hub = e->model == HPHI_MODEL_HUBBARD;
-    const size_t n = hub ? HRANK_N : CRANK_N;
-    std::vector<uint16_t> t(n);
-    if (hub) hphi_hrank_tables(t.data());
-    else hphi_crank_tables(t.data());
-    if (hipMalloc(&e->d_crank, sizeof(uint16_t) * n) != hipSuccess ||
-        hipMemcpy(e->d_crank, t.data(), sizeof(uint16_t) * n, hipMemcpyHostToDevice) != hipSuccess) {
-      hphi_engine_destroy(e);
-      return hphi_set_error("hipMalloc(rank tables) failed");
-    }
-    e->bytes += sizeof(uint16_t) * n;
-  }
+  e->d_terms = (GTerm *)dev;
+  e->d_dterms = (DTerm *)(dev + ob);
+  if (cb) e->d_crank = (uint16_t *)(dev + oc);
+  e->bytes += up.size();
   if (e->c2_crank_ok) {  // rank tables (5 / 13 KB of LDS): many resident workgroups
     e->c2_crank = 1;
     e->c2_tpb = 256;
@@ -974,7 +971,6 @@ extern "C" void hphi_engine_destroy(hphi_engine *e) {
   (void)hipFree(e->d_list1);
   (void)hipFree(e->d_l21);
   (void)hipFree(e->d_l22);
-  (void)hipFree(e->d_crank);
   (void)hipFree(e->d_hb);
   (void)hipFree(e->d_blkpos);
   (void)hipFree(e->d_v1t);
@@ -983,8 +979,7 @@ extern "C" void hphi_engine_destroy(hphi_engine *e) {
   (void)hipFree(e->d_cls);
   (void)hipFree(e->d_jb);
   (void)hipFree(e->d_diag);
-  (void)hipFree(e->d_terms);
-  (void)hipFree(e->d_dterms);
+  (void)hipFree(e->d_terms);  // holds d_dterms and d_crank
   (void)hipFree(e->d_partial);
   (void)hipFree(e->d_prdct);
   (void)hipFree(e->d_coef);
@@ -1115,7 +1110,7 @@ extern "C" int hphi_engine_get_tune(const hphi_engine *e, const char *knob, int 
   else if (k == "use_c2") *value = e->use_c2 && e->c2_ok;
   else if (k == "grid_per_cu") *value = e->grid_per_cu;
   else if (k == "use_blk") *value = e->use_blk && hphi_blk_ok(e);
-  else if (k == "cls") *value = hphi_cls_wanted(e);
+  else if (k == "cls") *value = hphi_cls_wanted(e, 1);
   else if (k == "cls_blocks") *value = hphi_cls_blocks(e);
   else if (k == "cls_wgs_per_cu") *value = e->cls_wgs_per_cu;
   else if (k == "gc_tile") *value = hphi_gc_wanted(e, 1) || hphi_gc_wanted(e, 2) || hphi_gc_wanted(e, 4) ||
@@ -1195,6 +1190,8 @@ int hphi_build_tables(hphi_engine *e) {
   HIPCHK(hipMalloc(&e->d_jb, sizeof(uint64_t) * (e->sdim + 1)));
   e->bytes += sizeof(uint64_t) * (e->dim + e->size22 + e->sdim + 1) + sizeof(uint32_t) * e->size21;
   if (hphi_launch_tables(P, e->sdim, e->size21, e->d_jb, e->d_l21, e->d_l22, e->d_list1, e->stream)) return -1;
+  std::vector<char> up;
+  if (hphi_cls_build(e, up)) return -1;  // before the wait below, which covers it
   uint64_t total = 0;
   HIPCHK(hipMemcpyAsync(&total, e->d_jb + e->sdim, sizeof total, hipMemcpyDeviceToHost, e->stream));
   HIPCHK(hipStreamSynchronize(e->stream));
@@ -1202,7 +1199,6 @@ int hphi_build_tables(hphi_engine *e) {
     return hphi_set_error("basis count %llu differs from idim_max %llu", (unsigned long long)total,
                           (unsigned long long)e->dim);
   e->tables_ready = true;
-  if (hphi_cls_build(e)) return -1;
   // plan of the high-half pass now, outside any H·v launch (it copies list_2_2 to the host)
   if (hphi_hi_split_on(e) < 0) return -1;
   return 0;
@@ -1319,10 +1315,15 @@ int hphi_hv_launch_ex(hphi_engine *e, int k, double *v0, const double *v1, int o
 
 // which kernel a launch for k columns uses, and its workgroups (each writes k
 // partial sums of prdct)
-enum { HV_PATH_CANON, HV_PATH_GC, HV_PATH_BLK, HV_PATH_GENERIC };
+enum { HV_PATH_CANON, HV_PATH_CLS, HV_PATH_GC, HV_PATH_BLK, HV_PATH_GENERIC };
 static int hv_path(const hphi_engine *e, int k, int *grid, int gather = 0) {
+  const bool cls = hphi_cls_wanted(e, k) && (!gather || hphi_cls_same_order(e));
+  if (cls) {
+    *grid = hphi_cls_grid(e, k);
+    return HV_PATH_CLS;
+  }
   if (k == 1 && e->c2_ok && e->use_c2) {
-    *grid = hphi_cls_wanted(e) ? hphi_cls_grid(e) : canon_grid(e);
+    *grid = canon_grid(e);
     return HV_PATH_CANON;
   }
   if (!gather && hphi_gc_wanted(e, k)) {
@@ -1337,24 +1338,24 @@ static int hv_path(const hphi_engine *e, int k, int *grid, int gather = 0) {
   return HV_PATH_GENERIC;
 }
 
-// launch of prepared arguments: the canonical single-vector kernel, the block
-// kernel, or the generic kernel; then the partials in A.partial are reduced
+// launch of prepared arguments: the class, the single-vector, the tile, the block
+// or the generic kernel; then the partials in A.partial are reduced
 // into prdct_out[0..k)
 static int hv_launch_args(hphi_engine *e, int k, HvArgs &A, double2 *prdct_out, int gather) {
   int g = 0;
   const int path = hv_path(e, k, &g, gather);
-  if (path == HV_PATH_CANON) {
-    // canonical Spin: the high-half terms in a second pass over a tile-major
-    // copy of v1 (only with the engine's own partial-sum buffer, which holds
-    // both grids)
-    const int split = A.partial == (double2 *)e->d_partial ? hphi_hi_split_on(e) : 0;
+  if (path == HV_PATH_CANON || path == HV_PATH_CLS) {
+    // canonical Spin, one column: the high-half terms in a second pass over a
+    // tile-major copy of v1 (only with the engine's own partial-sum buffer,
+    // which holds both grids)
+    const int split = k == 1 && A.partial == (double2 *)e->d_partial ? hphi_hi_split_on(e) : 0;
     if (split < 0) return -1;
     if (split && e->hi_fuse_copy) {  // the first pass also writes the tile-major copy of v1
       A.v1t = e->d_v1t;
       A.tofs = e->d_tofs;
     }
-    if (hphi_cls_wanted(e)) {
-      if (hphi_hv_launch_cls(e, A, g, split)) return -1;
+    if (path == HV_PATH_CLS) {
+      if (hphi_hv_launch_cls(e, A, k, g, split)) return -1;
     } else {
       if (split) g = canon_grid(e, e->hi_p1_wgs_per_cu);  // the first pass without the high terms
       if (hphi_hv_launch_canon(e, A, g, split)) return -1;
@@ -1449,7 +1450,6 @@ extern "C" int hphi_mltply_block_dev(hphi_engine *e, int k, double *V0, const do
 // array's name to a kernel (on the host it is only a stand-in), but the
 // device address hipGetSymbolAddress returned for that device, recorded
 // once per device when an engine is created there.
-#define HV_NOALLOC_PARTIALS (1 << 18)  // k x workgroups of one launch (4 MiB)
 static __device__ __align__(256) double2 scratch[HV_NOALLOC_PARTIALS + 16];
 #define HV_MAX_DEVICES 64
 static double2 *g_scratch_dev[HV_MAX_DEVICES];

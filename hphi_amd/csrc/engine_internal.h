@@ -12,6 +12,7 @@
 #define HV_UNROLL 8       // terms per unrolled gather batch of the generic kernels
 #define HV_TERM_PAD 16    // term groups are padded with never-active terms to a multiple of
                           // this, so every batch size in use (8, 16) reads whole groups
+#define HV_NOALLOC_PARTIALS (1 << 18)  // k x workgroups of an allocation-free H·v (4 MiB of partial sums)
 #define HV_MAX_GRID 65536 // upper bound of H·v workgroups (sizes the partial-sum buffer)
 
 // predicate kinds of a gather term, evaluated on the TARGET state x
@@ -275,11 +276,13 @@ int hphi_hi_wanted(const hphi_engine *e);
 int hphi_hi_split_on(hphi_engine *e);
 // launches the high-half pass: accumulates into A.v0, partials at partial[0..*grid)
 int hphi_hv_launch_high(hphi_engine *e, const HvArgs &A, double2 *partial, int *grid);
-int hphi_cls_build(hphi_engine *e);
-int hphi_cls_wanted(const hphi_engine *e);
+int hphi_cls_build(hphi_engine *e, std::vector<char> &up);
+int hphi_cls_wanted(const hphi_engine *e, int k);
+int hphi_cls_same_order(const hphi_engine *e);
 int hphi_cls_blocks(const hphi_engine *e);
-int hphi_cls_grid(const hphi_engine *e);
-int hphi_hv_launch_cls(hphi_engine *e, const HvArgs &H, int g, int skip_high);
+int hphi_cls_grid(const hphi_engine *e, int k);
+void hphi_cls_shape(const hphi_engine *e, int k, int *cb, int *cpl);
+int hphi_hv_launch_cls(hphi_engine *e, const HvArgs &H, int k, int g, int skip_high);
 int hphi_gc_wanted(const hphi_engine *e, int k);
 int hphi_gc_plan_build(hphi_engine *e);
 int hphi_gc_partials(const hphi_engine *e, int k);  // workgroups of all passes of one H·v

@@ -27,6 +27,16 @@
 // The small ones are a chain of latencies, the middle ones were bound by that
 // arithmetic and are now by the L1's 64 bytes per cycle and L2; on 8x4 each of
 // the two halves of the terms misses L2 for 200 GB, 5.5 TB/s with the streams.
+//
+// Blocks of K columns: LPS = K / CPL lanes share a state and a wave takes 64 / LPS
+// ranks.  k_hv_blk / this kernel, microseconds: 6x4 J1-J2 k = 2 492 / 302, k = 4 880 /
+// 600, k = 8 1,795 / 1,338, k = 16 3,926 / 3,266; 23-site chain k = 8 496 / 334;
+// 16-site chain k = 8 20.7 / 11.3; 12-site Hubbard k = 8 215 / 145; 7x4 k = 4 19,285 /
+// 16,455.  6x4 with k = 8 misses L2 for 9.1 GB, 7.1 TB/s: a state's columns fill a
+// 128-byte line, so nothing of a gather is shared by neighbours, and the gathers
+// of 32 CUs reach further than their 4 MB.  Rank-slice order of the units (2 to
+// 64 tiles of every block before the next slice) gave nothing there and cost 10-25 %
+// on 8x4.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -47,13 +57,13 @@ typedef const ClsTerm __attribute__((address_space(4))) *CClsTerm;
 #define CL_U 8  // gathers in flight per lane: CL_U / CB terms per batch (4 and 16 within 3 % or slower)
 #define CL_NONE 0xffffffffu  // the term does not act in this block
 
-// 16 x the rank of low-half value y within its class (byte offset of its amplitude)
+// rank of low-half value y within its class
 template <int RK>
-__device__ __forceinline__ uint32_t cl_rank16(const uint16_t *t, uint32_t y) {
+__device__ __forceinline__ uint32_t cl_rank(const uint16_t *t, uint32_t y) {
   if (RK == 3)
-    return ((uint32_t)t[y & 255u] + (uint32_t)t[256u + 25u * (y >> 8) + 5u * (uint32_t)__popc(y & 0x55u) +
-                                                 (uint32_t)__popc(y & 0xAAu)]) << 4;
-  return ((uint32_t)t[y & 255u] + (uint32_t)t[256u + 9u * (y >> 8) + (uint32_t)__popc(y & 255u)]) << 4;
+    return (uint32_t)t[y & 255u] + (uint32_t)t[256u + 25u * (y >> 8) + 5u * (uint32_t)__popc(y & 0x55u) +
+                                                (uint32_t)__popc(y & 0xAAu)];
+  return (uint32_t)t[y & 255u] + (uint32_t)t[256u + 9u * (y >> 8) + (uint32_t)__popc(y & 255u)];
 }
 
 __device__ __forceinline__ double2 cl_at(const double2 *base, uint32_t off) {
@@ -69,6 +79,9 @@ __device__ __forceinline__ void cl_mac(double2 &a, double cr, double ci, double2
     a.y += ci * g.x;
   }
 }
+
+// terms per batch: eight gathers in flight
+constexpr int cl_batch(int per_term) { return per_term >= CL_U ? 1 : CL_U / per_term; }
 
 __device__ __forceinline__ ClsTerm cl_term(CClsTerm p) {
   ClsTerm t;
@@ -86,28 +99,32 @@ __device__ __forceinline__ ClsTerm cl_term(CClsTerm p) {
 
 // n low-half terms of one predicate kind (PAR: the parity of the masked bits is
 // odd; else the masked bits have a value) on CB blocks
-template <int CB, bool PAR, bool REALC, int RK>
-__device__ __forceinline__ void cl_low(CClsTerm TL, int n, uint32_t ia, const double2 *v1, const uint32_t *base,
-                                       const uint16_t *s21, double2 *acc) {
-  constexpr int U = CL_U / CB;
+template <int K, int CPL, int CB, bool PAR, bool REALC, int RK>
+__device__ __forceinline__ void cl_low(CClsTerm TL, int n, uint32_t ia, uint32_t coff, const double2 *v1,
+                                       const uint32_t *base, const uint16_t *s21, double2 (&acc)[CB][CPL]) {
+  constexpr int U = cl_batch(CB * CPL);
 #pragma unroll 1
   for (int t = 0; t < n; t += U) {
-    double2 g[U][CB];
+    double2 g[U][CB][CPL];
     uint32_t off[U];
     bool act[U];
 #pragma unroll
     for (int q = 0; q < U; q++) {
       const ClsTerm T = cl_term(TL + t + q);
       act[q] = PAR ? (__popc(ia & T.tmask) & 1) != 0 : (ia & T.tmask) == T.tval;
-      off[q] = cl_rank16<RK>(s21, ia ^ T.flip);
+      off[q] = cl_rank<RK>(s21, ia ^ T.flip) * (16u * K) + coff;
     }
 #pragma unroll
     for (int q = 0; q < U; q++) {
 #pragma unroll
-      for (int b = 0; b < CB; b++) g[q][b] = make_double2(0.0, 0.0);
+      for (int b = 0; b < CB; b++)
+#pragma unroll
+        for (int i = 0; i < CPL; i++) g[q][b][i] = make_double2(0.0, 0.0);
       if (act[q]) {
 #pragma unroll
-        for (int b = 0; b < CB; b++) g[q][b] = cl_at(v1 + base[b], off[q]);
+        for (int b = 0; b < CB; b++)
+#pragma unroll
+          for (int i = 0; i < CPL; i++) g[q][b][i] = cl_at(v1 + (uint64_t)base[b] * K, off[q] + 16 * (K / CPL) * i);
       }
     }
 #pragma unroll
@@ -116,20 +133,23 @@ __device__ __forceinline__ void cl_low(CClsTerm TL, int n, uint32_t ia, const do
       const bool neg = RK == 3 && (__popc(ia & T.sgn) & 1);
       const double cr = neg ? -T.cre : T.cre, ci = neg ? -T.cim : T.cim;
 #pragma unroll
-      for (int b = 0; b < CB; b++) cl_mac<REALC>(acc[b], cr, ci, g[q][b]);
+      for (int b = 0; b < CB; b++)
+#pragma unroll
+        for (int i = 0; i < CPL; i++) cl_mac<REALC>(acc[b][i], cr, ci, g[q][b][i]);
     }
   }
 }
 
 // n mixed terms of one predicate kind: the low half's part of the predicate per
 // lane, the high half's per block; tgt: the terms' first column of the table
-template <int CB, bool PAR, bool REALC, int RK>
+template <int K, int CPL, int CB, bool PAR, bool REALC, int RK>
 __device__ __forceinline__ void cl_mixed(CClsTerm TM, int n, uint32_t ia, const double2 *v1, const uint32_t *xh,
-                                         CU32 tgt, const uint32_t *row, const uint32_t *sla, double2 *acc) {
-  constexpr int U = CL_U / CB;
+                                         CU32 tgt, const uint32_t *row, const uint32_t *sla,
+                                         double2 (&acc)[CB][CPL]) {
+  constexpr int U = cl_batch(CB * CPL);
 #pragma unroll 1
   for (int t = 0; t < n; t += U) {
-    double2 g[U][CB];
+    double2 g[U][CB][CPL];
     uint32_t off[U], lp[U], to[U][CB];
 #pragma unroll
     for (int b = 0; b < CB; b++)
@@ -149,8 +169,12 @@ __device__ __forceinline__ void cl_mixed(CClsTerm TM, int n, uint32_t ia, const 
         // scalar: what lp must be in this block (2: never)
         const uint32_t ok = PAR ? ((uint32_t)__popc(xh[b] & T.tmask) & 1u) ^ 1u : 1u;
         const uint32_t want = to[q][b] == CL_NONE ? 2u : ok;
-        g[q][b] = make_double2(0.0, 0.0);
-        if (lp[q] == want) g[q][b] = cl_at(v1 + to[q][b], off[q]);
+#pragma unroll
+        for (int i = 0; i < CPL; i++) g[q][b][i] = make_double2(0.0, 0.0);
+        if (lp[q] == want) {
+#pragma unroll
+          for (int i = 0; i < CPL; i++) g[q][b][i] = cl_at(v1 + (uint64_t)to[q][b] * K, off[q] + 16 * (K / CPL) * i);
+        }
       }
     }
 #pragma unroll
@@ -160,15 +184,18 @@ __device__ __forceinline__ void cl_mixed(CClsTerm TM, int n, uint32_t ia, const 
 #pragma unroll
       for (int b = 0; b < CB; b++) {
         const bool neg = RK == 3 && ((ls + (uint32_t)__popc(xh[b] & T.sgn)) & 1u);
-        cl_mac<REALC>(acc[b], neg ? -T.cre : T.cre, neg ? -T.cim : T.cim, g[q][b]);
+#pragma unroll
+        for (int i = 0; i < CPL; i++) cl_mac<REALC>(acc[b][i], neg ? -T.cre : T.cre, neg ? -T.cim : T.cim, g[q][b][i]);
       }
     }
   }
 }
 
-template <int CB, bool REALC, int RK>
+template <int K, int CPL, int CB, bool REALC, int RK>
 __global__ __launch_bounds__(CL_TPB) void k_hv_cls(const HvArgs A, const ClsArgs C) {
-  constexpr int U = CL_U / CB;  // terms per batch
+  constexpr int U = cl_batch(CB * CPL);  // terms per batch
+  constexpr int LPS = K / CPL;           // lanes per state
+  constexpr int RPT = 64 / LPS;          // ranks per tile
   constexpr bool SGN = RK == 3;
   constexpr int NT = RK == 3 ? HRANK_N : CRANK_N;
   __shared__ uint16_t s21[NT];
@@ -185,7 +212,10 @@ __global__ __launch_bounds__(CL_TPB) void k_hv_cls(const HvArgs A, const ClsArgs
   const uint32_t xcd = blockIdx.x & 7u, slot = (blockIdx.x >> 3) * (CL_TPB / 64) + wave;
   const uint32_t nslot = (gridDim.x >> 3) * (CL_TPB / 64);
   const uint32_t U1 = (uint32_t)((uint64_t)C.units * (xcd + 1) / 8);
-  double pre = 0.0, pim = 0.0;
+  const uint32_t coff = (lane % LPS) * 16u;  // this lane's first column; the others at steps of LPS
+  double pre[CPL], pim[CPL];
+#pragma unroll
+  for (int i = 0; i < CPL; i++) pre[i] = pim[i] = 0.0;
   for (uint32_t u = (uint32_t)((uint64_t)C.units * xcd / 8) + slot; u < U1; u += nslot) {
     int c = 0, hi = C.ncls;  // upre[c] <= u < upre[hi]
     while (hi - c > 1) {
@@ -196,11 +226,11 @@ __global__ __launch_bounds__(CL_TPB) void k_hv_cls(const HvArgs A, const ClsArgs
     const uint32_t loc = u - C.upre[c], ntile = C.ntile[c], size = C.size[c];
     const uint32_t grp = loc / ntile, tile = loc % ntile;
     const uint32_t p0 = C.start[c] + grp * CB, nb = C.start[c] + C.nblk[c] - p0;  // blocks from here on
-    const uint32_t r = tile * 64u + lane;
+    const uint32_t r = tile * RPT + lane / LPS;
     if (r >= size) continue;
-    const uint32_t own_off = r << 4;
+    const uint32_t own_off = r * (16u * K) + coff;
     uint32_t base[CB], xh[CB], row[CB];
-    double2 acc[CB];
+    double2 acc[CB][CPL];
 #pragma unroll
     for (int b = 0; b < CB; b++) {
       const uint32_t p = p0 + (b < (int)nb ? b : 0);  // past the class's last block: the first again, not stored
@@ -210,27 +240,32 @@ __global__ __launch_bounds__(CL_TPB) void k_hv_cls(const HvArgs A, const ClsArgs
     }
     const uint32_t ia = (uint32_t)A.list1[base[0] + r] & (uint32_t)A.irght;
 #pragma unroll
-    for (int b = 0; b < CB; b++) acc[b] = cl_at(v1 + base[b], own_off);
-    if (A.v1t) {  // tile-major copy for the high-half pass
+    for (int b = 0; b < CB; b++)
+#pragma unroll
+      for (int i = 0; i < CPL; i++) acc[b][i] = cl_at(v1 + (uint64_t)base[b] * K, own_off + 16 * (K / CPL) * i);
+    if (K == 1 && A.v1t) {  // tile-major copy for the high-half pass
 #pragma unroll
       for (int b = 0; b < CB; b++)
         if (b < (int)nb) {
           const ulonglong2 ts = A.tofs[xh[b] >> A.nlow];
-          A.v1t[ts.x + (uint64_t)(r / HI_RT) * ts.y + r % HI_RT] = acc[b];
+          A.v1t[ts.x + (uint64_t)(r / HI_RT) * ts.y + r % HI_RT] = acc[b][0];
         }
     }
 #pragma unroll
     for (int b = 0; b < CB; b++) {
       const double d = *(const double *)((const char *)(A.diag + base[b]) + (r << 3));
-      acc[b].x *= d;
-      acc[b].y *= d;
+#pragma unroll
+      for (int i = 0; i < CPL; i++) {
+        acc[b][i].x *= d;
+        acc[b][i].y *= d;
+      }
     }
     // ---- low-half terms: one predicate and one target rank for all blocks
-    cl_low<CB, true, REALC, RK>(TL, C.n_lowp, ia, v1, base, s21, acc);
-    cl_low<CB, false, REALC, RK>(TL + C.n_lowp, C.n_low - C.n_lowp, ia, v1, base, s21, acc);
+    cl_low<K, CPL, CB, true, REALC, RK>(TL, C.n_lowp, ia, coff, v1, base, s21, acc);
+    cl_low<K, CPL, CB, false, REALC, RK>(TL + C.n_lowp, C.n_low - C.n_lowp, ia, coff, v1, base, s21, acc);
     // ---- high-half terms: the same rank of another block
     for (int t = C.skip; t < C.n_high; t += U) {
-      double2 g[U][CB];
+      double2 g[U][CB][CPL];
       uint32_t to[U][CB];
 #pragma unroll
       for (int b = 0; b < CB; b++)
@@ -240,8 +275,12 @@ __global__ __launch_bounds__(CL_TPB) void k_hv_cls(const HvArgs A, const ClsArgs
       for (int q = 0; q < U; q++)
 #pragma unroll
         for (int b = 0; b < CB; b++) {
-          g[q][b] = make_double2(0.0, 0.0);
-          if (to[q][b] != CL_NONE) g[q][b] = cl_at(v1 + to[q][b], own_off);
+#pragma unroll
+          for (int i = 0; i < CPL; i++) g[q][b][i] = make_double2(0.0, 0.0);
+          if (to[q][b] != CL_NONE) {
+#pragma unroll
+            for (int i = 0; i < CPL; i++) g[q][b][i] = cl_at(v1 + (uint64_t)to[q][b] * K, own_off + 16 * (K / CPL) * i);
+          }
         }
 #pragma unroll
       for (int q = 0; q < U; q++) {
@@ -249,47 +288,56 @@ __global__ __launch_bounds__(CL_TPB) void k_hv_cls(const HvArgs A, const ClsArgs
 #pragma unroll
         for (int b = 0; b < CB; b++) {
           const bool neg = SGN && (__popc(xh[b] & T.sgn) & 1);
-          cl_mac<REALC>(acc[b], neg ? -T.cre : T.cre, neg ? -T.cim : T.cim, g[q][b]);
+#pragma unroll
+          for (int i = 0; i < CPL; i++)
+            cl_mac<REALC>(acc[b][i], neg ? -T.cre : T.cre, neg ? -T.cim : T.cim, g[q][b][i]);
         }
       }
     }
     // ---- mixed terms: another rank of another block
-    for (int q = 0; q < C.nlo; q++) sla[q * CL_TPB + tid] = cl_rank16<RK>(s21, ia ^ C.lo[q]);
-    cl_mixed<CB, true, REALC, RK>(TM, C.n_mixp, ia, v1, xh, tgt + C.n_high, row, sla, acc);
-    cl_mixed<CB, false, REALC, RK>(TM + C.n_mixp, C.n_mixed - C.n_mixp, ia, v1, xh, tgt + C.n_high + C.n_mixp, row, sla,
+    for (int q = 0; q < C.nlo; q++) sla[q * CL_TPB + tid] = cl_rank<RK>(s21, ia ^ C.lo[q]) * (16u * K) + coff;
+    cl_mixed<K, CPL, CB, true, REALC, RK>(TM, C.n_mixp, ia, v1, xh, tgt + C.n_high, row, sla, acc);
+    cl_mixed<K, CPL, CB, false, REALC, RK>(TM + C.n_mixp, C.n_mixed - C.n_mixp, ia, v1, xh, tgt + C.n_high + C.n_mixp, row, sla,
                                    acc);
 #pragma unroll
     for (int b = 0; b < CB; b++) {
       if (b < (int)nb) {
-        const double2 a = cl_at(v1 + base[b], own_off);
-        double2 *out = (double2 *)((char *)(v0 + base[b]) + own_off);
-        double2 o = make_double2(A.c1 * acc[b].x, A.c1 * acc[b].y);
-        if (!A.overwrite) {
-          const double2 p = *out;
-          o.x += A.c0 * p.x;
-          o.y += A.c0 * p.y;
+#pragma unroll
+        for (int i = 0; i < CPL; i++) {
+          const double2 a = cl_at(v1 + (uint64_t)base[b] * K, own_off + 16 * (K / CPL) * i);
+          double2 *out = (double2 *)((char *)(v0 + (uint64_t)base[b] * K) + own_off + 16 * (K / CPL) * i);
+          double2 o = make_double2(A.c1 * acc[b][i].x, A.c1 * acc[b][i].y);
+          if (!A.overwrite) {
+            const double2 p = *out;
+            o.x += A.c0 * p.x;
+            o.y += A.c0 * p.y;
+          }
+          *out = o;
+          pre[i] += a.x * acc[b][i].x + a.y * acc[b][i].y;
+          pim[i] += a.x * acc[b][i].y - a.y * acc[b][i].x;
         }
-        *out = o;
-        pre += a.x * acc[b].x + a.y * acc[b].y;
-        pim += a.x * acc[b].y - a.y * acc[b].x;
       }
     }
   }
+  // prdct per column: lanes with equal lane % LPS hold the same columns
+  __shared__ double2 red[CL_TPB / 64][K];
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    pre += __shfl_xor(pre, off, 64);
-    pim += __shfl_xor(pim, off, 64);
-  }
-  __shared__ double2 red[CL_TPB / 64];
-  if (lane == 0) red[wave] = make_double2(pre, pim);
-  __syncthreads();
-  if (tid == 0) {
-    double2 s = red[0];
-    for (int w = 1; w < CL_TPB / 64; w++) {
-      s.x += red[w].x;
-      s.y += red[w].y;
+  for (int i = 0; i < CPL; i++) {
+#pragma unroll
+    for (int off = 32; off >= LPS; off >>= 1) {
+      pre[i] += __shfl_xor(pre[i], off, 64);
+      pim[i] += __shfl_xor(pim[i], off, 64);
     }
-    A.partial[blockIdx.x] = s;
+    if (lane < (uint32_t)LPS) red[wave][lane + LPS * i] = make_double2(pre[i], pim[i]);
+  }
+  __syncthreads();
+  if (tid < (uint32_t)K) {
+    double2 s = red[0][tid];
+    for (int w = 1; w < CL_TPB / 64; w++) {
+      s.x += red[w][tid].x;
+      s.y += red[w][tid].y;
+    }
+    A.partial[(uint64_t)blockIdx.x * K + tid] = s;
   }
 }
 
@@ -335,13 +383,13 @@ static bool cls_possible(const hphi_engine *e) {
   return true;
 }
 
-// Blocks per wave.  Few states: one, for more waves (12,870 states: 10.8 us with
-// one, 13.1 with two, 18.1 with four; 184,756: 16.8, 17.5, 22.3).  Where the
-// vectors sit in the caches and arithmetic counts: two for Spin (1.35e6: 56.9,
-// 50.5, 56.4; 2.7e6: 168, 151, 169), four for Hubbard, whose rank lookup costs
-// more (8.5e5: 43.0, 37.8, 34.4; 1.7e8: 14,005, 13,378, 12,885).  Spin vectors
-// beyond the caches: one, whose rank tiles follow closest on each other in a
-// block (4.0e7: 3,380, 3,688, 3,711; 6.0e8: 75,400, 78,213, 80,848).
+// Blocks per wave, one column.  Few states: one, for more waves (12,870 states:
+// 10.8 us with one, 13.1 with two, 18.1 with four; 184,756: 16.8, 17.5, 22.3).
+// Where the vectors sit in the caches and arithmetic counts: two for Spin
+// (1.35e6: 56.9, 50.5, 56.4; 2.7e6: 168, 151, 169), four for Hubbard, whose rank
+// lookup costs more (8.5e5: 43.0, 37.8, 34.4; 1.7e8: 14,005, 13,378, 12,885).
+// Spin vectors beyond the caches: one, whose rank tiles follow closest on each
+// other in a block (4.0e7: 3,380, 3,688, 3,711; 6.0e8: 75,400, 78,213, 80,848).
 int hphi_cls_blocks(const hphi_engine *e) {
   if (e->cls_blocks > 0) return e->cls_blocks;
   const uint64_t d = e->dim;
@@ -349,16 +397,42 @@ int hphi_cls_blocks(const hphi_engine *e) {
   return d < ((uint64_t)1 << 18) || d >= ((uint64_t)1 << 24) ? 1 : 2;
 }
 
-// a shape of k_hv_canon set by hand keeps that kernel
-int hphi_cls_wanted(const hphi_engine *e) {
-  if (!e->d_cls || !e->use_c2 || !e->c2_crank || e->cls == 0) return 0;
-  return e->cls == 1 || !e->c2_tuned;
+// Blocks per wave and columns per lane of a block of k columns.  One column per
+// lane: a load instruction then covers whole states (Spin 2.7e6, k = 8, two
+// blocks: 1,338 us with one column per lane, 1,459 with two, 1,668 with four).
+// Hubbard's rank lookup is worth sharing by two (8.5e5, k = 8: 170, 145, 187).
+// Blocks: one while k columns still leave few waves (12,870 states, k = 8: 11.3,
+// 13.0, 17.6 us with one, two, four), then two (2.7e6: 1,384, 1,338, 1,364), four
+// beyond the caches (4.0e7, k = 4: 17,865, 17,159, 16,455).
+void hphi_cls_shape(const hphi_engine *e, int k, int *cb, int *cpl) {
+  *cb = hphi_cls_blocks(e);
+  *cpl = 1;
+  if (k == 1) return;
+  const uint64_t n = e->dim * (uint64_t)k;
+  if (e->cls_blocks == 0) *cb = n < ((uint64_t)1 << 18) ? 1 : e->dim < ((uint64_t)1 << 24) ? 2 : 4;
+  if (e->model == HPHI_MODEL_HUBBARD && n >= ((uint64_t)1 << 18)) *cpl = 2;
+}
+
+// a launch shape of the other kernel for k columns set by hand keeps that kernel
+int hphi_cls_wanted(const hphi_engine *e, int k) {
+  if (!e->d_cls || !e->c2_crank || e->cls == 0) return 0;
+  if (k == 1) return e->use_c2 && (e->cls == 1 || !e->c2_tuned);
+  const int slot = k == 2 ? 0 : k == 4 ? 1 : k == 8 ? 2 : 3;
+  return e->use_blk && (e->cls == 1 || !(e->bk_tpb || e->bk_wgs_per_cu || e->bk_cpl[slot]));
+}
+
+// Sums bit-equal to the gather kernels': no group holds both kinds of
+// predicate, whose terms stand in another order here.
+int hphi_cls_same_order(const hphi_engine *e) {
+  const ClsArgs &A = e->cls_args;
+  return (A.n_lowp == 0 || A.n_lowp == A.n_low) && (A.n_mixp == 0 || A.n_mixp == A.n_mixed);
 }
 
 // Blocks by class, their first indices and high halves, the terms in three
 // groups (padded with terms that never act) and the target table: one device
-// allocation.  Sectors or terms the layout does not fit keep k_hv_canon.
-int hphi_cls_build(hphi_engine *e) {
+// allocation, written on e->stream, which the caller waits for before it frees up.
+// Sectors or terms the layout does not fit keep k_hv_canon.
+int hphi_cls_build(hphi_engine *e, std::vector<char> &up) {
   if (e->d_cls || e->cls == 0 || !cls_possible(e)) return 0;
   const int nhigh = e->nbits - e->nlow;
   const bool hub = e->model == HPHI_MODEL_HUBBARD;
@@ -402,7 +476,6 @@ int hphi_cls_build(hphi_engine *e) {
     A.start[A.ncls] = (uint32_t)at.size();
     A.nblk[A.ncls] = (uint32_t)k.second.at.size();
     A.size[A.ncls] = (uint32_t)k.second.size;
-    A.ntile[A.ncls] = (uint32_t)((k.second.size + 63) / 64);
     A.ncls++;
     at.insert(at.end(), k.second.at.begin(), k.second.at.end());
     xh.insert(xh.end(), k.second.xh.begin(), k.second.xh.end());
@@ -461,11 +534,11 @@ int hphi_cls_build(hphi_engine *e) {
   A.bxh = A.bstart + np;
   uint32_t *tgt = (uint32_t *)(A.bxh + np);
   A.tgt = tgt;
-  std::vector<char> up(tb + 8 * np);
+  up.resize(tb + 8 * np);
   std::copy(terms.begin(), terms.end(), (ClsTerm *)up.data());
   std::copy(at.begin(), at.end(), (uint32_t *)(up.data() + tb));
   std::copy(xh.begin(), xh.end(), (uint32_t *)(up.data() + tb) + np);
-  HIPCHK(hipMemcpy(p, up.data(), up.size(), hipMemcpyHostToDevice));
+  HIPCHK(hipMemcpyAsync(p, up.data(), up.size(), hipMemcpyHostToDevice, e->stream));
   const uint64_t n = (uint64_t)np * A.nt;
   if (n)
     hipLaunchKernelGGL(k_cls_targets, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, e->stream, A.bxh, e->d_l22,
@@ -474,31 +547,36 @@ int hphi_cls_build(hphi_engine *e) {
   return 0;
 }
 
-// units (a rank tile of a group of blocks) of the launch, and its workgroups
-static void cls_units(const hphi_engine *e, ClsArgs &A, int cb) {
+// units (a rank tile of a group of blocks) of a launch with cb blocks per wave
+// and rpt ranks per tile
+static void cls_units(ClsArgs &A, int cb, int rpt) {
   uint32_t u = 0;
   for (int c = 0; c < A.ncls; c++) {
     A.upre[c] = u;
+    A.ntile[c] = (A.size[c] + rpt - 1) / rpt;
     u += (A.nblk[c] + cb - 1) / cb * A.ntile[c];
   }
   A.upre[A.ncls] = u;
   A.units = u;
 }
 
-int hphi_cls_grid(const hphi_engine *e) {
+int hphi_cls_grid(const hphi_engine *e, int k) {
   ClsArgs A = e->cls_args;
-  cls_units(e, A, hphi_cls_blocks(e));
+  int cb, cpl;
+  hphi_cls_shape(e, k, &cb, &cpl);
+  cls_units(A, cb, 64 * cpl / k);
   const uint64_t want = (A.units + CL_TPB / 64 - 1) / (CL_TPB / 64);
   uint64_t g = std::min<uint64_t>(want, (uint64_t)e->cls_wgs_per_cu * std::max(e->num_cu, 1));
   g = std::max<uint64_t>((g + 7) / 8 * 8, 8);
-  return (int)std::min<uint64_t>(g, HV_MAX_GRID);
+  // HV_NOALLOC_PARTIALS / k partial sums per column
+  return (int)std::min<uint64_t>(g, k > 4 ? HV_NOALLOC_PARTIALS / k : HV_MAX_GRID);
 }
 
-template <int CB>
+template <int K, int CPL, int CB>
 static int cls_launch(hphi_engine *e, const HvArgs &H, const ClsArgs &A, int g) {
   const size_t lds = sizeof(uint32_t) * CL_TPB * std::max(A.nlo, 1);
   const bool hub = e->model == HPHI_MODEL_HUBBARD;
-#define CL_GO(R, K) hipLaunchKernelGGL((k_hv_cls<CB, R, K>), dim3(g), dim3(CL_TPB), lds, e->stream, H, A)
+#define CL_GO(R, RK) hipLaunchKernelGGL((k_hv_cls<K, CPL, CB, R, RK>), dim3(g), dim3(CL_TPB), lds, e->stream, H, A)
   if (e->c2_realc) {
     if (hub) CL_GO(true, 3);
     else CL_GO(true, 2);
@@ -511,10 +589,25 @@ static int cls_launch(hphi_engine *e, const HvArgs &H, const ClsArgs &A, int g) 
   return 0;
 }
 
-int hphi_hv_launch_cls(hphi_engine *e, const HvArgs &H, int g, int skip_high) {
+int hphi_hv_launch_cls(hphi_engine *e, const HvArgs &H, int k, int g, int skip_high) {
   ClsArgs A = e->cls_args;
-  const int cb = hphi_cls_blocks(e);
-  cls_units(e, A, cb);
+  int cb, cpl;
+  hphi_cls_shape(e, k, &cb, &cpl);
+  cls_units(A, cb, 64 * cpl / k);
   if (skip_high) A.skip = A.n_high;  // the high terms have a pass of their own
-  return cb == 4 ? cls_launch<4>(e, H, A, g) : cb == 2 ? cls_launch<2>(e, H, A, g) : cls_launch<1>(e, H, A, g);
+#define CASE(KK, CC, BB) \
+  if (k == KK && cpl == CC && cb == BB) return cls_launch<KK, CC, BB>(e, H, A, g);
+#define CASES(KK, CC) CASE(KK, CC, 1) CASE(KK, CC, 2) CASE(KK, CC, 4)
+  CASES(1, 1)
+  CASES(2, 1)
+  CASES(4, 1)
+  CASES(8, 1)
+  CASES(16, 1)
+  CASES(2, 2)
+  CASES(4, 2)
+  CASES(8, 2)
+  CASES(16, 2)
+#undef CASES
+#undef CASE
+  return hphi_set_error("no class kernel for k=%d, %d columns per lane, %d blocks", k, cpl, cb);
 }

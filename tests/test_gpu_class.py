@@ -90,3 +90,35 @@ def test_class_kernel_before_the_high_half_pass(A, spec, cb):
         e.close()
     for r in res[1:]:
         assert np.max(np.abs(r - res[0])) <= TOL * np.max(np.abs(res[0]))
+
+
+TWO_BODY = [(n, s) for n, s in two_body_cases().items() if s.model in (L.SPIN, L.HUBBARD)]
+
+
+@pytest.mark.parametrize("k", [2, 4, 8, 16])
+@pytest.mark.parametrize("name,spec", CASES + TWO_BODY, ids=[c[0] for c in CASES + TWO_BODY])
+def test_class_kernel_block(A, name, spec, k):
+    """Blocks of k columns equal k_hv_blk's, with and without allocations."""
+    out = []
+    for tune in (dict(cls=0), dict(cls=1), dict(cls=1, cls_blocks=4, cls_wgs_per_cu=1)):
+        print(f"[gpu] class kernel {name} k {k} {tune}", flush=True)
+        e = A.Engine.from_spec(spec)
+        e.tune(**tune)
+        e.sz(copy=False)
+        e.diagonalcalc(copy=False)
+        assert e.get_tune("cls") == tune["cls"]
+        rng = np.random.default_rng(7)
+        v = rng.standard_normal(2 * e.dim * k).view(np.complex128)
+        w = rng.standard_normal(2 * e.dim * k).view(np.complex128)
+        v1, v0 = A.DeviceArray(e.dim * k).upload(v), A.DeviceArray(e.dim * k).upload(w)
+        p = e.mltply_block_dev(k, v0, v1)
+        a = v0.download()
+        v0.upload(w)
+        q = e.mltply_block_dev_noalloc(k, v0, v1)
+        assert np.array_equal(v0.download(), a) and np.array_equal(p, q)
+        out.append((a, p, np.linalg.norm(v) * np.linalg.norm(a)))
+        e.close()
+    a, p, s = out[0]
+    for b, q, _ in out[1:]:
+        assert np.max(np.abs(b - a)) <= TOL * np.max(np.abs(a))
+        assert np.max(np.abs(q - p)) <= TOL * s
