@@ -150,7 +150,7 @@ struct ClsTerm {
   double cre, cim;
   uint32_t flip, tmask, tval, sgn;
   uint32_t tlo;            // the low half's part of tval
-  int parity, never, lo;   // parity predicate (else value); padding; index of a mixed term's low-half flip
+  int parity, src, lo;     // parity predicate (else value); compiled term (-1: padding); low-half flip of a mixed term
 };
 #define CL_TPB 256
 #define CL_MAXC 96
@@ -158,7 +158,7 @@ struct ClsTerm {
 struct ClsArgs {
   int ncls, n_low, n_high, n_mixed, nt, nlo, skip;
   int n_lowp, n_mixp;  // of the low and mixed terms, those with a parity predicate (first)
-  uint32_t units;
+  uint32_t units, np;  // np: blocks
   uint32_t start[CL_MAXC], nblk[CL_MAXC], size[CL_MAXC], ntile[CL_MAXC], upre[CL_MAXC + 1];
   uint32_t lo[CL_MAXLO];
   const ClsTerm *terms;
@@ -277,6 +277,11 @@ int hphi_hi_split_on(hphi_engine *e);
 // launches the high-half pass: accumulates into A.v0, partials at partial[0..*grid)
 int hphi_hv_launch_high(hphi_engine *e, const HvArgs &A, double2 *partial, int *grid);
 int hphi_cls_build(hphi_engine *e, std::vector<char> &up);
+bool hphi_cls_plan(const hphi_engine *e, ClsArgs &A, std::vector<char> &up);
+size_t hphi_cls_bytes(const ClsArgs &A);
+size_t hphi_cls_bytes_bound(const hphi_engine *e);
+int hphi_cls_upload(const hphi_engine *e, ClsArgs &A, char *dev, const void *up, const uint64_t *l22, hipStream_t st);
+void hphi_cls_units(ClsArgs &A, int cb, int rpt);
 int hphi_cls_wanted(const hphi_engine *e, int k);
 int hphi_cls_same_order(const hphi_engine *e);
 int hphi_cls_blocks(const hphi_engine *e);

@@ -44,6 +44,7 @@
 #include <vector>
 
 #include "engine_internal.h"
+#include "hv_class.h"
 
 #define HIPCHK(x)                                                                  \
   do {                                                                             \
@@ -51,11 +52,7 @@
     if (e_ != hipSuccess) return hphi_set_error("%s failed: %s", #x, hipGetErrorString(e_)); \
   } while (0)
 
-typedef const uint32_t __attribute__((address_space(4))) *CU32;
-typedef const ClsTerm __attribute__((address_space(4))) *CClsTerm;
-
 #define CL_U 8  // gathers in flight per lane: CL_U / CB terms per batch (4 and 16 within 3 % or slower)
-#define CL_NONE 0xffffffffu  // the term does not act in this block
 
 // rank of low-half value y within its class
 template <int RK>
@@ -64,10 +61,6 @@ __device__ __forceinline__ uint32_t cl_rank(const uint16_t *t, uint32_t y) {
     return (uint32_t)t[y & 255u] + (uint32_t)t[256u + 25u * (y >> 8) + 5u * (uint32_t)__popc(y & 0x55u) +
                                                 (uint32_t)__popc(y & 0xAAu)];
   return (uint32_t)t[y & 255u] + (uint32_t)t[256u + 9u * (y >> 8) + (uint32_t)__popc(y & 255u)];
-}
-
-__device__ __forceinline__ double2 cl_at(const double2 *base, uint32_t off) {
-  return *(const double2 *)((const char *)base + off);
 }
 
 template <bool REALC>
@@ -82,20 +75,6 @@ __device__ __forceinline__ void cl_mac(double2 &a, double cr, double ci, double2
 
 // terms per batch: eight gathers in flight
 constexpr int cl_batch(int per_term) { return per_term >= CL_U ? 1 : CL_U / per_term; }
-
-__device__ __forceinline__ ClsTerm cl_term(CClsTerm p) {
-  ClsTerm t;
-  t.cre = p->cre;
-  t.cim = p->cim;
-  t.flip = p->flip;
-  t.tmask = p->tmask;
-  t.tval = p->tval;
-  t.sgn = p->sgn;
-  t.lo = p->lo;
-  t.tlo = p->tlo;
-  t.parity = t.never = 0;
-  return t;
-}
 
 // n low-half terms of one predicate kind (PAR: the parity of the masked bits is
 // odd; else the masked bits have a value) on CB blocks
@@ -352,7 +331,7 @@ __global__ __launch_bounds__(256) void k_cls_targets(const uint32_t *bxh, const 
   const ClsTerm T = terms[n_low + t];
   const uint32_t xh = bxh[p], hm = T.tmask & ~irght;
   bool ok;
-  if (T.never) ok = false;
+  if (T.src < 0) ok = false;
   else if (T.parity) ok = (int)t >= n_high || (__popc(xh & hm) & 1);  // a mixed one: either value, the low half decides
   else ok = (xh & hm) == (T.tval & ~irght);
   const uint64_t s = ok ? l22[((xh ^ T.flip) & ~irght) >> nlow] : 0;
@@ -373,10 +352,11 @@ static bool conserves(const GTerm &t, uint64_t up) {
          __builtin_popcountll(t.tval & ~up) == __builtin_popcountll(y & ~up);
 }
 
-// Can this engine's H·v go by classes (host check; the plan is built with the tables)?
+// Does the layout fit this sector and these terms?
 static bool cls_possible(const hphi_engine *e) {
   const int nhigh = e->nbits - e->nlow;
-  if (!e->c2_ok || !e->c2_crank_ok || e->nlow > 16 || nhigh < 1 || nhigh > 16 || e->dim >= CL_NONE) return false;
+  if (hphi_model_gc(e->model) || !(e->model == HPHI_MODEL_SPIN || e->model == HPHI_MODEL_HUBBARD)) return false;
+  if (e->nbits > 32 || e->nlow > 16 || nhigh < 1 || nhigh > 16 || e->dim >= CL_NONE) return false;
   const uint64_t up = e->model == HPHI_MODEL_HUBBARD ? 0x5555555555555555ull : ~0ull;
   for (const GTerm &t : e->h_terms_dev)
     if (!(t.kind == P_EQ && t.tmask == 0 && t.tval != 0) && !conserves(t, up)) return false;
@@ -428,12 +408,11 @@ int hphi_cls_same_order(const hphi_engine *e) {
   return (A.n_lowp == 0 || A.n_lowp == A.n_low) && (A.n_mixp == 0 || A.n_mixp == A.n_mixed);
 }
 
-// Blocks by class, their first indices and high halves, the terms in three
-// groups (padded with terms that never act) and the target table: one device
-// allocation, written on e->stream, which the caller waits for before it frees up.
-// Sectors or terms the layout does not fit keep k_hv_canon.
-int hphi_cls_build(hphi_engine *e, std::vector<char> &up) {
-  if (e->d_cls || e->cls == 0 || !cls_possible(e)) return 0;
+// Blocks by class, their first indices and high halves, and the terms in three
+// groups (padded with terms that never act): counts into A, terms, first
+// indices and high halves into up.  false: the layout does not fit.
+bool hphi_cls_plan(const hphi_engine *e, ClsArgs &A, std::vector<char> &up) {
+  if (!cls_possible(e)) return false;
   const int nhigh = e->nbits - e->nlow;
   const bool hub = e->model == HPHI_MODEL_HUBBARD;
   const SzParams S = hphi_sz_params(e);
@@ -468,9 +447,8 @@ int hphi_cls_build(hphi_engine *e, std::vector<char> &up) {
     k.at.push_back((uint32_t)pos);
     pos += n;
   }
-  if (pos != e->dim || cls.size() > CL_MAXC) return 0;
+  if (pos != e->dim || cls.size() > CL_MAXC) return false;
   std::vector<uint32_t> at, xh;
-  ClsArgs &A = e->cls_args;
   A = ClsArgs{};
   for (const auto &k : cls) {
     A.start[A.ncls] = (uint32_t)at.size();
@@ -483,7 +461,8 @@ int hphi_cls_build(hphi_engine *e, std::vector<char> &up) {
   // terms by group: pure low, pure high, the others
   std::vector<ClsTerm> grp[5];  // low by parity, low by value, high, mixed by parity, mixed by value
   std::vector<uint32_t> lo;
-  for (const GTerm &t : e->h_terms_dev) {
+  for (size_t i = 0; i < e->h_terms_dev.size(); i++) {
+    const GTerm &t = e->h_terms_dev[i];
     if (t.kind == P_EQ && t.tmask == 0 && t.tval != 0) continue;
     const uint64_t all = t.flip | t.tmask | t.sgn, hm = ~e->irght;
     ClsTerm c{};
@@ -495,6 +474,7 @@ int hphi_cls_build(hphi_engine *e, std::vector<char> &up) {
     c.tlo = (uint32_t)(t.tval & e->irght);
     c.sgn = (uint32_t)t.sgn;
     c.parity = t.kind == P_DIFF;
+    c.src = (int)i;
     const int g = (all & hm) == 0 ? 0 : (all & e->irght) == 0 ? 1 : 2;
     if (g == 2) {
       const uint32_t f = (uint32_t)(t.flip & e->irght);
@@ -504,10 +484,10 @@ int hphi_cls_build(hphi_engine *e, std::vector<char> &up) {
     }
     grp[g == 1 ? 2 : g == 0 ? (c.parity ? 0 : 1) : (c.parity ? 3 : 4)].push_back(c);
   }
-  if (lo.size() > CL_MAXLO) return 0;
+  if (lo.size() > CL_MAXLO) return false;
   ClsTerm never{};  // an empty mask has neither odd parity nor this value
   never.tval = never.tlo = 1;
-  never.never = 1;
+  never.src = -1;
   for (auto &g : grp)
     while (g.size() % 8) g.push_back(never);
   A.n_lowp = (int)grp[0].size();
@@ -520,36 +500,69 @@ int hphi_cls_build(hphi_engine *e, std::vector<char> &up) {
   std::copy(lo.begin(), lo.end(), A.lo);
   std::vector<ClsTerm> terms;
   for (auto &g : grp) terms.insert(terms.end(), g.begin(), g.end());
-  const size_t np = at.size(), tb = sizeof(ClsTerm) * std::max<size_t>(terms.size(), 1);
-  const size_t bytes = tb + 4 * (2 * np + np * (size_t)A.nt);
+  A.np = (uint32_t)at.size();
+  const size_t tb = sizeof(ClsTerm) * terms.size();
+  up.resize(tb + 8 * (size_t)A.np);
+  std::copy(terms.begin(), terms.end(), (ClsTerm *)up.data());
+  std::copy(at.begin(), at.end(), (uint32_t *)(up.data() + tb));
+  std::copy(xh.begin(), xh.end(), (uint32_t *)(up.data() + tb) + A.np);
+  return true;
+}
+
+// device bytes of a plan: up, then the target table
+size_t hphi_cls_bytes(const ClsArgs &A) {
+  return sizeof(ClsTerm) * (size_t)(A.n_low + A.nt) + 4 * (size_t)A.np * (2 + (size_t)A.nt);
+}
+
+// at most hphi_cls_bytes of the plan, without building it; 0: none
+size_t hphi_cls_bytes_bound(const hphi_engine *e) {
+  if (!cls_possible(e)) return 0;
+  size_t n[3] = {0, 0, 0};
+  for (const GTerm &t : e->h_terms_dev) {
+    const uint64_t all = t.flip | t.tmask | t.sgn;
+    n[(all & ~e->irght) == 0 ? 0 : (all & e->irght) == 0 ? 1 : 2]++;
+  }
+  for (auto &x : n) x += 14;  // padding of two predicate kinds
+  const size_t np = std::min<size_t>((size_t)1 << (e->nbits - e->nlow), e->dim);
+  return sizeof(ClsTerm) * (n[0] + n[1] + n[2]) + 4 * np * (2 + n[1] + n[2]);
+}
+
+// the plan on the device at dev: up is copied on st (and has to live until the
+// copy is done), then the target table computed from list_2_2
+int hphi_cls_upload(const hphi_engine *e, ClsArgs &A, char *dev, const void *up, const uint64_t *l22, hipStream_t st) {
+  const size_t tb = sizeof(ClsTerm) * (size_t)(A.n_low + A.nt);
+  A.terms = (const ClsTerm *)dev;
+  A.bstart = (const uint32_t *)(dev + tb);
+  A.bxh = A.bstart + A.np;
+  uint32_t *tgt = (uint32_t *)(A.bxh + A.np);
+  A.tgt = tgt;
+  HIPCHK(hipMemcpyAsync(dev, up, tb + 8 * (size_t)A.np, hipMemcpyHostToDevice, st));
+  const uint64_t n = (uint64_t)A.np * A.nt;
+  if (n)
+    hipLaunchKernelGGL(k_cls_targets, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, A.bxh, l22, A.np, e->nlow,
+                       A.terms, A.n_low, A.nt, A.n_high, (uint32_t)e->irght, tgt);
+  HIPCHK(hipGetLastError());
+  return 0;
+}
+
+// One device allocation, written on e->stream, which the caller waits for before it
+// frees up.  Sectors or terms the layout does not fit keep k_hv_canon.
+int hphi_cls_build(hphi_engine *e, std::vector<char> &up) {
+  if (e->d_cls || e->cls == 0 || !e->c2_ok || !e->c2_crank_ok || !hphi_cls_plan(e, e->cls_args, up)) return 0;
+  const size_t bytes = hphi_cls_bytes(e->cls_args);
   char *p = nullptr;
-  if (hipMalloc((void **)&p, bytes) != hipSuccess) {
+  if (hipMalloc((void **)&p, std::max<size_t>(bytes, 1)) != hipSuccess) {
     (void)hipGetLastError();
     return 0;  // no room: k_hv_canon serves this engine
   }
   e->d_cls = p;
   e->bytes += bytes;
-  A.terms = (const ClsTerm *)p;
-  A.bstart = (const uint32_t *)(p + tb);
-  A.bxh = A.bstart + np;
-  uint32_t *tgt = (uint32_t *)(A.bxh + np);
-  A.tgt = tgt;
-  up.resize(tb + 8 * np);
-  std::copy(terms.begin(), terms.end(), (ClsTerm *)up.data());
-  std::copy(at.begin(), at.end(), (uint32_t *)(up.data() + tb));
-  std::copy(xh.begin(), xh.end(), (uint32_t *)(up.data() + tb) + np);
-  HIPCHK(hipMemcpyAsync(p, up.data(), up.size(), hipMemcpyHostToDevice, e->stream));
-  const uint64_t n = (uint64_t)np * A.nt;
-  if (n)
-    hipLaunchKernelGGL(k_cls_targets, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, e->stream, A.bxh, e->d_l22,
-                       (uint32_t)np, e->nlow, A.terms, A.n_low, A.nt, A.n_high, (uint32_t)e->irght, tgt);
-  HIPCHK(hipGetLastError());
-  return 0;
+  return hphi_cls_upload(e, e->cls_args, p, up.data(), e->d_l22, e->stream);
 }
 
 // units (a rank tile of a group of blocks) of a launch with cb blocks per wave
 // and rpt ranks per tile
-static void cls_units(ClsArgs &A, int cb, int rpt) {
+void hphi_cls_units(ClsArgs &A, int cb, int rpt) {
   uint32_t u = 0;
   for (int c = 0; c < A.ncls; c++) {
     A.upre[c] = u;
@@ -564,7 +577,7 @@ int hphi_cls_grid(const hphi_engine *e, int k) {
   ClsArgs A = e->cls_args;
   int cb, cpl;
   hphi_cls_shape(e, k, &cb, &cpl);
-  cls_units(A, cb, 64 * cpl / k);
+  hphi_cls_units(A, cb, 64 * cpl / k);
   const uint64_t want = (A.units + CL_TPB / 64 - 1) / (CL_TPB / 64);
   uint64_t g = std::min<uint64_t>(want, (uint64_t)e->cls_wgs_per_cu * std::max(e->num_cu, 1));
   g = std::max<uint64_t>((g + 7) / 8 * 8, 8);
@@ -593,7 +606,7 @@ int hphi_hv_launch_cls(hphi_engine *e, const HvArgs &H, int k, int g, int skip_h
   ClsArgs A = e->cls_args;
   int cb, cpl;
   hphi_cls_shape(e, k, &cb, &cpl);
-  cls_units(A, cb, 64 * cpl / k);
+  hphi_cls_units(A, cb, 64 * cpl / k);
   if (skip_high) A.skip = A.n_high;  // the high terms have a pass of their own
 #define CASE(KK, CC, BB) \
   if (k == KK && cpl == CC && cb == BB) return cls_launch<KK, CC, BB>(e, H, A, g);

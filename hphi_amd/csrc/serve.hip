@@ -8,7 +8,8 @@
 // Lanczos vectors, the diagonal and the couplings.  One lane per basis state
 // decodes the state's bits, predicates, Jordan-Wigner signs and target
 // indices once and applies them to every running column of its slab, so up
-// to SL_K jobs pay for one index decode and read one 64-byte row per term.
+// to SL_K jobs pay for one index decode and read one 64-byte row per term;
+// slabs whose sector has a class layout run by classes (k_sl_cls).
 //
 // A tick
 //   1. admits waiting jobs: first, free columns of running slabs go to arrived
@@ -59,6 +60,7 @@
 #include <vector>
 
 #include "engine_internal.h"
+#include "hv_class.h"
 #include "hphi_amd.h"
 
 #define HIPCHK(x)                                                                  \
@@ -87,6 +89,8 @@ struct SlabDev {
   int mask;   // columns with a running job
   int realc;  // columns whose couplings are all real
   int slot[SL_K];
+  const ClsArgs *cls;  // class layout of the slab, or null
+  int sgn;             // terms carry Jordan-Wigner signs
 };
 struct ColDev {  // one running job in one step of a tick
   int slab, col, slot;
@@ -96,6 +100,7 @@ struct ColDev {  // one running job in one step of a tick
 };
 typedef const SlabDev __attribute__((address_space(4))) *CSlab;
 typedef const ColDev __attribute__((address_space(4))) *CCol;
+typedef const ClsArgs __attribute__((address_space(4))) *CCls;
 typedef const uint64_t __attribute__((address_space(4))) *CU64;
 typedef const double __attribute__((address_space(4))) *CD2;  // couplings as (re, im) doubles
 
@@ -119,6 +124,16 @@ __device__ __forceinline__ int find_slab(CU64 prefix, int n, uint64_t tile) {
 // chunks at or past the launch's total (the rounding) have no work.
 __device__ __forceinline__ uint64_t sl_chunk() {
   return (uint64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+}
+
+// Pass 2 costs a workgroup more or less by its slab's terms, so each XCD takes
+// an eighth of every slab, not of the launch: slab sb has prefix[sb + 1] - prefix[sb]
+// chunks, a multiple of 8; workgroup b takes chunk (b % 8) of its slab's eight ranges.
+__device__ __forceinline__ uint64_t sl_chunk8(CU64 prefix, int ns, int *sb) {
+  const uint64_t slot = blockIdx.x >> 3, p0 = prefix[0];
+  *sb = find_slab(prefix, ns, p0 + 8 * slot);
+  const uint64_t at = prefix[*sb], m = prefix[*sb + 1] - at;
+  return at + (uint64_t)(blockIdx.x & 7) * (m >> 3) + (slot - ((at - p0) >> 3));
 }
 
 // pass 1: w = r - alpha_{m-1} s_{m-1} q over R per running column, |w|^2 per
@@ -352,9 +367,8 @@ __global__ __launch_bounds__(SV_TPB) void k_sl_hv(const SlabDev *slabs, const ui
                                                   const double *js, double2 *partial) {
   extern __shared__ uint4 s21v[];
   const uint16_t *s21 = (const uint16_t *)s21v;
-  const uint64_t chunk = sl_chunk();
-  if (chunk >= ((CU64)prefix)[ns]) return;
-  const int sb = find_slab((CU64)prefix, ns, chunk);
+  int sb;
+  const uint64_t chunk = sl_chunk8((CU64)prefix, ns, &sb);
   CSlab S = (CSlab)slabs + sb;
   const uint32_t n8 = (uint32_t)((S->size21 + 7) / 8);  // 16-byte rows of the packed table
   for (uint32_t i = threadIdx.x; i < n8; i += SV_TPB) s21v[i] = S->l21p[i];
@@ -388,6 +402,246 @@ __global__ __launch_bounds__(SV_TPB) void k_sl_hv(const SlabDev *slabs, const ui
   if (threadIdx.x < SL_K) {
     double2 s = red[0][threadIdx.x];
     for (int w = 1; w < SV_TPB / 64; w++) {
+      s.x += red[w][threadIdx.x].x;
+      s.y += red[w][threadIdx.x].y;
+    }
+    partial[chunk * SL_K + threadIdx.x] = s;
+  }
+}
+
+// ---- pass 2 by classes (the layout of hv_class.hip): a wave takes 64 / SL_K ranks
+// of one class in SC_B blocks of it, one column per lane, so a load instruction
+// covers whole rows; low-half targets come once for all blocks, the blocks of
+// high-half and mixed targets from the slab's table, couplings from LDS.
+//
+// A burst of 40 jobs (24-site sectors and smaller), microseconds per launch:
+// k_sl_hv 1,126; this kernel with an eighth of the launch per XCD 1,023 (XCDs
+// with the heavier slabs last), an eighth of every slab 803, units dealt so that
+// workgroups running together stay neighbours 733.  It misses L2 for 4.0 GB per
+// launch, 5.5 TB/s, the rate of a large copy; one or four blocks per wave cost 8 %.
+#define SC_B 2                    // blocks per wave
+#define SC_RPT (64 / SL_K)        // ranks per tile
+#define SC_W (SV_TPB / 64)        // waves per workgroup
+#define SC_U 8                    // terms per batch (4 the same, 2 slower)
+#define SC_G 128                  // workgroups of an XCD taken to run together (64 and 256 2 % slower)
+#define SC_UPW 4                  // units per wave: 1 and 2 fill LDS more often (1 %), 16 leave a tail (9 %)
+
+template <bool REAL>
+__device__ __forceinline__ void sc_mac(double2 &a, const double *cf, bool neg, double2 g) {
+  const double cr = neg ? -cf[0] : cf[0];
+  a.x = __builtin_fma(cr, g.x, a.x);
+  a.y = __builtin_fma(cr, g.y, a.y);
+  if (!REAL) {  // as sl_mac: a zero imaginary part adds zeros
+    const double ci = neg ? -cf[1] : cf[1];
+    a.x = __builtin_fma(-ci, g.y, a.x);
+    a.y = __builtin_fma(ci, g.x, a.y);
+  }
+}
+
+// sco: the terms' couplings, [term][SL_K] of (REAL ? 1 : 2) doubles; sla: row
+// offsets of the mixed terms' low-half flips, [flip][ranks of the workgroup]
+template <bool REAL, bool SGN>
+__device__ __forceinline__ void sc_units(CSlab S, CCls C, uint32_t u0, uint32_t u1, uint32_t step,
+                                         const uint16_t *s21, uint32_t *sla, const double *sco, const double *js,
+                                         double *pre, double *pim) {
+  constexpr int CW = REAL ? 1 : 2;
+  const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t col = lane % SL_K, coff = col * 16u, irght = (uint32_t)S->irght;
+  const CU32 bstart = (CU32)C->bstart, bxh = (CU32)C->bxh, tgt = (CU32)C->tgt;
+  const int n_low = C->n_low, n_high = C->n_high, n_mixed = C->n_mixed, nt = C->nt;
+  const int n_lowp = C->n_lowp, n_mixp = C->n_mixp;
+  const CClsTerm TL = (CClsTerm)C->terms, TH = TL + n_low, TM = TH + n_high;
+  const double2 *__restrict__ R = S->R;
+  const bool run = (S->mask >> col) & 1;
+  const int sl = S->slot[col];
+  const double sc = js[sl * JS_STRIDE + 3], cc = -js[sl * JS_STRIDE + 2] * js[sl * JS_STRIDE + 1];
+  const double *cfl = sco + col * CW, *cfh = cfl + n_low * SL_K * CW, *cfm = cfh + n_high * SL_K * CW;
+  uint32_t *la = sla + wave * SC_RPT + lane / SL_K;
+  for (uint32_t u = u0 + wave; u < u1; u += step) {
+    int c = 0, hi = C->ncls;  // upre[c] <= u < upre[hi]
+    while (hi - c > 1) {
+      const int mid = (c + hi) >> 1;
+      if (C->upre[mid] <= u) c = mid;
+      else hi = mid;
+    }
+    const uint32_t loc = u - C->upre[c], ntile = C->ntile[c], size = C->size[c];
+    const uint32_t grp = loc / ntile, r = (loc % ntile) * SC_RPT + lane / SL_K;
+    const uint32_t p0 = C->start[c] + grp * SC_B, nb = C->start[c] + C->nblk[c] - p0;  // blocks from here on
+    if (r >= size) continue;
+    const uint32_t own = r * (16u * SL_K) + coff;
+    uint32_t base[SC_B], xh[SC_B], row[SC_B];
+    double2 acc[SC_B];
+#pragma unroll
+    for (int b = 0; b < SC_B; b++) {
+      const uint32_t p = p0 + (b < (int)nb ? b : 0);  // past the class's last block: the first again, not stored
+      base[b] = bstart[p];
+      xh[b] = bxh[p];
+      row[b] = p * (uint32_t)nt;
+    }
+    const uint32_t ia = (uint32_t)S->list1[base[0] + r] & irght;
+#pragma unroll
+    for (int b = 0; b < SC_B; b++) {
+      const double2 w = cl_at(R + (uint64_t)base[b] * SL_K, own);
+      const double d = S->diag[((uint64_t)base[b] + r) * SL_K + col];
+      acc[b] = make_double2(d * w.x, d * w.y);
+    }
+    // ---- low-half terms
+    for (int t = 0; t < n_low; t += SC_U) {
+      double2 g[SC_U][SC_B];
+      bool neg[SC_U];
+#pragma unroll
+      for (int q = 0; q < SC_U; q++) {
+        const ClsTerm T = cl_term(TL + t + q);
+        const uint32_t m = ia & T.tmask;
+        const bool act = t < n_lowp ? (__popc(m) & 1) != 0 : m == T.tval;
+        const uint32_t off = ((uint32_t)s21[ia ^ T.flip] - 2u) * (16u * SL_K) + coff;
+        neg[q] = SGN && (__popc(ia & T.sgn) & 1);
+#pragma unroll
+        for (int b = 0; b < SC_B; b++) g[q][b] = make_double2(0.0, 0.0);
+        if (act) {
+#pragma unroll
+          for (int b = 0; b < SC_B; b++) g[q][b] = cl_at(R + (uint64_t)base[b] * SL_K, off);
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < SC_U; q++)
+#pragma unroll
+        for (int b = 0; b < SC_B; b++) sc_mac<REAL>(acc[b], cfl + (t + q) * SL_K * CW, neg[q], g[q][b]);
+    }
+    // ---- high-half terms: the same rank of another block
+    for (int t = 0; t < n_high; t += SC_U) {
+      double2 g[SC_U][SC_B];
+      uint32_t to[SC_U][SC_B];
+#pragma unroll
+      for (int b = 0; b < SC_B; b++)
+#pragma unroll
+        for (int q = 0; q < SC_U; q++) to[q][b] = tgt[row[b] + t + q];
+#pragma unroll
+      for (int q = 0; q < SC_U; q++)
+#pragma unroll
+        for (int b = 0; b < SC_B; b++) {
+          g[q][b] = make_double2(0.0, 0.0);
+          if (to[q][b] != CL_NONE) g[q][b] = cl_at(R + (uint64_t)to[q][b] * SL_K, own);
+        }
+#pragma unroll
+      for (int q = 0; q < SC_U; q++) {
+        const ClsTerm T = cl_term(TH + t + q);
+#pragma unroll
+        for (int b = 0; b < SC_B; b++)
+          sc_mac<REAL>(acc[b], cfh + (t + q) * SL_K * CW, SGN && (__popc(xh[b] & T.sgn) & 1), g[q][b]);
+      }
+    }
+    // ---- mixed terms: the lanes of a state share its row offsets
+    for (int q = (int)col; q < C->nlo; q += SL_K) la[q * (SC_W * SC_RPT)] = ((uint32_t)s21[ia ^ C->lo[q]] - 2u) * (16u * SL_K);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    for (int t = 0; t < n_mixed; t += SC_U) {
+      const bool par = t < n_mixp;
+      double2 g[SC_U][SC_B];
+      uint32_t to[SC_U][SC_B];
+      uint32_t ls[SC_U];
+#pragma unroll
+      for (int b = 0; b < SC_B; b++)
+#pragma unroll
+        for (int q = 0; q < SC_U; q++) to[q][b] = tgt[row[b] + n_high + t + q];
+#pragma unroll
+      for (int q = 0; q < SC_U; q++) {
+        const ClsTerm T = cl_term(TM + t + q);
+        const uint32_t off = la[T.lo * (SC_W * SC_RPT)] + coff;
+        const uint32_t m = ia & T.tmask, lp = par ? (uint32_t)__popc(m) & 1u : (m == T.tlo ? 1u : 0u);
+        ls[q] = SGN ? (uint32_t)__popc(ia & T.sgn) : 0u;
+#pragma unroll
+        for (int b = 0; b < SC_B; b++) {
+          // scalar: what lp must be in this block (2: never)
+          const uint32_t ok = par ? ((uint32_t)__popc(xh[b] & T.tmask) & 1u) ^ 1u : 1u;
+          const uint32_t want = to[q][b] == CL_NONE ? 2u : ok;
+          g[q][b] = make_double2(0.0, 0.0);
+          if (lp == want) g[q][b] = cl_at(R + (uint64_t)to[q][b] * SL_K, off);
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < SC_U; q++) {
+        const ClsTerm T = cl_term(TM + t + q);
+#pragma unroll
+        for (int b = 0; b < SC_B; b++)
+          sc_mac<REAL>(acc[b], cfm + (t + q) * SL_K * CW, SGN && ((ls[q] + (uint32_t)__popc(xh[b] & T.sgn)) & 1u),
+                       g[q][b]);
+      }
+    }
+    if (run) {
+#pragma unroll
+      for (int b = 0; b < SC_B; b++) {
+        if (b < (int)nb) {
+          const double2 w = cl_at(R + (uint64_t)base[b] * SL_K, own);
+          double2 *q = (double2 *)((char *)(S->Q + (uint64_t)base[b] * SL_K) + own);
+          const double2 p = *q;
+          *q = make_double2(cc * p.x + sc * acc[b].x, cc * p.y + sc * acc[b].y);
+          *pre += w.x * acc[b].x + w.y * acc[b].y;
+          *pim += w.x * acc[b].y - w.y * acc[b].x;
+        }
+      }
+    }
+  }
+}
+
+// couplings in class order into LDS; a padding term's are zero
+template <bool REAL>
+__device__ __forceinline__ void sc_coef(CSlab S, CCls C, double *sco) {
+  const ClsTerm *T = C->terms;
+  const int n = (C->n_low + C->nt) * SL_K;
+  for (int i = threadIdx.x; i < n; i += SV_TPB) {
+    const int src = T[i / SL_K].src;
+    const double2 v = src < 0 ? make_double2(0.0, 0.0) : S->coef[src * SL_K + i % SL_K];
+    if (REAL) sco[i] = v.x;
+    else ((double2 *)sco)[i] = v;
+  }
+}
+
+// dynamic LDS: list_2_1 (n21 16-byte rows), row offsets (nla uint32), couplings
+__global__ __launch_bounds__(SV_TPB) void k_sl_cls(const SlabDev *slabs, const uint64_t *prefix, int ns,
+                                                   const double *js, double2 *partial, uint32_t n21, uint32_t nla) {
+  extern __shared__ uint4 s21v[];
+  const uint16_t *s21 = (const uint16_t *)s21v;
+  uint32_t *sla = (uint32_t *)(s21v + n21);
+  double *sco = (double *)(sla + nla);
+  int sb;
+  const uint64_t chunk = sl_chunk8((CU64)prefix, ns, &sb);
+  CSlab S = (CSlab)slabs + sb;
+  const CCls C = (CCls)S->cls;
+  const int full = (1 << SL_K) - 1;
+  const bool real = ((S->realc | ~S->mask) & full) == full;  // every running column has real couplings
+  const uint32_t n8 = (uint32_t)((S->size21 + 7) / 8);
+  for (uint32_t i = threadIdx.x; i < n8; i += SV_TPB) s21v[i] = S->l21p[i];
+  if (real) sc_coef<true>(S, C, sco);
+  else sc_coef<false>(S, C, sco);
+  __syncthreads();
+  // an eighth of the units per XCD, dealt to groups of SC_G workgroups, whose
+  // waves take every (4 x group)-th unit: workgroups that run together work on
+  // neighbouring units, whose gathers meet in L2
+  const uint32_t m = (uint32_t)(((CU64)prefix)[sb + 1] - ((CU64)prefix)[sb]) / 8;
+  const uint32_t i = (uint32_t)(chunk - ((CU64)prefix)[sb]), x = i / m, g0 = i % m / SC_G * SC_G;
+  const uint32_t gn = g0 + SC_G < m ? SC_G : m - g0;
+  const uint64_t X0 = (uint64_t)C->units * x / 8, XN = (uint64_t)C->units * (x + 1) / 8 - X0;
+  const uint32_t u0 = (uint32_t)(X0 + XN * g0 / m) + (i % m - g0) * SC_W, u1 = (uint32_t)(X0 + XN * (g0 + gn) / m);
+  double pre = 0.0, pim = 0.0;
+  if (S->sgn) {
+    if (real) sc_units<true, true>(S, C, u0, u1, gn * SC_W, s21, sla, sco, js, &pre, &pim);
+    else sc_units<false, true>(S, C, u0, u1, gn * SC_W, s21, sla, sco, js, &pre, &pim);
+  } else {
+    if (real) sc_units<true, false>(S, C, u0, u1, gn * SC_W, s21, sla, sco, js, &pre, &pim);
+    else sc_units<false, false>(S, C, u0, u1, gn * SC_W, s21, sla, sco, js, &pre, &pim);
+  }
+  __shared__ double2 red[SC_W][SL_K];
+  for (int off = 32; off >= SL_K; off >>= 1) {
+    pre += __shfl_xor(pre, off, 64);
+    pim += __shfl_xor(pim, off, 64);
+  }
+  if ((threadIdx.x & 63) < SL_K) red[threadIdx.x >> 6][threadIdx.x & 63] = make_double2(pre, pim);
+  __syncthreads();
+  if (threadIdx.x < SL_K) {
+    double2 s = red[0][threadIdx.x];
+    for (int w = 1; w < SC_W; w++) {
       s.x += red[w][threadIdx.x].x;
       s.y += red[w][threadIdx.x].y;
     }
@@ -664,6 +918,7 @@ struct Job {
   Slab *slab = nullptr;
   int col = -1, slot = -1;
   int realc = 1;
+  bool cls = false;  // its slab has the class layout
   std::vector<double> alpha, beta;
   int step = 0, nprev = 0, tick_steps = 0;
   double prev[16];
@@ -755,6 +1010,9 @@ struct Slab {
   DTerm *dterms = nullptr;  // [SL_K][nd]
   double *hist = nullptr;   // [SL_K][2][max_iter + 2]
   std::vector<double2> coef_host;
+  ClsArgs cls{};             // class layout (plan with device addresses)
+  ClsArgs *d_cls = nullptr;  // its copy on the device; null: k_sl_hv serves the slab
+  uint64_t hv_chunks = 0;    // workgroups of its H·v
   uint64_t nnz = 0;  // off-diagonal elements of one column's H (hphi_term_nnz)
   Job *col[SL_K] = {};
   int used() const {
@@ -764,11 +1022,22 @@ struct Slab {
   }
 };
 
-size_t slab_footprint(const hphi_engine &h, int max_iter) {
+// arena bytes of a slab; cls: with the class layout
+size_t slab_footprint(const hphi_engine &h, int max_iter, bool cls) {
   const size_t nt = std::max<size_t>(h.h_terms_dev.size(), 1), nd = std::max<size_t>(h.h_dterms.size(), 1);
   return al256(8 * h.dim) + al256(4 * h.size21) + al256(16 * ((h.size21 + 7) / 8)) + al256(8 * h.size22) + al256(8 * (h.sdim + 1)) +
          al256(sizeof(GTerm) * nt) + al256(16 * SL_K * nt) + al256(8 * SL_K * h.dim) + 2 * al256(16 * SL_K * h.dim) +
-         al256(sizeof(DTerm) * SL_K * nd) + al256(8 * SL_K * 2 * (size_t)(max_iter + 2));
+         al256(sizeof(DTerm) * SL_K * nd) + al256(8 * SL_K * 2 * (size_t)(max_iter + 2)) +
+         (cls ? al256(sizeof(ClsArgs)) + al256(hphi_cls_bytes_bound(&h)) : 0);
+}
+
+// The class layout, if the sector and its terms fit it, its tables leave the
+// slab within the arena and list_2_1 (32 KB), row offsets (16 KB) and couplings
+// (64 KB) fit LDS; the answer depends on the structure and the arena alone, so
+// every slab of a structure runs the same kernel.
+bool slab_cls(const hphi_engine &h, int max_iter, size_t arena) {
+  return h.size21 <= 16384 && h.h_terms_dev.size() + 5 * 7 <= 1024 && hphi_cls_bytes_bound(&h) &&
+         slab_footprint(h, max_iter, true) <= arena;
 }
 
 double mono_now() {
@@ -833,8 +1102,8 @@ extern "C" int hphi_server_create(const hphi_server_params *p, hphi_server **out
       hipMalloc(&s->d_out, sizeof(double) * 2 * mj * SL_SMAX) != hipSuccess ||
       hipMalloc(&s->d_slabs, sizeof(SlabDev) * mj * SL_SMAX) != hipSuccess ||
       hipMalloc(&s->d_cols, sizeof(ColDev) * mj * SL_SMAX) != hipSuccess ||
-      hipMalloc(&s->d_prefix, sizeof(uint64_t) * (mj + 1) * SL_SMAX) != hipSuccess ||
-      hipMalloc(&s->d_part, sizeof(double2) * SL_K * s->max_tiles) != hipSuccess ||
+      hipMalloc(&s->d_prefix, sizeof(uint64_t) * 2 * (mj + 1) * SL_SMAX) != hipSuccess ||
+      hipMalloc(&s->d_part, sizeof(double2) * SL_K * (s->max_tiles + 8 * (size_t)mj)) != hipSuccess ||
       hipHostMalloc(&s->h_out, sizeof(double) * 2 * mj * SL_SMAX, hipHostMallocDefault) != hipSuccess ||
       hipMalloc(&s->d_ev, sizeof(double) * 17 * mj) != hipSuccess ||
       hipHostMalloc(&s->h_ev, sizeof(double) * 17 * mj, hipHostMallocDefault) != hipSuccess)
@@ -896,7 +1165,8 @@ extern "C" int hphi_server_submit(hphi_server *s, const hphi_model_desc *d, uint
   j->shash = structure_hash(j->h);
   for (const GTerm &t : j->h.h_terms_dev)
     if (t.cim != 0.0) j->realc = 0;
-  const size_t fp = slab_footprint(j->h, s->p.max_iter);
+  j->cls = slab_cls(j->h, s->p.max_iter, s->arena.size);
+  const size_t fp = slab_footprint(j->h, s->p.max_iter, j->cls);
   if (fp > s->arena.size) {
     delete j;
     return hphi_set_error("job footprint %zu exceeds the HBM budget", fp);
@@ -936,7 +1206,10 @@ static int slab_create(hphi_server *s, const Job *j, size_t off, size_t bytes, S
   const hphi_engine &h = j->h;
   const size_t nt = std::max<size_t>(h.h_terms_dev.size(), 1), nd = std::max<size_t>(h.h_dterms.size(), 1);
   const size_t tb = sizeof(GTerm) * h.h_terms_dev.size();
-  if (s->stage_used + al256(tb) > s->stage_size) return 1;
+  ClsArgs plan{};
+  std::vector<char> up;
+  const bool cls = j->cls && hphi_cls_plan(&h, plan, up);
+  if (s->stage_used + al256(tb) + al256(up.size()) + al256(sizeof plan) > s->stage_size) return 1;
   Slab *b = new Slab();
   b->proto = h;
   b->nnz = hphi_term_nnz(&h);
@@ -955,7 +1228,7 @@ static int slab_create(hphi_server *s, const Job *j, size_t off, size_t bytes, S
   b->R = (double2 *)p, p += al256(16 * SL_K * h.dim);
   b->Q = (double2 *)p, p += al256(16 * SL_K * h.dim);
   b->dterms = (DTerm *)p, p += al256(sizeof(DTerm) * SL_K * nd);
-  b->hist = (double *)p;
+  b->hist = (double *)p, p += al256(8 * SL_K * 2 * (size_t)(s->p.max_iter + 2));
   b->coef_host.assign(SL_K * nt, make_double2(0.0, 0.0));
   int rc = 0;
   if (tb) {
@@ -970,6 +1243,19 @@ static int slab_create(hphi_server *s, const Job *j, size_t off, size_t bytes, S
     hipLaunchKernelGGL(k_pack21, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s->stream, b->l21, h.size21, n,
                        b->l21p);
     if (hipGetLastError() != hipSuccess) rc = hphi_set_error("slab table packing failed");
+  }
+  b->hv_chunks = (h.dim + (uint64_t)SL_TPW * SV_TPB - 1) / ((uint64_t)SL_TPW * SV_TPB);
+  if (!rc && cls) {
+    b->cls = plan;
+    hphi_cls_units(b->cls, SC_B, SC_RPT);
+    // SC_UPW units per wave, fewer while that leaves CUs idle; no more workgroups than k_sl_hv has
+    const uint64_t w = (b->cls.units + SC_W - 1) / SC_W;
+    b->hv_chunks = std::min<uint64_t>(b->hv_chunks, std::max<uint64_t>(w / SC_UPW, std::min<uint64_t>(w, 256)));
+    b->d_cls = (ClsArgs *)p, p += al256(sizeof(ClsArgs));
+    if (hphi_cls_upload(&h, b->cls, p, stage(s, up.data(), up.size()), b->l22, s->stream)) rc = -1;
+    if (!rc && hipMemcpyAsync(b->d_cls, stage(s, &b->cls, sizeof plan), sizeof plan, hipMemcpyHostToDevice,
+                              s->stream) != hipSuccess)
+      rc = hphi_set_error("slab class layout upload failed");
   }
   if (rc) {
     delete b;
@@ -1093,7 +1379,7 @@ static int admit(hphi_server *s, double now) {
     }
     bool fresh = false;
     if (!b) {
-      const size_t bytes = slab_footprint(j->h, s->p.max_iter);
+      const size_t bytes = slab_footprint(j->h, s->p.max_iter, j->cls);
       size_t off;
       if (!s->arena.alloc(bytes, &off)) break;
       const int rc = slab_create(s, j, off, bytes, &b);
@@ -1202,7 +1488,8 @@ extern "C" int hphi_server_tick(hphi_server *s, int *n_active, int *n_waiting) {
     for (int i = 0; i < n; i++) s_chk[nst[i] - 1]++;
     std::vector<SlabDev> sd;
     std::vector<ColDev> cd;
-    std::vector<uint64_t> prefix;
+    std::vector<uint64_t> prefix;  // per step: tiles of pass 1 by slab, then workgroups of pass 2 by slab
+    std::vector<int> s_nk(S), s_pv0(S);  // slabs with a class layout (the first ones); start of pass 2's prefix
     std::vector<int> s_ns(S), s_nc(S), s_sd0(S), s_cd0(S), s_pf0(S);
     // algorithmic bytes of each step's slab H·v: per slab 8 dim (list_1), per
     // running column 56 dim (own row, diagonal, Q read and write) + 16 per
@@ -1210,14 +1497,21 @@ extern "C" int hphi_server_tick(hphi_server *s, int *n_active, int *n_waiting) {
     std::vector<double> s_bytes(S, 0.0);
     std::map<const Slab *, int> index;
     const size_t hl = (size_t)s->p.max_iter + 2;
-    uint64_t tiles = 0, max21 = 0;
+    uint64_t tiles = 0, max21 = 0, maxk21 = 0, maxla = 0, maxco = 0;
+    std::vector<Slab *> order(s->slabs);
+    std::stable_sort(order.begin(), order.end(), [](const Slab *a, const Slab *b) {  // the largest slabs start first
+      return (a->d_cls != nullptr) > (b->d_cls != nullptr) ||
+             ((a->d_cls != nullptr) == (b->d_cls != nullptr) && a->nnz > b->nnz);
+    });
+    std::vector<uint64_t> pv;
     for (int st = 0; st < S; st++) {
       s_sd0[st] = (int)sd.size();
       s_cd0[st] = (int)cd.size();
       s_pf0[st] = (int)prefix.size();
       prefix.push_back(0);
+      pv.assign(1, 0);
       index.clear();
-      for (Slab *b : s->slabs) {
+      for (Slab *b : order) {
         const hphi_engine &h = b->proto;
         SlabDev d{};
         for (int c = 0; c < SL_K; c++) {
@@ -1244,12 +1538,22 @@ extern "C" int hphi_server_tick(hphi_server *s, int *n_active, int *n_waiting) {
         d.n_high = h.n_high;
         d.n_mixed = h.n_mixed;
         d.nlow = h.nlow;
+        d.cls = b->d_cls;
+        d.sgn = h.model == HPHI_MODEL_HUBBARD;
         index[b] = (int)sd.size() - s_sd0[st];
         s_bytes[st] += 8.0 * (double)h.dim +
                        (double)__builtin_popcount(d.mask) * (56.0 * (double)h.dim + 16.0 * (double)b->nnz);
         sd.push_back(d);
         prefix.push_back(prefix.back() + (h.dim + (uint64_t)SL_TPW * SV_TPB - 1) / ((uint64_t)SL_TPW * SV_TPB));
-        max21 = std::max<uint64_t>(max21, h.size21);
+        pv.push_back(pv.back() + (b->hv_chunks + 7) / 8 * 8);
+        if (b->d_cls) {
+          s_nk[st]++;
+          maxk21 = std::max<uint64_t>(maxk21, h.size21);
+          maxla = std::max<uint64_t>(maxla, (uint64_t)b->cls.nlo * SC_W * SC_RPT);
+          maxco = std::max<uint64_t>(maxco, (uint64_t)(b->cls.n_low + b->cls.nt) * SL_K * 16);
+        } else {
+          max21 = std::max<uint64_t>(max21, h.size21);
+        }
         std::swap(b->R, b->Q);  // roles after this step
       }
       for (int i = 0; i < n; i++) {
@@ -1261,11 +1565,17 @@ extern "C" int hphi_server_tick(hphi_server *s, int *n_active, int *n_waiting) {
       s_ns[st] = (int)sd.size() - s_sd0[st];
       s_nc[st] = (int)cd.size() - s_cd0[st];
       tiles = std::max<uint64_t>(tiles, prefix.back());
+      s_pv0[st] = (int)prefix.size();
+      prefix.insert(prefix.end(), pv.begin(), pv.end());
     }
     if (tiles > s->max_tiles) return hphi_set_error("too many tiles in flight");
     const size_t lds = 16 * (size_t)((max21 + 7) / 8);  // list_2_1 as uint16 (rank + 2 < 2^16 for <= 16 low bits)
     if (lds > 65536)
       (void)hipFuncSetAttribute((const void *)k_sl_hv, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    const uint32_t n21 = (uint32_t)((maxk21 + 7) / 8), nla = (uint32_t)((maxla + 3) / 4 * 4);
+    const size_t ldsk = 16 * (size_t)n21 + 4 * (size_t)nla + maxco;
+    if (ldsk > 65536)
+      (void)hipFuncSetAttribute((const void *)k_sl_cls, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldsk);
     HIPCHK(hipMemcpyAsync(s->d_slabs, sd.data(), sizeof(SlabDev) * sd.size(), hipMemcpyHostToDevice, s->stream));
     HIPCHK(hipMemcpyAsync(s->d_cols, cd.data(), sizeof(ColDev) * cd.size(), hipMemcpyHostToDevice, s->stream));
     HIPCHK(hipMemcpyAsync(s->d_prefix, prefix.data(), sizeof(uint64_t) * prefix.size(), hipMemcpyHostToDevice,
@@ -1283,10 +1593,16 @@ extern "C" int hphi_server_tick(hphi_server *s, int *n_active, int *n_waiting) {
       hipLaunchKernelGGL(k_sl_norm, dim3(nc), dim3(256), 0, s->stream, dcl, dpf, (const double *)s->d_part,
                          s->d_js);
       HIPCHK(hipEventRecord(s->ev_hv[2 * st], s->stream));
-      hipLaunchKernelGGL(k_sl_hv, dim3(T), dim3(SV_TPB), lds, s->stream, dsl, dpf, ns, (const double *)s->d_js,
-                         (double2 *)s->d_part);
+      const uint64_t *dpv = s->d_prefix + s_pv0[st], *pvh = prefix.data() + s_pv0[st];
+      const int nk = s_nk[st];
+      if (nk)
+        hipLaunchKernelGGL(k_sl_cls, dim3((unsigned)pvh[nk]), dim3(SV_TPB), ldsk, s->stream, dsl, dpv,
+                           nk, (const double *)s->d_js, (double2 *)s->d_part, n21, nla);
+      if (ns > nk)
+        hipLaunchKernelGGL(k_sl_hv, dim3((unsigned)(pvh[ns] - pvh[nk])), dim3(SV_TPB), lds, s->stream,
+                           dsl + nk, dpv + nk, ns - nk, (const double *)s->d_js, (double2 *)s->d_part);
       HIPCHK(hipEventRecord(s->ev_hv[2 * st + 1], s->stream));
-      hipLaunchKernelGGL(k_sl_alpha, dim3(nc), dim3(256), 0, s->stream, dcl, dpf, (const double2 *)s->d_part,
+      hipLaunchKernelGGL(k_sl_alpha, dim3(nc), dim3(256), 0, s->stream, dcl, dpv, (const double2 *)s->d_part,
                          s->d_js, out);
       if (s_chk[st]) hipLaunchKernelGGL(k_sl_check, dim3(nc), dim3(CK_TPB), 0, s->stream, dcl, s->p.n_eigen, s->d_ev);
       HIPCHK(hipGetLastError());

@@ -1,4 +1,5 @@
-"""The service's device eigenvalue check: every number of wanted values and check
+"""The service's slab H·v, by classes and by list_2_1 and list_2_2 alone, and its
+device eigenvalue check: every number of wanted values and check
 interval against dense diagonalisation, from one-state sectors on.  Tolerance:
 the service's own, 1e-10."""
 
@@ -6,6 +7,7 @@ import numpy as np
 import pytest
 
 from hphi_amd import lattice as L
+from tests.golden.cases import two_body_cases
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-10
@@ -52,3 +54,30 @@ def test_device_check_finds_the_lowest_distinct_values(A, want, every):
         assert np.max(np.abs(got[:n] - ref[:n])) <= TOL, (s.name, got, ref)
         for g in got:
             assert np.min(np.abs(distinct(A, s) - g)) <= TOL, (s.name, g)
+
+
+# class layout: uneven splits, classes of a few ranks, odd particle numbers, real and complex couplings
+# with value predicates; without it (list_2_1 past 16,384 entries): 30 sites
+SLABS = [(n, s) for n, s in two_body_cases().items() if s.model in (L.SPIN, L.HUBBARD) and s.dim <= 1000]
+SLABS += [("chain11_3", L.heisenberg_chain(11, 1.0, 0.4, two_sz=-5)), ("ladder10", L.j1j2_ladder(5, 1.0, 0.6)),
+          ("square12_2", L.j1j2_square(4, 3, 1.0, 0.3, two_sz=-8)), ("hub5_3", L.hubbard_chain(5, 1.0, 2.0, ncond=3)),
+          ("hub6", L.hubbard_chain(6, 1.0, 4.0)), ("chain30_1", L.heisenberg_chain(30, 1.0, 0.2, two_sz=-28)),
+          ("chain30_2", L.heisenberg_chain(30, 1.0, 0.2, two_sz=-26))]
+
+
+@pytest.mark.parametrize("name,spec", SLABS, ids=[n for n, _ in SLABS])
+def test_slab_hv_finds_the_lowest_value(A, name, spec):
+    """Five jobs of one structure (a full slab and one more) with the sector's ground state."""
+    print(f"[gpu] slab {name}", flush=True)
+    srv = A.Server(hbm_budget=1 << 28, max_jobs=8, n_eigen=1, eps=1e-12, check_every=2)
+    ids = [srv.submit(spec, 31 + i, 0.0) for i in range(5)]
+    res = {}
+    for _ in range(5000):
+        a, w = srv.tick()
+        res.update({r.id: r for r in srv.results()})
+        if a == 0 and w == 0:
+            break
+    srv.close()
+    ref = distinct(A, spec)[0]
+    for i in ids:
+        assert abs(res[i].eigenvalues[0] - ref) <= TOL * max(abs(ref), 1.0), (name, res[i].eigenvalues[0], ref)
