@@ -30,21 +30,46 @@ static double wall(void) {
   return ts.tv_sec + 1e-9 * ts.tv_nsec;
 }
 
-/* number of eigenvalues of the symmetric tridiagonal (a[0..n), b[0..n-1)) below x */
-static int sturm_count(const double *a, const double *b, int n, double x) {
-  int c = 0;
-  double q = a[0] - x;
+/* Numbers of eigenvalues of the symmetric tridiagonal (a[0..n), b[0..n-1)) below
+ * each of TL_N points x.  A Sturm count is a chain of n dependent divisions, some
+ * 20 cycles each; TL_N chains side by side in vectors run at the divider's rate. */
+typedef double tl_vd __attribute__((vector_size(32)));
+typedef long long tl_vl __attribute__((vector_size(32)));
+#define TL_V 4
+#define TL_N (4 * TL_V)
+#if defined(__x86_64__) && defined(__GNUC__)
+__attribute__((target_clones("avx2", "default")))
+#endif
+static void sturm_counts(const double *a, const double *b, int n, const double *x, int *count) {
   const double tiny = 1e-300;
-  if (q < 0) c++;
-  for (int i = 1; i < n; i++) {
-    if (fabs(q) < tiny) q = -tiny;
-    q = (a[i] - x) - b[i - 1] * b[i - 1] / q;
-    if (q < 0) c++;
+  const tl_vd small = {tiny, tiny, tiny, tiny};
+  tl_vd X[TL_V], q[TL_V];
+  tl_vl c[TL_V];
+#pragma GCC unroll 4
+  for (int j = 0; j < TL_V; j++) {
+    memcpy(&X[j], x + 4 * j, sizeof X[j]);
+    q[j] = a[0] - X[j];
+    c[j] = (tl_vl){0, 0, 0, 0};
   }
-  return c;
+  for (int i = 1; i < n; i++) {
+    const double ai = a[i], bb = b[i - 1] * b[i - 1];
+#pragma GCC unroll 4
+    for (int j = 0; j < TL_V; j++) {
+      /* a vanishing pivot becomes -tiny, and counts as that: x may be an
+       * eigenvalue of a leading block exactly */
+      const tl_vl z = (q[j] < small) & (q[j] > -small);
+      q[j] = (tl_vd)(((tl_vl)q[j] & ~z) | ((tl_vl)-small & z));
+      c[j] += q[j] < 0;
+      q[j] = (ai - X[j]) - bb / q[j];
+    }
+  }
+  for (int j = 0; j < TL_V; j++) c[j] += q[j] < 0;
+  for (int j = 0; j < TL_N; j++) count[j] = -(int)c[j / 4][j % 4];
 }
 
-/* k lowest eigenvalues (ascending) of the tridiagonal by bisection */
+/* k lowest eigenvalues (ascending) of the tridiagonal, by Sturm counts down to
+ * adjacent numbers: up to TL_N eigenvalues at a time, the points of a round shared
+ * among them (one each: its middle; more: equal sections). */
 int hphi_tridiag_lowest(const double *a, const double *b, int n, int k, double *ev) {
   if (n <= 0 || k <= 0) return 0;
   if (k > n) k = n;
@@ -57,16 +82,35 @@ int hphi_tridiag_lowest(const double *a, const double *b, int n, int k, double *
   double span = hi - lo;
   lo -= 1e-12 * span + 1e-300;
   hi += 1e-12 * span + 1e-300;
-  for (int m = 0; m < k; m++) {
-    double l = (m > 0) ? ev[m - 1] - 1e-15 * (fabs(ev[m - 1]) + span) : lo, h = hi;
-    if (l < lo) l = lo;
+  for (int m0 = 0; m0 < k; m0 += TL_N) {
+    const int g = k - m0 < TL_N ? k - m0 : TL_N, per = TL_N / g;
+    double l[TL_N], h[TL_N], x[TL_N];
+    int count[TL_N];
+    for (int j = 0; j < g; j++) l[j] = lo, h[j] = hi;
+    for (int j = 0; j < TL_N; j++) x[j] = hi;
     for (int it = 0; it < 200; it++) {
-      double mid = 0.5 * (l + h);
-      if (mid <= l || mid >= h) break;
-      if (sturm_count(a, b, n, mid) > m) h = mid;
-      else l = mid;
+      int open = 0;
+      for (int j = 0; j < g; j++) {
+        const double mid = 0.5 * (l[j] + h[j]), d = (h[j] - l[j]) / (per + 1);
+        open |= mid > l[j] && mid < h[j];
+        for (int p = 0; p < per; p++) x[j * per + p] = p == (per - 1) / 2 ? mid : l[j] + d * (p + 1);
+      }
+      if (!open) break;
+      sturm_counts(a, b, n, x, count);
+      for (int j = 0; j < g; j++) {
+        const double mid = 0.5 * (l[j] + h[j]);
+        if (!(mid > l[j] && mid < h[j])) continue;
+        for (int p = 0; p < per; p++) { /* the last point not above eigenvalue m0 + j, and the first above */
+          const double y = x[j * per + p];
+          if (count[j * per + p] > m0 + j) {
+            if (y < h[j]) h[j] = y;
+            break;
+          }
+          if (y > l[j]) l[j] = y;
+        }
+      }
     }
-    ev[m] = 0.5 * (l + h);
+    for (int j = 0; j < g; j++) ev[m0 + j] = 0.5 * (l[j] + h[j]);
   }
   return k;
 }

@@ -718,13 +718,12 @@ __global__ __launch_bounds__(256) void k_sl_alpha(const ColDev *cols, const uint
 __device__ __forceinline__ int ck_sturm(const double *a, const double *b, int n, double x) {
   int c = 0;
   double q = a[0] - x;
-  if (q < 0) c++;
   for (int i = 1; i < n; i++) {
-    if (fabs(q) < 1e-300) q = -1e-300;
-    q = (a[i] - x) - b[i - 1] * b[i - 1] / q;
+    if (fabs(q) < 1e-300) q = -1e-300;  // a vanishing pivot, and counted as such
     if (q < 0) c++;
+    q = (a[i] - x) - b[i - 1] * b[i - 1] / q;
   }
-  return c;
+  return c + (q < 0);
 }
 
 __global__ __launch_bounds__(CK_TPB) void k_sl_check(const ColDev *cols, int want, double *out) {
