@@ -13,6 +13,7 @@
 #define HV_TERM_PAD 16    // term groups are padded with never-active terms to a multiple of
                           // this, so every batch size in use (8, 16) reads whole groups
 #define HV_NOALLOC_PARTIALS (1 << 18)  // k x workgroups of an allocation-free H·v (4 MiB of partial sums)
+#define HV_HOST_PARTIALS 256  // partial sums of prdct a call adds up on the host
 #define HV_MAX_GRID 65536 // upper bound of H·v workgroups (sizes the partial-sum buffer)
 
 // predicate kinds of a gather term, evaluated on the TARGET state x
@@ -207,6 +208,7 @@ struct hphi_engine {
   int n_low = 0, n_high = 0, n_mixed = 0;
   int r_low = 0, r_high = 0, r_mixed = 0;  // compiled terms per group, before padding
   void *d_partial = nullptr, *d_prdct = nullptr, *h_prdct = nullptr, *d_coef = nullptr;
+  void *hd_prdct = nullptr;  // h_prdct (pinned) as the device addresses it
   double *d_stage0 = nullptr, *d_stage1 = nullptr;
   // host-pointer calls: per worker thread a stream and two pinned bounce
   // buffers of HOST_CHUNK bytes, with the events that free them
@@ -255,7 +257,6 @@ int hphi_build_diag(hphi_engine *e);
 int hphi_hv_launch(hphi_engine *e, int k, double *v0, const double *v1);
 int hphi_hv_launch_ex(hphi_engine *e, int k, double *v0, const double *v1, int overwrite);
 int hphi_hv_launch_gather(hphi_engine *e, int k, double *v0, const double *v1);
-int hphi_fetch_prdct(hphi_engine *e, int k, double *prdct);
 int hphi_hv_grid(const hphi_engine *e, int k);
 int hphi_canon_config(hphi_engine *e);
 void hphi_crank_tables(uint16_t *t);

@@ -219,10 +219,8 @@ static int vo_grid(uint64_t n) {
 // scratch: e->d_partial holds HV_MAX_GRID*16 double2 = enough for VO_GRID*32 doubles
 static int finish_sum(hphi_engine *e, int g, int m, double *host_out) {
   double *part = (double *)e->d_partial;
-  double *out = (double *)e->d_prdct;
-  hipLaunchKernelGGL(k_sum_partials, dim3(m), dim3(VO_TPB), 0, e->stream, part, g, m, out);
+  hipLaunchKernelGGL(k_sum_partials, dim3(m), dim3(VO_TPB), 0, e->stream, part, g, m, (double *)e->hd_prdct);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(e->h_prdct, out, sizeof(double) * m, hipMemcpyDeviceToHost, e->stream));
   HIPCHK(hipStreamSynchronize(e->stream));
   memcpy(host_out, e->h_prdct, sizeof(double) * m);
   return 0;
