@@ -455,9 +455,9 @@ static int grid_for(uint64_t n, int tpb) { return (int)((n + tpb - 1) / tpb); }
 int hphi_engine_alloc_scratch(hphi_engine *e) {
   if (e->d_partial) return 0;
   HIPCHK(hipMalloc(&e->d_partial, sizeof(double2) * (size_t)HV_MAX_GRID * 16));
-  HIPCHK(hipMalloc(&e->d_prdct, sizeof(double2) * 16));
+  HIPCHK(hipMalloc(&e->d_prdct, sizeof(double2) * 32));  // prdct, then the state of a Lanczos run
   HIPCHK(hipMalloc(&e->d_coef, sizeof(double2) * 64));
-  HIPCHK(hipHostMalloc(&e->h_prdct, sizeof(double2) * HV_HOST_PARTIALS, hipHostMallocDefault));
+  HIPCHK(hipHostMalloc(&e->h_prdct, sizeof(double2) * HV_HOST_PARTIALS + 32 * LZ_RING, hipHostMallocDefault));
   HIPCHK(hipHostGetDevicePointer(&e->hd_prdct, e->h_prdct, 0));
   e->bytes += sizeof(double2) * ((size_t)HV_MAX_GRID * 16 + 16);
   return 0;
@@ -994,6 +994,8 @@ extern "C" void hphi_engine_destroy(hphi_engine *e) {
     }
     if (e->h_stream[t]) (void)hipStreamDestroy(e->h_stream[t]);
   }
+  for (int i = 0; i < 2; i++)
+    if (e->lz_ev[i]) (void)hipEventDestroy(e->lz_ev[i]);
   if (e->h_prdct) (void)hipHostFree(e->h_prdct);
   if (e->stream) (void)hipStreamDestroy(e->stream);
   delete e;
@@ -1306,6 +1308,12 @@ int hphi_hv_launch_gather(hphi_engine *e, int k, double *v0, const double *v1) {
   HvArgs A = hphi_hv_args(e, k, v0, v1);
   A.overwrite = 1;
   return hv_launch_args(e, k, A, (double2 *)e->d_prdct, 1);
+}
+
+int hphi_hv_launch_cdev(hphi_engine *e, double *v0, const double *v1, const double *cdev) {
+  HvArgs A = hphi_hv_args(e, 1, v0, v1);
+  A.cdev = cdev;
+  return hv_launch_args(e, 1, A, (double2 *)e->d_prdct);
 }
 
 int hphi_hv_launch_ex(hphi_engine *e, int k, double *v0, const double *v1, int overwrite) {

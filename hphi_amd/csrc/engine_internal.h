@@ -13,6 +13,7 @@
 #define HV_TERM_PAD 16    // term groups are padded with never-active terms to a multiple of
                           // this, so every batch size in use (8, 16) reads whole groups
 #define HV_NOALLOC_PARTIALS (1 << 18)  // k x workgroups of an allocation-free H·v (4 MiB of partial sums)
+#define LZ_RING 64             // Lanczos steps in flight at most, 4 doubles each after the host partials
 #define HV_HOST_PARTIALS 256  // partial sums of prdct a call adds up on the host
 #define HV_MAX_GRID 65536 // upper bound of H·v workgroups (sizes the partial-sum buffer)
 
@@ -102,6 +103,7 @@ struct HvArgs {
   uint64_t size21;
   int overwrite;  // 1: v0 = c1 H v1 (v0 not read); 0: v0 = c0 v0 + c1 H v1 (reference: c0 = c1 = 1)
   double c0, c1;  // scale factors of the output (prdct stays <v1|H v1>)
+  const double *cdev;  // (c0, c1) on the device instead, where the caller has them there (k = 1)
   // canonical Spin: list_2_1[ia] = rank of ia among the values of its popcount
   // + 2, from two byte tables (hphi_crank_tables)
   const uint16_t *crank;
@@ -110,6 +112,13 @@ struct HvArgs {
   double2 *v1t;
   const ulonglong2 *tofs;
 };
+
+// scale factors of the output
+__device__ __forceinline__ double2 hv_scale(double c0, double c1, const double *cdev) {
+  if (!cdev) return make_double2(c0, c1);
+  const double __attribute__((address_space(4))) *c = (const double __attribute__((address_space(4))) *)cdev;
+  return make_double2(c[0], c[1]);
+}
 
 // byte tables of the combinatorial rank (spin, nlow <= 16): rank(ia) =
 // t[ia & 255] + t[256 + 9 * ((ia >> 8) & 255) + popcount(ia & 255)]
@@ -208,6 +217,7 @@ struct hphi_engine {
   int n_low = 0, n_high = 0, n_mixed = 0;
   int r_low = 0, r_high = 0, r_mixed = 0;  // compiled terms per group, before padding
   void *d_partial = nullptr, *d_prdct = nullptr, *h_prdct = nullptr, *d_coef = nullptr;
+  hipEvent_t lz_ev[2] = {};
   void *hd_prdct = nullptr;  // h_prdct (pinned) as the device addresses it
   double *d_stage0 = nullptr, *d_stage1 = nullptr;
   // host-pointer calls: per worker thread a stream and two pinned bounce
@@ -256,6 +266,8 @@ int hphi_build_tables(hphi_engine *e);
 int hphi_build_diag(hphi_engine *e);
 int hphi_hv_launch(hphi_engine *e, int k, double *v0, const double *v1);
 int hphi_hv_launch_ex(hphi_engine *e, int k, double *v0, const double *v1, int overwrite);
+// v0 <- c0 v0 + c1 H v1 with (c0, c1) read from cdev; prdct in d_prdct
+int hphi_hv_launch_cdev(hphi_engine *e, double *v0, const double *v1, const double *cdev);
 int hphi_hv_launch_gather(hphi_engine *e, int k, double *v0, const double *v1);
 int hphi_hv_grid(const hphi_engine *e, int k);
 int hphi_canon_config(hphi_engine *e);

@@ -60,6 +60,7 @@ template <int TPB, bool REALC, int RK, int UNR>
 __global__ __launch_bounds__(TPB) void k_hv_canon(const HvArgs A) {
   extern __shared__ uint16_t s21[];
   const uint32_t tid = threadIdx.x;
+  const double2 cs = hv_scale(A.c0, A.c1, A.cdev);
   if (RK == 1) {
     for (uint32_t i = tid; i < (uint32_t)A.size21; i += TPB) s21[i] = (uint16_t)A.l21[i];
     __syncthreads();
@@ -238,11 +239,11 @@ __global__ __launch_bounds__(TPB) void k_hv_canon(const HvArgs A) {
     }
 
     if (valid) {
-      double2 o = make_double2(A.c1 * ar, A.c1 * ai);
+      double2 o = make_double2(cs.y * ar, cs.y * ai);
       if (!A.overwrite) {
         const double2 p = v0[j];
-        o.x += A.c0 * p.x;
-        o.y += A.c0 * p.y;
+        o.x += cs.x * p.x;
+        o.y += cs.x * p.y;
       }
       v0[j] = o;
       pre += a.x * ar + a.y * ai;
@@ -322,6 +323,7 @@ __global__ __launch_bounds__(256) void k_hv_high(const HvArgs A, const HiPlan P,
                                                  const uint32_t *__restrict__ blkpos,
                                                  const double2 *__restrict__ v1t, double2 *__restrict__ partial) {
   const uint32_t tid = threadIdx.x;
+  const double2 cs = hv_scale(A.c0, A.c1, A.cdev);
   double2 *__restrict__ v0 = (double2 *)A.v0;
   const int nlow = A.nlow;
   const CTerm th = (CTerm)A.terms + A.n_low;
@@ -369,7 +371,7 @@ __global__ __launch_bounds__(256) void k_hv_high(const HvArgs A, const HiPlan P,
       const uint64_t j = A.l22[ib] - 1 + r;
       const double2 a = tile[(uint64_t)p * HI_RT];
       const double2 o = v0[j];
-      v0[j] = make_double2(o.x + A.c1 * ar, o.y + A.c1 * ai);
+      v0[j] = make_double2(o.x + cs.y * ar, o.y + cs.y * ai);
       pre += a.x * ar + a.y * ai;
       pim += a.x * ai - a.y * ar;
     }

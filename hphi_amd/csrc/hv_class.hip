@@ -191,6 +191,7 @@ __global__ __launch_bounds__(CL_TPB) void k_hv_cls(const HvArgs A, const ClsArgs
   const uint32_t xcd = blockIdx.x & 7u, slot = (blockIdx.x >> 3) * (CL_TPB / 64) + wave;
   const uint32_t nslot = (gridDim.x >> 3) * (CL_TPB / 64);
   const uint32_t U1 = (uint32_t)((uint64_t)C.units * (xcd + 1) / 8);
+  const double2 cs = hv_scale(A.c0, A.c1, A.cdev);
   const uint32_t coff = (lane % LPS) * 16u;  // this lane's first column; the others at steps of LPS
   double pre[CPL], pim[CPL];
 #pragma unroll
@@ -285,11 +286,11 @@ __global__ __launch_bounds__(CL_TPB) void k_hv_cls(const HvArgs A, const ClsArgs
         for (int i = 0; i < CPL; i++) {
           const double2 a = cl_at(v1 + (uint64_t)base[b] * K, own_off + 16 * (K / CPL) * i);
           double2 *out = (double2 *)((char *)(v0 + (uint64_t)base[b] * K) + own_off + 16 * (K / CPL) * i);
-          double2 o = make_double2(A.c1 * acc[b][i].x, A.c1 * acc[b][i].y);
+          double2 o = make_double2(cs.y * acc[b][i].x, cs.y * acc[b][i].y);
           if (!A.overwrite) {
             const double2 p = *out;
-            o.x += A.c0 * p.x;
-            o.y += A.c0 * p.y;
+            o.x += cs.x * p.x;
+            o.y += cs.x * p.y;
           }
           *out = o;
           pre[i] += a.x * acc[b][i].x + a.y * acc[b][i].y;

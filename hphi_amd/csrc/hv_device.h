@@ -156,17 +156,18 @@ __device__ __forceinline__ void hv_tile(const HvArgs &A, uint64_t tile, double &
   const int vec = threadIdx.x & (K - 1);
   const int sl = threadIdx.x / K;
   double2 *__restrict__ v0 = (double2 *)A.v0;
+  const double2 cs = hv_scale(A.c0, A.c1, A.cdev);
   {
     const uint64_t j = tile * SPT + sl;
     if (j >= A.dim) return;
     double2 a;
     double ar, ai;
     hv_row<K, CANON>(A, j, vec, a, ar, ai);
-    double2 o = make_double2(A.c1 * ar, A.c1 * ai);
+    double2 o = make_double2(cs.y * ar, cs.y * ai);
     if (!A.overwrite) {
       const double2 p = v0[j * K + vec];
-      o.x += A.c0 * p.x;
-      o.y += A.c0 * p.y;
+      o.x += cs.x * p.x;
+      o.y += cs.x * p.y;
     }
     v0[j * K + vec] = o;
     // conj(a) * acc

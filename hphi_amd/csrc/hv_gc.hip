@@ -53,6 +53,7 @@ struct GcArgs {
   int nother, nrem;
   int K, overwrite;
   double c0, c1;
+  const double *cdev;
   uint64_t nouter;            // tiles per column group: 2^(n - s)
   uint32_t xe[GC_E];          // state bits of element e
   uint32_t sb[16];            // state bit of each local bit
@@ -245,7 +246,8 @@ __global__ __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     }
     __syncthreads();  // the next tile overwrites this one
     const bool add = !FIRST || !A.overwrite;
-    const double c0 = add ? (FIRST ? A.c0 : 1.0) : 0.0, c1 = A.c1;
+    const double2 cs = hv_scale(A.c0, A.c1, A.cdev);
+    const double c0 = add ? (FIRST ? cs.x : 1.0) : 0.0, c1 = cs.y;
 #pragma unroll
     for (int h = 0; h < GC_E; h += 4) {
       double2 old[4];
@@ -585,6 +587,7 @@ int hphi_hv_launch_gc(hphi_engine *e, const HvArgs &A, int k, int *grid) {
     G.overwrite = A.overwrite;
     G.c0 = A.c0;
     G.c1 = A.c1;
+    G.cdev = A.cdev;
     G.nrun = Q.nrun;
     G.nouter = (uint64_t)1 << Q.nob;
     std::copy(Q.sb, Q.sb + 16, G.sb);

@@ -47,9 +47,14 @@ __global__ __launch_bounds__(VO_TPB) void k_lanczos_beta(const double2 *v0, cons
 // Lanczos residual with the normalisation deferred: r <- r - f w (f = alpha_m
 // s_m, w the unnormalised Lanczos vector of step m), |r|^2 per block; with vg
 // also vg += cg w (the eigenvector sum).  One pass of 48 bytes per state.
+// With lz (the state of a run, see k_lz_step) f comes from it and prdct.
 __global__ __launch_bounds__(VO_TPB) void k_lz_resid(double2 *r, const double2 *w, double2 *vg, uint64_t n, double f,
-                                                     double cg, double *partial) {
+                                                     double cg, double *partial, double *lz, const double2 *prdct) {
   __shared__ double sh[VO_TPB / 64];
+  if (lz) {
+    f = lz[1] * lz[1] * prdct->x * lz[1];
+    if (blockIdx.x == 0 && threadIdx.x == 0) lz[2] = (double)wall_clock64();
+  }
   double s = 0.0;
   for (uint64_t i = (uint64_t)blockIdx.x * VO_TPB + threadIdx.x; i < n; i += (uint64_t)gridDim.x * VO_TPB) {
     const double2 a = r[i], b = w[i];
@@ -231,8 +236,85 @@ extern "C" int hphi_vec_lanczos_resid(hphi_engine *e, double *r, const double *w
   if (!e || !r || !w || !r2) return hphi_set_error("hphi_vec_lanczos_resid: NULL argument");
   int g = vo_grid(e->dim);
   hipLaunchKernelGGL(k_lz_resid, dim3(g), dim3(VO_TPB), 0, e->stream, (double2 *)r, (const double2 *)w,
-                     (double2 *)vg, e->dim, f, cg, (double *)e->d_partial);
+                     (double2 *)vg, e->dim, f, cg, (double *)e->d_partial, (double *)nullptr, (const double2 *)nullptr);
   return finish_sum(e, g, 1, r2);
+}
+
+// ---- Lanczos steps without the host: lz = (c0, c1 = s_m) of the next H·v and
+// the clock at the start of its residual pass
+__global__ void k_lz_set(double *lz, double c0, double c1) {
+  lz[0] = c0;
+  lz[1] = c1;
+}
+
+// Ends a step: |r|^2 (summed as k_sum_partials does), alpha_m and beta_m, the
+// scale factors of the next step, and (alpha, beta, ticks of the residual
+// pass) to the host's ring.  The same operations as the host's, so a run gives
+// the same bits either way.
+__global__ __launch_bounds__(VO_TPB) void k_lz_step(const double *partial, int nblk, const double2 *prdct, double *lz,
+                                                    double *ring) {
+  __shared__ double sh[VO_TPB];
+  double t = 0.0;
+  for (int b = threadIdx.x; b < nblk; b += VO_TPB) t += partial[b];
+  sh[threadIdx.x] = t;
+  __syncthreads();
+  for (int st = VO_TPB / 2; st > 0; st >>= 1) {
+    if (threadIdx.x < st) sh[threadIdx.x] += sh[threadIdx.x + st];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    const double s = lz[1], beta = sqrt(sh[0]);
+    ring[0] = s * s * prdct->x;
+    ring[1] = beta;
+    ring[2] = (double)wall_clock64() - lz[2];
+    lz[0] = -beta * s;
+    lz[1] = 1.0 / beta;
+  }
+}
+
+static double *lz_state_dev(hphi_engine *e) { return (double *)e->d_prdct + 32; }
+static double *lz_ring(void *base) { return (double *)base + 2 * HV_HOST_PARTIALS; }
+
+// the next step's H·v will be v0 <- c0 v0 + c1 H v1
+extern "C" int hphi_lz_set(hphi_engine *e, double c0, double c1) {
+  if (hphi_build_tables(e) || hphi_build_diag(e)) return -1;  // a restarted run comes here first
+  for (int i = 0; i < 2; i++)
+    if (!e->lz_ev[i]) HIPCHK(hipEventCreateWithFlags(&e->lz_ev[i], hipEventDisableTiming));
+  hipLaunchKernelGGL(k_lz_set, dim3(1), dim3(1), 0, e->stream, lz_state_dev(e), c0, c1);
+  HIPCHK(hipGetLastError());
+  return 0;
+}
+
+// Queues one step: r <- c0 r + c1 H w, then the residual pass r <- r - alpha s w;
+// slot: the ring entry of its results.  Waits for nothing.
+extern "C" int hphi_lz_step(hphi_engine *e, double *r, const double *w, int slot) {
+  double *lz = lz_state_dev(e);
+  const double2 *prdct = (const double2 *)e->d_prdct;
+  if (hphi_hv_launch_cdev(e, r, w, lz)) return -1;
+  const int g = vo_grid(e->dim);
+  hipLaunchKernelGGL(k_lz_resid, dim3(g), dim3(VO_TPB), 0, e->stream, (double2 *)r, (const double2 *)w,
+                     (double2 *)nullptr, e->dim, 0.0, 0.0, (double *)e->d_partial, lz, prdct);
+  hipLaunchKernelGGL(k_lz_step, dim3(1), dim3(VO_TPB), 0, e->stream, (const double *)e->d_partial, g, prdct, lz,
+                     lz_ring(e->hd_prdct) + 4 * (slot % LZ_RING));
+  HIPCHK(hipGetLastError());
+  return 0;
+}
+
+extern "C" int hphi_lz_mark(hphi_engine *e, int i) {
+  HIPCHK(hipEventRecord(e->lz_ev[i & 1], e->stream));
+  return 0;
+}
+extern "C" int hphi_lz_wait(hphi_engine *e, int i) {
+  HIPCHK(hipEventSynchronize(e->lz_ev[i & 1]));
+  return 0;
+}
+
+// a waited step's alpha, beta and the seconds of its residual pass
+extern "C" void hphi_lz_read(const hphi_engine *e, int slot, double *out) {
+  const double *p = lz_ring(e->h_prdct) + 4 * (slot % LZ_RING);
+  out[0] = p[0];
+  out[1] = p[1];
+  out[2] = 1e-8 * p[2];  // 100 MHz
 }
 
 extern "C" int hphi_vec_lanczos_beta(hphi_engine *e, const double *v0, const double *v1, double alpha,
