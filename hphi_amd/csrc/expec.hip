@@ -7,12 +7,14 @@
 //                               <v|c+_{i s1} c_{j s2} c+_{k s3} c_{l s4}|v>
 //
 // Every Green's function entry is compiled on the host into gather terms (the
-// same forms the Hamiltonian uses), each tagged with its output slot.  One
-// kernel pass evaluates EX_CW slots for all states: lane j holds target state
-// x = list_1[j] (or j), and for each active term adds
-// conj(v[j]) * c * sign * v[idx(x ^ flip)], i.e. <v|O|v> = sum_x conj(v_x) (O v)_x.
+// same forms the Hamiltonian uses).  A term without its factor is an item; terms
+// of several entries that agree share one (densities and exchanges of (i, k) and
+// (k, i)).  One workgroup evaluates EX_CW items: lane j holds target state x = list_1[j]
+// (or j) and adds sign * conj(v[j]) * v[idx(x ^ flip)] of each item that acts,
+// <v|O|v> = sum_x conj(v_x) (O v)_x; an entry is the sum of factor times item.
 // Reductions run in a fixed order (waves, then blocks), so results are
 // reproducible run to run.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <utility>
@@ -22,13 +24,13 @@
 
 #define EX_TPB 256
 #define EX_GRID 512
-#define EX_CW 8  // output slots per pass
+#define EX_CW 8  // items per workgroup
 
 namespace {
 
+template <typename W>
 struct CorrTerm {
-  uint64_t flip, tmask, tval, sgn;
-  double cre, cim;
+  W flip, tmask, tval, sgn;
 };
 
 __device__ __forceinline__ double wave_sum(double s) {
@@ -76,46 +78,93 @@ __global__ __launch_bounds__(EX_TPB) void k_moments(const double2 *v, const uint
   }
 }
 
-// block (bx, c): slots c*EX_CW .. c*EX_CW+EX_CW-1; the terms of slot s are
-// terms[toff[s] .. toff[s+1])
+__device__ __forceinline__ uint32_t ex_popc(uint32_t x) { return (uint32_t)__popc(x); }
+__device__ __forceinline__ uint32_t ex_popc(uint64_t x) { return (uint32_t)__popcll(x); }
+
+// One state against EX_CW items.  PROJ: items without flip and sign, |v_j|^2 alone.
+template <typename W, bool CANON, bool PROJ>
+__device__ __forceinline__ void corr_state(const double2 *v, const uint32_t *l21, const uint64_t *l22, uint64_t dim,
+                                           W irght, int nlow, const CorrTerm<W> (&T)[EX_CW], W x, double2 a,
+                                           double (&ar)[EX_CW], double (&ai)[EX_CW]) {
+  if (PROJ) {
+    const double w = a.x * a.x + a.y * a.y;
+#pragma unroll
+    for (int q = 0; q < EX_CW; q++)
+      if ((x & T[q].tmask) == T[q].tval) ar[q] += w;
+    return;
+  }
+  bool act[EX_CW];
+  uint64_t idx[EX_CW];
+#pragma unroll
+  for (int q = 0; q < EX_CW; q++) {
+    act[q] = (x & T[q].tmask) == T[q].tval;
+    idx[q] = (uint64_t)(x ^ T[q].flip);
+  }
+  if (CANON) {  // rank tables, 0 = not in the sector
+    uint32_t la[EX_CW];
+    uint64_t lb[EX_CW];
+#pragma unroll
+    for (int q = 0; q < EX_CW; q++) {
+      la[q] = 0;
+      lb[q] = 0;
+      if (act[q]) {
+        la[q] = l21[(W)idx[q] & irght];
+        lb[q] = l22[(W)idx[q] >> nlow];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < EX_CW; q++) {
+      idx[q] = la[q] + lb[q] - 3;
+      act[q] = la[q] != 0 && lb[q] != 0;
+    }
+  }
+  double2 u[EX_CW];
+#pragma unroll
+  for (int q = 0; q < EX_CW; q++) {
+    act[q] = act[q] && idx[q] < dim;
+    u[q] = make_double2(0.0, 0.0);
+    if (act[q]) u[q] = v[idx[q]];
+  }
+#pragma unroll
+  for (int q = 0; q < EX_CW; q++) {
+    if (!act[q]) continue;
+    const bool neg = ex_popc((W)(x & T[q].sgn)) & 1u;
+    const double ux = neg ? -u[q].x : u[q].x, uy = neg ? -u[q].y : u[q].y;
+    ar[q] += a.x * ux + a.y * uy;
+    ai[q] += a.x * uy - a.y * ux;
+  }
+}
+
+// block (bx, c): items c*EX_CW .. c*EX_CW+EX_CW-1, the first np chunks projectors.
+// Their masks stay in scalar registers over all the workgroup's states, eight
+// items' table lookups and gathers are in flight together, and the grid gives
+// each lane several states, so that the sums over the workgroup cost little.
+// (One slot after another per state, one state per lane, 64-bit: 1,330 us for the 2,360
+// entries of a 20-site chain; now 135, with 1,180 items left of them.)
+template <typename W, bool CANON>
 __global__ __launch_bounds__(EX_TPB) void k_corr(const double2 *v, const uint64_t *list1, const uint32_t *l21,
-                                                  const uint64_t *l22, uint64_t dim, uint64_t irght, int nlow,
-                                                  const CorrTerm *terms, const int *toff, int nslot,
-                                                  double2 *partial) {
-  const int s0 = blockIdx.y * EX_CW;
+                                                 const uint64_t *l22, uint64_t dim, W irght, int nlow,
+                                                 const CorrTerm<W> *terms, int np, double2 *partial) {
+  typedef const CorrTerm<W> __attribute__((address_space(4))) *CT;
+  CorrTerm<W> T[EX_CW];
+  const CT t = (CT)terms + (size_t)blockIdx.y * EX_CW;
+#pragma unroll
+  for (int q = 0; q < EX_CW; q++) {
+    T[q].flip = t[q].flip;
+    T[q].tmask = t[q].tmask;
+    T[q].tval = t[q].tval;
+    T[q].sgn = t[q].sgn;
+  }
   double ar[EX_CW], ai[EX_CW];
 #pragma unroll
   for (int q = 0; q < EX_CW; q++) ar[q] = ai[q] = 0.0;
-  for (uint64_t j = (uint64_t)blockIdx.x * EX_TPB + threadIdx.x; j < dim; j += (uint64_t)gridDim.x * EX_TPB) {
-    const uint64_t x = list1 ? list1[j] : j;
-    const double2 vj = v[j];
-#pragma unroll
-    for (int q = 0; q < EX_CW; q++) {
-      if (s0 + q >= nslot) break;
-      for (int t = toff[s0 + q]; t < toff[s0 + q + 1]; t++) {
-        const CorrTerm T = terms[t];
-        if ((x & T.tmask) != T.tval) continue;
-        const uint64_t y = x ^ T.flip;
-        uint64_t idx = y;
-        if (list1) {  // canonical: rank tables, 0 = not in the sector
-          const uint64_t la = l21[y & irght], lb = l22[y >> nlow];
-          if (la == 0 || lb == 0) continue;
-          idx = la + lb - 3;
-        }
-        if (idx >= dim) continue;
-        const double2 u = v[idx];
-        // c * sign * u
-        double cr = T.cre, ci = T.cim;
-        if (__popcll(x & T.sgn) & 1) {
-          cr = -cr;
-          ci = -ci;
-        }
-        const double wr = cr * u.x - ci * u.y, wi = cr * u.y + ci * u.x;
-        // conj(vj) * w
-        ar[q] += vj.x * wr + vj.y * wi;
-        ai[q] += vj.x * wi - vj.y * wr;
-      }
-    }
+  const uint64_t j0 = (uint64_t)blockIdx.x * EX_TPB + threadIdx.x, dj = (uint64_t)gridDim.x * EX_TPB;
+  if ((int)blockIdx.y < np) {
+    for (uint64_t j = j0; j < dim; j += dj)
+      corr_state<W, CANON, true>(v, l21, l22, dim, irght, nlow, T, CANON ? (W)list1[j] : (W)j, v[j], ar, ai);
+  } else {
+    for (uint64_t j = j0; j < dim; j += dj)
+      corr_state<W, CANON, false>(v, l21, l22, dim, irght, nlow, T, CANON ? (W)list1[j] : (W)j, v[j], ar, ai);
   }
   __shared__ double sh[EX_TPB / 64][EX_CW][2];
 #pragma unroll
@@ -137,18 +186,20 @@ __global__ __launch_bounds__(EX_TPB) void k_corr(const double2 *v, const uint64_
   }
 }
 
-// slot s: sum over the blocks of its chunk in block order
-__global__ void k_corr_final(const double2 *partial, int nblk, int nslot, double2 *out) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= nslot) return;
+// item s: sum over the blocks of its chunk, a wave per item (one thread took 128 us)
+__global__ __launch_bounds__(EX_TPB) void k_corr_final(const double2 *partial, int nblk, int n, double2 *out) {
+  const int s = blockIdx.x * (EX_TPB / 64) + (threadIdx.x >> 6);
+  if (s >= n) return;
   const int c = s / EX_CW, q = s % EX_CW;
   double sr = 0.0, si = 0.0;
-  for (int b = 0; b < nblk; b++) {
+  for (int b = threadIdx.x & 63; b < nblk; b += 64) {
     const double2 p = partial[((uint64_t)c * nblk + b) * EX_CW + q];
     sr += p.x;
     si += p.y;
   }
-  out[s] = make_double2(sr, si);
+  sr = wave_sum(sr);
+  si = wave_sum(si);
+  if ((threadIdx.x & 63) == 0) out[s] = make_double2(sr, si);
 }
 
 int ex_grid(uint64_t dim) {
@@ -166,65 +217,122 @@ void push_proj(std::vector<GTerm> &out, uint64_t mask, uint64_t val) {
   out.push_back(g);
 }
 
+// Items of the compiled slots: distinct terms without their factors, projectors
+// first, both kinds padded to EX_CW with items that never act.
+struct Items {
+  std::vector<CorrTerm<uint64_t>> t;
+  std::vector<int> of;  // item of every term, slot after slot
+  size_t nproj = 0;     // projectors with their padding
+  explicit Items(const std::vector<std::vector<GTerm>> &slots) {
+    size_t n = 0, cap = 64;
+    for (const auto &sl : slots) n += sl.size();
+    while (cap < 2 * n) cap *= 2;
+    std::vector<int> table(cap, -1), kind[2];
+    std::vector<CorrTerm<uint64_t>> uniq;
+    of.reserve(n);
+    for (const auto &sl : slots)
+      for (const GTerm &g : sl) {
+        uint64_t h = (g.flip * 0x9E3779B97F4A7C15ull) ^ (g.tmask * 0xBF58476D1CE4E5B9ull) ^
+                     (g.tval * 0x94D049BB133111EBull) ^ (g.sgn * 0xD6E8FEB86659FD93ull);
+        h ^= h >> 31;
+        for (;; h++) {
+          int &k = table[h & (cap - 1)];
+          if (k < 0) {
+            k = (int)uniq.size();
+            uniq.push_back(CorrTerm<uint64_t>{g.flip, g.tmask, g.tval, g.sgn});
+            kind[g.flip || g.sgn ? 1 : 0].push_back(k);
+          }
+          const CorrTerm<uint64_t> &u = uniq[k];
+          if (u.flip == g.flip && u.tmask == g.tmask && u.tval == g.tval && u.sgn == g.sgn) {
+            of.push_back(k);
+            break;
+          }
+        }
+      }
+    std::vector<int> at(uniq.size());
+    for (int c = 0; c < 2; c++) {
+      for (int k : kind[c]) {
+        at[k] = (int)t.size();
+        t.push_back(uniq[k]);
+      }
+      while (t.size() % EX_CW) t.push_back(CorrTerm<uint64_t>{0, 0, 1, 0});
+      if (c == 0) nproj = t.size();
+    }
+    for (int &k : of) k = at[k];
+  }
+};
+
+template <typename W, bool CANON>
+int corr_launch(hphi_engine *e, const double2 *v, const CorrTerm<W> *terms, int g, int nchunk, int np, double2 *part) {
+  for (int c0 = 0; c0 < nchunk; c0 += 65535) {  // grid.y limit
+    const int nc = nchunk - c0 < 65535 ? nchunk - c0 : 65535;
+    hipLaunchKernelGGL((k_corr<W, CANON>), dim3(g, nc), dim3(EX_TPB), 0, e->stream, v, e->d_list1, e->d_l21, e->d_l22,
+                       e->dim, (W)e->irght, e->nlow, terms + (size_t)c0 * EX_CW, np - c0,
+                       part + (size_t)c0 * g * EX_CW);
+    if (hipGetLastError() != hipSuccess) return hphi_set_error("hphi_expec: k_corr launch failed");
+  }
+  return 0;
+}
+
 // evaluate the compiled slots on v; out[2*s], out[2*s+1] = re, im
 int run_corr(hphi_engine *e, const double *v, const std::vector<std::vector<GTerm>> &slots, double *out) {
   const int nslot = (int)slots.size();
   if (nslot == 0) return 0;
   if (hphi_build_tables(e)) return -1;
-  std::vector<CorrTerm> h;
-  std::vector<int> toff(1, 0);
-  for (const auto &sl : slots) {
-    for (const GTerm &g : sl) h.push_back(CorrTerm{g.flip, g.tmask, g.tval, g.sgn, g.cre, g.cim});
-    toff.push_back((int)h.size());
-  }
-  const bool gc = hphi_model_gc(e->model);
-  const int g = ex_grid(e->dim), nchunk = (nslot + EX_CW - 1) / EX_CW;
-  CorrTerm *d_terms = nullptr;
-  int *d_toff = nullptr;
-  double2 *d_part = nullptr, *d_out = nullptr;
-  int rc = -1;
-  if (hphi_dev_alloc(sizeof(CorrTerm) * (h.size() + 1), (void **)&d_terms) ||
-      hphi_dev_alloc(sizeof(int) * toff.size(), (void **)&d_toff) ||
-      hphi_dev_alloc(sizeof(double2) * (size_t)nchunk * g * EX_CW, (void **)&d_part) ||
-      hphi_dev_alloc(sizeof(double2) * nslot, (void **)&d_out))
-    goto done;
-  if (!h.empty() && hipMemcpyAsync(d_terms, h.data(), sizeof(CorrTerm) * h.size(), hipMemcpyHostToDevice,
-                                   e->stream) != hipSuccess) {
-    hphi_set_error("hphi_expec: term upload failed");
-    goto done;
-  }
-  if (hipMemcpyAsync(d_toff, toff.data(), sizeof(int) * toff.size(), hipMemcpyHostToDevice, e->stream) !=
-      hipSuccess) {
-    hphi_set_error("hphi_expec: offset upload failed");
-    goto done;
-  }
-  for (int c0 = 0; c0 < nchunk; c0 += 65535) {  // grid.y limit
-    const int nc = nchunk - c0 < 65535 ? nchunk - c0 : 65535;
-    const int ns = (c0 + nc) * EX_CW < nslot ? (c0 + nc) * EX_CW : nslot;
-    // chunks c0.. run with blockIdx.y offset folded into the slot base
-    hipLaunchKernelGGL(k_corr, dim3(g, nc), dim3(EX_TPB), 0, e->stream, (const double2 *)v,
-                       gc ? (const uint64_t *)nullptr : e->d_list1, e->d_l21, e->d_l22, e->dim, e->irght, e->nlow,
-                       d_terms, d_toff + (size_t)c0 * EX_CW, ns - c0 * EX_CW, d_part + (size_t)c0 * g * EX_CW);
-    if (hipGetLastError() != hipSuccess) {
-      hphi_set_error("hphi_expec: k_corr launch failed");
-      goto done;
+  const Items I(slots);
+  std::vector<double> val(2 * I.t.size());
+  if (!I.t.empty()) {
+    const int n = (int)I.t.size(), nchunk = n / EX_CW, np = (int)(I.nproj / EX_CW);
+    // some 16 workgroups per CU over all chunks, and up to EX_GRID for one
+    int g = ex_grid(e->dim);
+    g = std::max(1, std::min(g, (16 * std::max(e->num_cu, 1) + nchunk - 1) / nchunk));
+    const bool narrow = e->nbits <= 32, gc = hphi_model_gc(e->model);
+    std::vector<CorrTerm<uint32_t>> t32;
+    const void *src = I.t.data();
+    size_t tb = sizeof(I.t[0]) * n;
+    if (narrow) {
+      for (const auto &t : I.t)
+        t32.push_back(CorrTerm<uint32_t>{(uint32_t)t.flip, (uint32_t)t.tmask, (uint32_t)t.tval, (uint32_t)t.sgn});
+      src = t32.data();
+      tb = sizeof(t32[0]) * n;
     }
+    const size_t at = (tb + 255) / 256 * 256, ao = at + sizeof(double2) * (size_t)nchunk * g * EX_CW;
+    char *d = nullptr;
+    if (hphi_dev_alloc(ao + sizeof(double2) * n, (void **)&d)) return -1;
+    double2 *part = (double2 *)(d + at), *res = (double2 *)(d + ao);
+    const double2 *vv = (const double2 *)v;
+    int rc = -1;
+    if (hipMemcpyAsync(d, src, tb, hipMemcpyHostToDevice, e->stream) != hipSuccess)
+      hphi_set_error("hphi_expec: term upload failed");
+    else if (narrow)
+      rc = gc ? corr_launch<uint32_t, false>(e, vv, (const CorrTerm<uint32_t> *)d, g, nchunk, np, part)
+              : corr_launch<uint32_t, true>(e, vv, (const CorrTerm<uint32_t> *)d, g, nchunk, np, part);
+    else
+      rc = gc ? corr_launch<uint64_t, false>(e, vv, (const CorrTerm<uint64_t> *)d, g, nchunk, np, part)
+              : corr_launch<uint64_t, true>(e, vv, (const CorrTerm<uint64_t> *)d, g, nchunk, np, part);
+    if (!rc) {
+      hipLaunchKernelGGL(k_corr_final, dim3((n + EX_TPB / 64 - 1) / (EX_TPB / 64)), dim3(EX_TPB), 0, e->stream,
+                         (const double2 *)part, g, n, res);
+      if (hipGetLastError() != hipSuccess ||
+          hipMemcpyAsync(val.data(), res, sizeof(double2) * n, hipMemcpyDeviceToHost, e->stream) != hipSuccess)
+        rc = hphi_set_error("hphi_expec: correlator pass failed");
+    }
+    if (hipStreamSynchronize(e->stream) != hipSuccess) rc = hphi_set_error("hphi_expec: correlator pass failed");
+    hphi_dev_free(d);
+    if (rc) return -1;
   }
-  hipLaunchKernelGGL(k_corr_final, dim3((nslot + 255) / 256), dim3(256), 0, e->stream, (const double2 *)d_part, g,
-                     nslot, d_out);
-  if (hipGetLastError() != hipSuccess ||
-      hipMemcpyAsync(out, d_out, sizeof(double2) * nslot, hipMemcpyDeviceToHost, e->stream) != hipSuccess ||
-      hipStreamSynchronize(e->stream) != hipSuccess) {
-    hphi_set_error("hphi_expec: correlator pass failed");
-    goto done;
+  size_t k = 0;
+  for (int s = 0; s < nslot; s++) {
+    double re = 0.0, im = 0.0;
+    for (const GTerm &g : slots[s]) {
+      const double *p = &val[2 * I.of[k++]];
+      re += g.cre * p[0] - g.cim * p[1];
+      im += g.cre * p[1] + g.cim * p[0];
+    }
+    out[2 * s] = re;
+    out[2 * s + 1] = im;
   }
-  rc = 0;
-done:
-  hphi_dev_free(d_terms);
-  hphi_dev_free(d_toff);
-  hphi_dev_free(d_part);
-  hphi_dev_free(d_out);
-  return rc;
+  return 0;
 }
 
 }  // namespace
