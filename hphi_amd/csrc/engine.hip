@@ -1071,6 +1071,9 @@ extern "C" int hphi_engine_tune(hphi_engine *e, const char *knob, int value) {
   } else if (k == "cls_blocks") {
     if (value != 0 && value != 1 && value != 2 && value != 4) return hphi_set_error("cls_blocks must be 0, 1, 2 or 4");
     e->cls_blocks = value;
+  } else if (k == "cls_order") {
+    if (value < -1 || value > 1) return hphi_set_error("cls_order must be -1, 0 or 1");
+    e->cls_order = value;
   } else if (k == "cls_wgs_per_cu") {
     if (value < 1 || value > 256) return hphi_set_error("cls_wgs_per_cu out of range");
     e->cls_wgs_per_cu = value;
@@ -1115,6 +1118,7 @@ extern "C" int hphi_engine_get_tune(const hphi_engine *e, const char *knob, int 
   else if (k == "use_blk") *value = e->use_blk && hphi_blk_ok(e);
   else if (k == "cls") *value = hphi_cls_wanted(e, 1);
   else if (k == "cls_blocks") *value = hphi_cls_blocks(e);
+  else if (k == "cls_order") *value = e->cls_args.groups[0] != nullptr;
   else if (k == "cls_wgs_per_cu") *value = e->cls_wgs_per_cu;
   else if (k == "gc_tile") *value = hphi_gc_wanted(e, 1) || hphi_gc_wanted(e, 2) || hphi_gc_wanted(e, 4) ||
                                     hphi_gc_wanted(e, 8) || hphi_gc_wanted(e, 16);

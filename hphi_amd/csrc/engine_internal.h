@@ -172,6 +172,11 @@ struct ClsArgs {
   uint32_t start[CL_MAXC], nblk[CL_MAXC], size[CL_MAXC], ntile[CL_MAXC], upre[CL_MAXC + 1];
   uint32_t lo[CL_MAXLO];
   const ClsTerm *terms;
+  // groups of 1, 2 and 4 blocks in launch order, (first slot, first block, blocks, ranks) each, and the group of
+  // every slot of 64 ranks; the launch's own in grp, sblk
+  const uint4 *groups[3], *grp;
+  const uint32_t *gslot[3], *sblk;
+  uint32_t ngroup[3], nslot[3];
   const uint32_t *bstart, *bxh, *tgt;  // per block in class order; tgt [block][high and mixed terms]
 };
 
@@ -250,8 +255,8 @@ struct hphi_engine {
   ulonglong2 *d_tofs = nullptr;  // per block: its first tile-major element, and the stride between its tiles
   HiPlan hi_plan{};
   // canonical H·v by classes: -1 unless a shape of k_hv_canon is set, 0 off, 1 on where the sector allows it
-  int cls = -1, cls_blocks = 0;
-  int cls_wgs_per_cu = 256;  // 8x4 J1-J2: 77.3 ms at 64, 75.1 at 256; 7x4: 3.67, 3.37; no effect below
+  int cls = -1, cls_blocks = 0, cls_order = -1;
+  int cls_wgs_per_cu = 256;  // by class: 8x4 J1-J2 77.3 ms at 64, 75.1 at 256; 7x4 3.67, 3.37; no effect below
   int c2_tuned = 0;  // a shape of k_hv_canon was set by hand
   void *d_cls = nullptr;
   ClsArgs cls_args{};

@@ -21,9 +21,9 @@
 // ones within a group).  Microseconds per H·v, k_hv_canon / this kernel:
 //   16-site J1-J2 chain (12,870 states)  15.6 / 10.8    6x4 J1-J2 (2.7e6)    292 / 151
 //   20-site ladder (184,756)             20.9 / 16.8    12-site Hubbard      55.3 / 34.4
-//   23-site chain (1.35e6)               90.2 / 50.5    7x4 J1-J2 (4.0e7)    5657 / 3380
-//   4x4 Hubbard (1.7e8)                14,350 / 12,880  8x4 J1-J2 (6.0e8, with the
-//   high-half pass)                    90,000 / 75,400
+//   23-site chain (1.35e6)               90.2 / 50.5    7x4 J1-J2 (4.0e7)    5657 / 3070
+//   4x4 Hubbard (1.7e8)                14,350 / 11,400  8x4 J1-J2 (6.0e8, with the
+//   high-half pass)                    90,000 / 69,700
 // The small ones are a chain of latencies, the middle ones were bound by that
 // arithmetic and are now by the L1's 64 bytes per cycle and L2; on 8x4 each of
 // the two halves of the terms misses L2 for 200 GB, 5.5 TB/s with the streams.
@@ -32,7 +32,7 @@
 // ranks.  k_hv_blk / this kernel, microseconds: 6x4 J1-J2 k = 2 492 / 302, k = 4 880 /
 // 600, k = 8 1,795 / 1,338, k = 16 3,926 / 3,266; 23-site chain k = 8 496 / 334;
 // 16-site chain k = 8 20.7 / 11.3; 12-site Hubbard k = 8 215 / 145; 7x4 k = 4 19,285 /
-// 16,455.  6x4 with k = 8 misses L2 for 9.1 GB, 7.1 TB/s: a state's columns fill a
+// 14,658.  6x4 with k = 8 misses L2 for 9.1 GB, 7.1 TB/s: a state's columns fill a
 // 128-byte line, so nothing of a gather is shared by neighbours, and the gathers
 // of 32 CUs reach further than their 4 MB.  Rank-slice order of the units (2 to
 // 64 tiles of every block before the next slice) gave nothing there and cost 10-25 %
@@ -40,6 +40,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstring>
 #include <map>
 #include <vector>
 
@@ -197,15 +198,26 @@ __global__ __launch_bounds__(CL_TPB) void k_hv_cls(const HvArgs A, const ClsArgs
 #pragma unroll
   for (int i = 0; i < CPL; i++) pre[i] = pim[i] = 0.0;
   for (uint32_t u = (uint32_t)((uint64_t)C.units * xcd / 8) + slot; u < U1; u += nslot) {
-    int c = 0, hi = C.ncls;  // upre[c] <= u < upre[hi]
-    while (hi - c > 1) {
-      const int mid = (c + hi) >> 1;
-      if (C.upre[mid] <= u) c = mid;
-      else hi = mid;
+    uint32_t p0, nb, size, tile;  // first block, blocks from there on in its class, ranks of the class, tile of ranks
+    if (C.sblk) {
+      const CU32 G = (CU32)C.grp + 4 * ((CU32)C.sblk)[u / LPS];
+      p0 = G[1];
+      nb = G[2];
+      size = G[3];
+      tile = u - G[0] * LPS;
+    } else {
+      int c = 0, hi = C.ncls;  // upre[c] <= u < upre[hi]
+      while (hi - c > 1) {
+        const int mid = (c + hi) >> 1;
+        if (C.upre[mid] <= u) c = mid;
+        else hi = mid;
+      }
+      const uint32_t loc = u - C.upre[c], ntile = C.ntile[c], grp = loc / ntile;
+      tile = loc % ntile;
+      size = C.size[c];
+      p0 = C.start[c] + grp * CB;
+      nb = C.start[c] + C.nblk[c] - p0;
     }
-    const uint32_t loc = u - C.upre[c], ntile = C.ntile[c], size = C.size[c];
-    const uint32_t grp = loc / ntile, tile = loc % ntile;
-    const uint32_t p0 = C.start[c] + grp * CB, nb = C.start[c] + C.nblk[c] - p0;  // blocks from here on
     const uint32_t r = tile * RPT + lane / LPS;
     if (r >= size) continue;
     const uint32_t own_off = r * (16u * K) + coff;
@@ -339,6 +351,13 @@ __global__ __launch_bounds__(256) void k_cls_targets(const uint32_t *bxh, const 
   tgt[i] = s ? (uint32_t)(s - 1) : CL_NONE;
 }
 
+// group of every slot
+__global__ __launch_bounds__(256) void k_cls_slots(const uint4 *grp, uint32_t n, uint32_t *sblk) {
+  const uint32_t g = blockIdx.x;
+  const uint32_t s0 = grp[g].x, m = (grp[g].w + 63) / 64;
+  for (uint32_t i = threadIdx.x; i < m; i += 256) sblk[s0 + i] = g;
+}
+
 // ---------------------------------------------------------------- host ----
 
 // the particle numbers a term changes, per species; false: not known from its masks
@@ -368,14 +387,15 @@ static bool cls_possible(const hphi_engine *e) {
 // 10.8 us with one, 13.1 with two, 18.1 with four; 184,756: 16.8, 17.5, 22.3).
 // Where the vectors sit in the caches and arithmetic counts: two for Spin
 // (1.35e6: 56.9, 50.5, 56.4; 2.7e6: 168, 151, 169), four for Hubbard, whose rank
-// lookup costs more (8.5e5: 43.0, 37.8, 34.4; 1.7e8: 14,005, 13,378, 12,885).
-// Spin vectors beyond the caches: one, whose rank tiles follow closest on each
-// other in a block (4.0e7: 3,380, 3,688, 3,711; 6.0e8: 75,400, 78,213, 80,848).
+// lookup costs more (8.5e5: 43.0, 37.8, 34.4).  Beyond the caches: one, whose rank
+// tiles follow closest on each other in a block (Spin 4.0e7: 3,070, 3,197, 3,527; 6.0e8:
+// 69,733, 72,963 with two; Hubbard 1.7e8: 11,393, 11,407, 11,573).
 int hphi_cls_blocks(const hphi_engine *e) {
   if (e->cls_blocks > 0) return e->cls_blocks;
   const uint64_t d = e->dim;
+  if (d >= (uint64_t)1 << 24) return 1;
   if (e->model == HPHI_MODEL_HUBBARD) return d < ((uint64_t)1 << 17) ? 1 : d < ((uint64_t)1 << 19) ? 2 : 4;
-  return d < ((uint64_t)1 << 18) || d >= ((uint64_t)1 << 24) ? 1 : 2;
+  return d < ((uint64_t)1 << 18) ? 1 : 2;
 }
 
 // Blocks per wave and columns per lane of a block of k columns.  One column per
@@ -384,7 +404,7 @@ int hphi_cls_blocks(const hphi_engine *e) {
 // Hubbard's rank lookup is worth sharing by two (8.5e5, k = 8: 170, 145, 187).
 // Blocks: one while k columns still leave few waves (12,870 states, k = 8: 11.3,
 // 13.0, 17.6 us with one, two, four), then two (2.7e6: 1,384, 1,338, 1,364), four
-// beyond the caches (4.0e7, k = 4: 17,865, 17,159, 16,455).
+// beyond the caches (4.0e7, k = 4: 15,032, 14,865, 14,658).
 void hphi_cls_shape(const hphi_engine *e, int k, int *cb, int *cpl) {
   *cb = hphi_cls_blocks(e);
   *cpl = 1;
@@ -546,11 +566,66 @@ int hphi_cls_upload(const hphi_engine *e, ClsArgs &A, char *dev, const void *up,
   return 0;
 }
 
+// The order of the units.  A vector that the 256 MB memory-side cache holds: class
+// after class, an XCD the next eighth of them after the other, so that each XCD's
+// gathers stay near its own part and meet in its L2 (2.7e6 states 151 us; with the
+// order below 175).  Beyond (2^24 states) gathers that miss L2 would miss that
+// cache too, at the 5.5 TB/s of HBM: groups follow the first index of their first
+// block and are dealt to the XCDs one by one, to the one with the fewest slots, so
+// that all XCDs work in one neighbourhood of the vector instead of eight.  Class
+// after class / by index, an eighth per XCD / dealt one by one / four by four:
+// 8x4 75.3, 72.7, 69.7, 70.5 ms; 7x4 3,380, 3,254, 3,070, 3,071 us, k = 4 16,455, 16,431,
+// 14,658; 4x4 Hubbard 12,880, 13,667 (one block per wave), 11,400, 11,634.
+static int cls_by_index(const hphi_engine *e) {
+  if (e->cls_order >= 0) return e->cls_order;
+  return e->dim >= (uint64_t)1 << 24;
+}
+
+// Groups of cb blocks of a class in the order of a vector beyond the caches.
+static uint32_t cls_groups(const hphi_engine *e, const ClsArgs &A, const uint32_t *xh, uint32_t cb,
+                           std::vector<uint4> &out) {
+  std::vector<uint32_t> at((size_t)1 << (e->nbits - e->nlow), CL_NONE);  // class and first block by high half
+  std::vector<uint32_t> cls(at.size());
+  for (int c = 0; c < A.ncls; c++)
+    for (uint32_t i = 0; i < A.nblk[c]; i += cb) {
+      const uint32_t h = xh[A.start[c] + i] >> e->nlow;
+      at[h] = A.start[c] + i;
+      cls[h] = c;
+    }
+  std::vector<uint4> q[8];
+  uint32_t load[8] = {};
+  for (size_t h = 0; h < at.size(); h++) {
+    if (at[h] == CL_NONE) continue;
+    const int c = cls[h], x = (int)(std::min_element(load, load + 8) - load);
+    q[x].push_back(make_uint4(0, at[h], std::min(cb, A.start[c] + A.nblk[c] - at[h]), A.size[c]));
+    load[x] += (A.size[c] + 63) / 64;
+  }
+  uint32_t slot = 0;
+  for (const auto &v : q)
+    for (uint4 g : v) {
+      g.x = slot;
+      slot += (g.w + 63) / 64;
+      out.push_back(g);
+    }
+  return slot;
+}
+
 // One device allocation, written on e->stream, which the caller waits for before it
 // frees up.  Sectors or terms the layout does not fit keep k_hv_canon.
 int hphi_cls_build(hphi_engine *e, std::vector<char> &up) {
-  if (e->d_cls || e->cls == 0 || !e->c2_ok || !e->c2_crank_ok || !hphi_cls_plan(e, e->cls_args, up)) return 0;
-  const size_t bytes = hphi_cls_bytes(e->cls_args);
+  ClsArgs &A = e->cls_args;
+  if (e->d_cls || e->cls == 0 || !e->c2_ok || !e->c2_crank_ok || !hphi_cls_plan(e, A, up)) return 0;
+  const size_t plan = (hphi_cls_bytes(A) + 255) / 256 * 256;
+  std::vector<uint4> grp;
+  const uint32_t *xh = (const uint32_t *)(up.data() + sizeof(ClsTerm) * (size_t)(A.n_low + A.nt)) + A.np;
+  uint64_t slots = 0;
+  for (int i = 0; i < 3 && cls_by_index(e); i++) {
+    const size_t n = grp.size();
+    A.nslot[i] = cls_groups(e, A, xh, 1u << i, grp);
+    A.ngroup[i] = (uint32_t)(grp.size() - n);
+    slots += A.nslot[i];
+  }
+  const size_t gb = sizeof(uint4) * grp.size(), bytes = plan + gb + 4 * slots;
   char *p = nullptr;
   if (hipMalloc((void **)&p, std::max<size_t>(bytes, 1)) != hipSuccess) {
     (void)hipGetLastError();
@@ -558,7 +633,35 @@ int hphi_cls_build(hphi_engine *e, std::vector<char> &up) {
   }
   e->d_cls = p;
   e->bytes += bytes;
-  return hphi_cls_upload(e, e->cls_args, p, up.data(), e->d_l22, e->stream);
+  const size_t at = (up.size() + 15) / 16 * 16;  // the groups follow the plan's upload
+  up.resize(at + gb);
+  if (gb) memcpy(up.data() + at, grp.data(), gb);
+  if (hphi_cls_upload(e, A, p, up.data(), e->d_l22, e->stream)) return -1;
+  if (!gb) return 0;
+  HIPCHK(hipMemcpyAsync(p + plan, up.data() + at, gb, hipMemcpyHostToDevice, e->stream));
+  const uint4 *dg = (const uint4 *)(p + plan);
+  uint32_t *ds = (uint32_t *)(p + plan + gb);
+  for (int i = 0; i < 3; i++) {
+    A.groups[i] = dg;
+    A.gslot[i] = ds;
+    hipLaunchKernelGGL(k_cls_slots, dim3(A.ngroup[i]), dim3(256), 0, e->stream, dg, A.ngroup[i], ds);
+    dg += A.ngroup[i];
+    ds += A.nslot[i];
+  }
+  HIPCHK(hipGetLastError());
+  return 0;
+}
+
+// groups and units (a tile of 64 / lps ranks of a group) of a launch with cb blocks per wave
+static void cls_launch_units(ClsArgs &A, int cb, int lps) {
+  const int i = cb == 4 ? 2 : cb - 1;
+  if (!A.groups[i]) {
+    hphi_cls_units(A, cb, 64 / lps);
+    return;
+  }
+  A.grp = A.groups[i];
+  A.sblk = A.gslot[i];
+  A.units = A.nslot[i] * (uint32_t)lps;
 }
 
 // units (a rank tile of a group of blocks) of a launch with cb blocks per wave
@@ -578,7 +681,7 @@ int hphi_cls_grid(const hphi_engine *e, int k) {
   ClsArgs A = e->cls_args;
   int cb, cpl;
   hphi_cls_shape(e, k, &cb, &cpl);
-  hphi_cls_units(A, cb, 64 * cpl / k);
+  cls_launch_units(A, cb, k / cpl);
   const uint64_t want = (A.units + CL_TPB / 64 - 1) / (CL_TPB / 64);
   uint64_t g = std::min<uint64_t>(want, (uint64_t)e->cls_wgs_per_cu * std::max(e->num_cu, 1));
   g = std::max<uint64_t>((g + 7) / 8 * 8, 8);
@@ -607,7 +710,7 @@ int hphi_hv_launch_cls(hphi_engine *e, const HvArgs &H, int k, int g, int skip_h
   ClsArgs A = e->cls_args;
   int cb, cpl;
   hphi_cls_shape(e, k, &cb, &cpl);
-  hphi_cls_units(A, cb, 64 * cpl / k);
+  cls_launch_units(A, cb, k / cpl);
   if (skip_high) A.skip = A.n_high;  // the high terms have a pass of their own
 #define CASE(KK, CC, BB) \
   if (k == KK && cpl == CC && cb == BB) return cls_launch<KK, CC, BB>(e, H, A, g);

@@ -118,7 +118,9 @@ int hphi_engine_info(const hphi_engine *e, uint64_t *dim, uint64_t *size21, uint
  *   canonical H·v by classes: "cls" -1|0|1 (-1: unless one of tpb, wgs_per_cu,
  *   lds21, c2_crank, c2_unroll or xcd_map is set, for k > 1 one of blk_tpb,
  *   blk_wgs_per_cu or blk_cpl of this k; read back: whether it is in use for
- *   k = 1), "cls_blocks" 0|1|2|4 (blocks per wave, 0 by size), "cls_wgs_per_cu" 1..256;
+ *   k = 1), "cls_blocks" 0|1|2|4 (blocks per wave, 0 by size), "cls_wgs_per_cu" 1..256,
+ *   "cls_order" -1|0|1 (units by class, or by index dealt to the XCDs one by one; -1:
+ *   by index from 2^24 states on; set before the tables are built);
  *   grand-canonical H·v in LDS tiles: "gc_tile" -1|0|1 (-1: sectors of at
  *   least 256 tiles, unless a block-kernel knob is set; 1: every sector with 8
  *   tiles, set before the diagonal is built; read back: whether the engine has

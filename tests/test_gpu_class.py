@@ -122,3 +122,26 @@ def test_class_kernel_block(A, name, spec, k):
     for b, q, _ in out[1:]:
         assert np.max(np.abs(b - a)) <= TOL * np.max(np.abs(a))
         assert np.max(np.abs(q - p)) <= TOL * s
+
+
+@pytest.mark.parametrize("k", [1, 2, 16])
+@pytest.mark.parametrize("name,spec", CASES, ids=[c[0] for c in CASES])
+def test_units_by_index_equal_units_by_class(A, name, spec, k):
+    """The order for vectors beyond the caches, for 1, 2 and 4 blocks per wave."""
+    out = []
+    for tune in [dict(cls_order=0)] + [dict(cls_order=1, cls_blocks=cb, cls_wgs_per_cu=w) for cb, w in ((1, 256), (2, 1), (4, 256))]:
+        print(f"[gpu] class order {name} k {k} {tune}", flush=True)
+        e = A.Engine.from_spec(spec)
+        e.tune(cls=1, **tune)
+        e.sz(copy=False)
+        e.diagonalcalc(copy=False)
+        assert e.get_tune("cls_order") == tune["cls_order"]
+        v = np.random.default_rng(8).standard_normal(2 * e.dim * k).view(np.complex128)
+        v1, v0 = A.DeviceArray(e.dim * k).upload(v), A.DeviceArray(e.dim * k).upload(2 * v)
+        p = e.mltply_block_dev(k, v0, v1)
+        out.append((v0.download(), p))
+        e.close()
+    a, p = out[0]
+    for b, q in out[1:]:
+        assert np.max(np.abs(b - a)) <= TOL * np.max(np.abs(a))
+        assert np.max(np.abs(q - p)) <= TOL * np.linalg.norm(v) * np.linalg.norm(a)
