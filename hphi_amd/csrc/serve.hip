@@ -649,25 +649,35 @@ __global__ __launch_bounds__(SV_TPB) void k_sl_cls(const SlabDev *slabs, const u
   }
 }
 
-// per job (one workgroup each): fixed-order sum over the slab's tiles of one column
+// per job (one workgroup each): fixed-order sum over the slab's tiles of one
+// column.  Latency-bound: up to 10,600 partial sums of a 24-site slab, eight loads
+// in flight on 1,024 threads (256 threads, one each: 19.1 and 13.7 us per launch for
+// beta and alpha in a burst of 40 jobs; now 8.0 and 8.4).
+#define CS_TPB 1024
+#define CS_U 8
 __device__ double col_sum(const double *part, int stride, uint64_t t0, uint64_t t1) {
-  __shared__ double s[256];
-  double a = 0.0;
-  for (uint64_t t = t0 + threadIdx.x; t < t1; t += 256) a += part[t * stride];
-  s[threadIdx.x] = a;
-  __syncthreads();
-  for (int st = 128; st > 0; st >>= 1) {
-    if (threadIdx.x < st) s[threadIdx.x] += s[threadIdx.x + st];
-    __syncthreads();
+  __shared__ double s[CS_TPB / 64];
+  double a[CS_U];
+#pragma unroll
+  for (int u = 0; u < CS_U; u++) a[u] = 0.0;
+  for (uint64_t t = t0 + threadIdx.x; t < t1; t += CS_TPB * CS_U) {
+#pragma unroll
+    for (int u = 0; u < CS_U; u++)
+      if (t + u * CS_TPB < t1) a[u] += part[(t + u * CS_TPB) * stride];
   }
-  const double r = s[0];
+#pragma unroll
+  for (int u = 1; u < CS_U; u++) a[0] += a[u];
+  for (int o = 32; o > 0; o >>= 1) a[0] += __shfl_xor(a[0], o, 64);
+  if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = a[0];
   __syncthreads();
+  double r = 0.0;
+  for (int w = 0; w < CS_TPB / 64; w++) r += s[w];
   return r;
 }
 
 // beta_{m-1} = |w_m| and s_m = 1/beta_{m-1}; a beta below 1e-14 ends the
 // recurrence (the Krylov space is exhausted) and s_m = 0 keeps pass 2 finite
-__global__ __launch_bounds__(256) void k_sl_norm(const ColDev *cols, const uint64_t *prefix, const double *partial,
+__global__ __launch_bounds__(CS_TPB) void k_sl_norm(const ColDev *cols, const uint64_t *prefix, const double *partial,
                                                  double *js) {
   CCol J = (CCol)cols + blockIdx.x;
   const double b2 = col_sum(partial + J->col, SL_K, ((CU64)prefix)[J->slab], ((CU64)prefix)[J->slab + 1]);
@@ -681,7 +691,7 @@ __global__ __launch_bounds__(256) void k_sl_norm(const ColDev *cols, const uint6
 }
 
 // alpha_m = s_m^2 Re <w|H w>; out = (alpha_m, beta_{m-1}) per job
-__global__ __launch_bounds__(256) void k_sl_alpha(const ColDev *cols, const uint64_t *prefix, const double2 *partial,
+__global__ __launch_bounds__(CS_TPB) void k_sl_alpha(const ColDev *cols, const uint64_t *prefix, const double2 *partial,
                                                   double *js, double *out) {
   CCol J = (CCol)cols + blockIdx.x;
   const double a = col_sum((const double *)partial + 2 * J->col, 2 * SL_K, ((CU64)prefix)[J->slab],
@@ -1589,7 +1599,7 @@ extern "C" int hphi_server_tick(hphi_server *s, int *n_active, int *n_waiting) {
       double *out = s->d_out + (size_t)st * 2 * n;
       hipLaunchKernelGGL(k_sl_resid, dim3(T), dim3(SV_TPB), 0, s->stream, dsl, dpf, ns, (const double *)s->d_js,
                          s->d_part);
-      hipLaunchKernelGGL(k_sl_norm, dim3(nc), dim3(256), 0, s->stream, dcl, dpf, (const double *)s->d_part,
+      hipLaunchKernelGGL(k_sl_norm, dim3(nc), dim3(CS_TPB), 0, s->stream, dcl, dpf, (const double *)s->d_part,
                          s->d_js);
       HIPCHK(hipEventRecord(s->ev_hv[2 * st], s->stream));
       const uint64_t *dpv = s->d_prefix + s_pv0[st], *pvh = prefix.data() + s_pv0[st];
@@ -1601,7 +1611,7 @@ extern "C" int hphi_server_tick(hphi_server *s, int *n_active, int *n_waiting) {
         hipLaunchKernelGGL(k_sl_hv, dim3((unsigned)(pvh[ns] - pvh[nk])), dim3(SV_TPB), lds, s->stream,
                            dsl + nk, dpv + nk, ns - nk, (const double *)s->d_js, (double2 *)s->d_part);
       HIPCHK(hipEventRecord(s->ev_hv[2 * st + 1], s->stream));
-      hipLaunchKernelGGL(k_sl_alpha, dim3(nc), dim3(256), 0, s->stream, dcl, dpv, (const double2 *)s->d_part,
+      hipLaunchKernelGGL(k_sl_alpha, dim3(nc), dim3(CS_TPB), 0, s->stream, dcl, dpv, (const double2 *)s->d_part,
                          s->d_js, out);
       if (s_chk[st]) hipLaunchKernelGGL(k_sl_check, dim3(nc), dim3(CK_TPB), 0, s->stream, dcl, s->p.n_eigen, s->d_ev);
       HIPCHK(hipGetLastError());
