@@ -259,9 +259,9 @@ def pmc_probe(args):
     eng.close()
 
 
-# kernels of one plain H·v: k_hv_canon, and for large canonical Spin sectors
+# kernels of one plain H·v: k_hv_cls (or k_hv_canon), and for large canonical Spin sectors
 # also the tile-major copy of v1 and the high-half pass (one dispatch each)
-HV_KERNELS = ("k_hv_canon", "k_hi_copy", "k_hv_high")
+HV_KERNELS = ("k_hv_cls", "k_hv_canon", "k_hi_copy", "k_hv_high")
 
 
 def _pmc_means(directory: str, counter: str):
@@ -363,9 +363,9 @@ def reduce_issue(directory: str, out: str, cmd: str, cfg: int = 2):
 
     spec = L.baseline_config(cfg)
     dim = spec.dim
-    vals = {c: _pmc_means(directory, c).get("k_hv_canon") for c in ISSUE_COUNTERS}
+    vals = {c: _pmc_means(directory, c).get("k_hv_cls") for c in ISSUE_COUNTERS}
     tiles = dim / 64.0
-    lines = [f"# issue counters of one plain H·v launch (k_hv_canon), {PMC_WORKLOADS[cfg][1]}",
+    lines = [f"# issue counters of one plain H·v launch (k_hv_cls), {PMC_WORKLOADS[cfg][1]}",
              f"# command: {cmd}"]
     for c in ISSUE_COUNTERS:
         v = vals[c]
@@ -810,7 +810,7 @@ def main():
             "speedup_vs_sequential": round(p0["solves_per_s"] / sv["sequential_solves_per_s"], 3),
             "rate_per_s": 120.0, "p50_s": round(p1["p50_s"], 3), "p99_s": round(p1["p99_s"], 3),
             "converged": [p0["converged"], p1["converged"]],
-            "slab_hv": {"kernel": "k_sl_hv", "achieved_gbs": p0["hv_gbs"], "frac": p0["hv_frac"],
+            "slab_hv": {"kernel": "k_sl_cls", "achieved_gbs": p0["hv_gbs"], "frac": p0["hv_frac"],
                         "launches": p0["hv_launches"],
                         "note": "algorithmic bytes (per slab 8 dim, per running column 56 dim + 16 per "
                                 "off-diagonal element) over HIP-event time of the slab H·v launches"},

@@ -16,6 +16,8 @@
 // Grand-canonical spin states are their own index (target = x ^ flip).
 // Same arithmetic as the per-term scatter of the reference
 // (mltplySpinCore.c:273-345, mltplyHubbardCore.c:305-347), in gather form.
+// Serves grand-canonical blocks below the tile kernel's size and LOBPCG's, and
+// canonical ones without the class layout (hv_class.hip).
 #include <hip/hip_runtime.h>
 
 #include "engine_internal.h"

@@ -1,5 +1,6 @@
 // Gather-form H·v for canonical models (Spin, Hubbard) with states of at
-// most 32 bits, one lane per basis state — the hot kernel of the plain path.
+// most 32 bits, one lane per basis state: the plain path where the class layout
+// (hv_class.hip) does not serve; and the high-half pass of both.
 //
 // Same arithmetic as k_hv in engine.hip (transpose of the reference's
 // per-term scatter, mltplySpinCore.c:273-307, mltplyHubbardCore.c:305-347),
@@ -288,7 +289,8 @@ __global__ __launch_bounds__(TPB) void k_hv_canon(const HvArgs A) {
 // while it is cached.  On the 8x4 J1-J2 sector: 101.6 ms in one pass; 89.8 ms
 // as k_hv_canon without the high group (62 ms), the copy (4.8 ms) and this
 // pass (23 ms); 90.0 ms with the copy fused and the first pass on a larger
-// grid, on a box where the single pass takes 107.4 ms.
+// grid, where the single pass takes 107.4 ms.  After k_hv_cls: 46.8 ms, and 20.7
+// for this pass, against 76.9 in one pass.
 
 __device__ __forceinline__ bool hi_unit(const HiPlan &P, uint64_t u, int &c, uint32_t &R, uint32_t &grp) {
   while (u >= P.wgp[c + 1]) c++;  // a workgroup's units only increase
@@ -419,7 +421,7 @@ __global__ __launch_bounds__(256) void k_hv_high(const HvArgs A, const HiPlan P,
 #define HI_UNR 8  // high terms per batch of the high-half pass (16: 95-101 ms against 93.5 on one box)
 
 // sectors of at least this many states take the high-half pass by default
-// (J1-J2 7x4, 40M states: 5.19 ms either way; 6x4, 2.7M: 0.29 against 0.29 ms)
+// (J1-J2 7x4, 40M states, after k_hv_cls: 3.55 ms in two passes, 3.08 in one)
 #define HI_AUTO_DIM ((uint64_t)1 << 27)
 
 // Hubbard orbitals 2i + sigma: up electrons at even bit positions
