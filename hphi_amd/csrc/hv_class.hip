@@ -23,10 +23,10 @@
 //   20-site ladder (184,756)             20.9 / 16.8    12-site Hubbard      55.3 / 34.4
 //   23-site chain (1.35e6)               90.2 / 50.5    7x4 J1-J2 (4.0e7)    5657 / 3070
 //   4x4 Hubbard (1.7e8)                14,350 / 11,400  8x4 J1-J2 (6.0e8, with the
-//   high-half pass)                    90,000 / 69,700
+//   high-half pass)                    90,000 / 67,400
 // The small ones are a chain of latencies, the middle ones were bound by that
-// arithmetic and are now by the L1's 64 bytes per cycle and L2; on 8x4 each of
-// the two halves of the terms misses L2 for 200 GB, 5.5 TB/s with the streams.
+// arithmetic and are now by the L1's 64 bytes per cycle and L2; the first pass of 8x4
+// fetches 240 GB from beyond L2 in 46.8 ms, 5.1 TB/s.
 //
 // Blocks of K columns: LPS = K / CPL lanes share a state and a wave takes 64 / LPS
 // ranks.  k_hv_blk / this kernel, microseconds: 6x4 J1-J2 k = 2 492 / 302, k = 4 880 /

@@ -719,7 +719,7 @@ __global__ __launch_bounds__(CS_TPB) void k_sl_alpha(const ColDev *cols, const u
 // CK_S - 1 others): some 14 rounds of 17 sections instead of 55 halvings down to
 // the same two adjacent numbers.  alpha and beta are staged in LDS (CK_LDS of
 // them; longer histories are read from memory), bounds and the ghost test use all lanes.
-// A burst of 40 jobs: 1,466 us per check with one lane per eigenvalue, 397 now.
+// A burst of 40 jobs: 1,466 us per check with one lane per eigenvalue, 360-400 now.
 #define CK_EXTRA 6
 #define CK_TPB 512
 #define CK_S 16       // lanes, i.e. points per round, of one eigenvalue's search
