@@ -16,6 +16,7 @@
 #include "hphi_amd.h"
 
 int hphi_set_error(const char *fmt, ...);
+int hphi_block_size_ok(const char *entry, int k);
 
 typedef struct {
   int n;
@@ -38,6 +39,7 @@ static int apply(hphi_engine *e, const cand_t *c) {
 int hphi_autotune(hphi_engine *e, int k, double *v0, const double *v1, int reps, char *report,
                   size_t report_len) {
   if (!e || !v0 || !v1) return hphi_set_error("hphi_autotune: NULL argument");
+  if (hphi_block_size_ok("hphi_autotune", k)) return -1;
   if (reps < 1) reps = 2;
   cand_t cands[96];
   int n = 0, c2 = 0, blk = 0, lds_ok = 0, crank_ok = 0, gc = 0, cls = 0;

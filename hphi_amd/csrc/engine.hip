@@ -1418,6 +1418,13 @@ static int hv_launch_args(hphi_engine *e, int k, HvArgs &A, double2 *prdct_out, 
   return 0;
 }
 
+// Block sizes with kernels: tested at every entry that takes one, before any
+// grid is computed from it.
+extern "C" int hphi_block_size_ok(const char *entry, int k) {
+  if (k == 1 || k == 2 || k == 4 || k == 8 || k == 16) return 0;
+  return hphi_set_error("%s: block size k=%d not in {1,2,4,8,16}", entry, k);
+}
+
 static int ensure_ready(hphi_engine *e) {
   if (hphi_build_tables(e)) return -1;
   if (hphi_build_diag(e)) return -1;
@@ -1474,6 +1481,7 @@ extern "C" int hphi_mltply_dev_scaled(hphi_engine *e, double *v0, const double *
 
 extern "C" int hphi_mltply_block_dev(hphi_engine *e, int k, double *V0, const double *V1, double *prdct) {
   if (!e || !V0 || !V1) return hphi_set_error("hphi_mltply_block_dev: NULL argument");
+  if (hphi_block_size_ok("hphi_mltply_block_dev", k)) return -1;
   if (ensure_ready(e)) return -1;
   HvArgs A = hphi_hv_args(e, k, V0, V1);
   return hv_call(e, k, A, prdct);
@@ -1504,8 +1512,7 @@ int hphi_noalloc_setup(int device) {
 
 extern "C" int hphi_mltply_block_dev_noalloc(hphi_engine *e, int k, double *V0, const double *V1, double *prdct) {
   if (!e || !V0 || !V1) return hphi_set_error("hphi_mltply_block_dev_noalloc: NULL argument");
-  if (k != 1 && k != 2 && k != 4 && k != 8 && k != 16)
-    return hphi_set_error("hphi_mltply_block_dev_noalloc: block size k=%d not in {1,2,4,8,16}", k);
+  if (hphi_block_size_ok("hphi_mltply_block_dev_noalloc", k)) return -1;
   if (!e->tables_ready || !e->diag_ready)
     return hphi_set_error("hphi_mltply_block_dev_noalloc: basis tables and diagonal are not built; call hphi_sz "
                           "and hphi_diagonalcalc first (this entry point allocates nothing)");
@@ -1694,6 +1701,7 @@ extern "C" int hphi_fill_random(double *v, uint64_t dim, int k, uint64_t seed) {
 extern "C" int hphi_time_mltply_dev(hphi_engine *e, int k, double *v0, const double *v1, int warmup,
                                     int reps, double *avg_ms) {
   if (!e || !v0 || !v1 || reps < 1) return hphi_set_error("hphi_time_mltply_dev: bad argument");
+  if (hphi_block_size_ok("hphi_time_mltply_dev", k)) return -1;
   if (ensure_ready(e)) return -1;
   for (int i = 0; i < warmup; i++)
     if (hphi_hv_launch(e, k, v0, v1)) return -1;

@@ -268,6 +268,7 @@ struct hphi_engine {
 };
 
 extern "C" int hphi_set_error(const char *fmt, ...);
+extern "C" int hphi_block_size_ok(const char *entry, int k);
 int hphi_build_tables(hphi_engine *e);
 int hphi_build_diag(hphi_engine *e);
 int hphi_hv_launch(hphi_engine *e, int k, double *v0, const double *v1);

@@ -418,7 +418,8 @@ void hphi_cls_shape(const hphi_engine *e, int k, int *cb, int *cpl) {
 int hphi_cls_wanted(const hphi_engine *e, int k) {
   if (!e->d_cls || !e->c2_crank || e->cls == 0) return 0;
   if (k == 1) return e->use_c2 && (e->cls == 1 || !e->c2_tuned);
-  const int slot = k == 2 ? 0 : k == 4 ? 1 : k == 8 ? 2 : 3;
+  const int slot = k == 2 ? 0 : k == 4 ? 1 : k == 8 ? 2 : k == 16 ? 3 : -1;
+  if (slot < 0) return 0;
   return e->use_blk && (e->cls == 1 || !(e->bk_tpb || e->bk_wgs_per_cu || e->bk_cpl[slot]));
 }
 

@@ -1,0 +1,29 @@
+"""Host-side plans of the H·v kernels (no device): which kernel serves which
+call, and how the terms are filed.  host_plans.hip prints the answers."""
+
+import os
+import subprocess
+
+import pytest
+
+from hphi_amd import build as B
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture(scope="module")
+def plans(tmp_path_factory):
+    from hphi_amd import capi
+    if not os.path.exists(capi.LIB_PATH):
+        B.build()
+    exe = str(tmp_path_factory.mktemp("plans") / "host_plans")
+    lib = os.path.dirname(capi.LIB_PATH)
+    subprocess.run([B.HIPCC] + B.HIP_FLAGS + ["--offload-host-only", "-O1", os.path.join(HERE, "host_plans.hip"), "-o", exe,
+                                              "-L" + lib, "-lhphi_amd", "-Wl,-rpath," + lib], check=True)
+    out = subprocess.run([exe], check=True, capture_output=True, text=True).stdout
+    return dict(ln.split(" ", 1) for ln in out.splitlines())
+
+
+@pytest.mark.parametrize("k", [1, 2, 4, 8, 16, 0, -1, 3, 32, 64, 65, 128, 1024, 1028])
+def test_class_kernel_serves_its_block_sizes_only(plans, k):
+    assert int(plans[f"cls_wanted_{k}"]) == (k in (1, 2, 4, 8, 16))
