@@ -480,7 +480,10 @@ bool hphi_cls_plan(const hphi_engine *e, ClsArgs &A, std::vector<char> &up) {
     at.insert(at.end(), k.second.at.begin(), k.second.at.end());
     xh.insert(xh.end(), k.second.xh.begin(), k.second.xh.end());
   }
-  // terms by group: pure low, pure high, the others
+  // terms by group: pure low; those that leave the high half for another block
+  // and touch no low bit, the same ones the engine files under high, so that
+  // the high-half pass applies exactly what this kernel then skips (a term
+  // without a flip whose mask lies in the high half is none of them); the others
   std::vector<ClsTerm> grp[5];  // low by parity, low by value, high, mixed by parity, mixed by value
   std::vector<uint32_t> lo;
   for (size_t i = 0; i < e->h_terms_dev.size(); i++) {
@@ -497,7 +500,7 @@ bool hphi_cls_plan(const hphi_engine *e, ClsArgs &A, std::vector<char> &up) {
     c.sgn = (uint32_t)t.sgn;
     c.parity = t.kind == P_DIFF;
     c.src = (int)i;
-    const int g = (all & hm) == 0 ? 0 : (all & e->irght) == 0 ? 1 : 2;
+    const int g = (all & hm) == 0 ? 0 : (all & e->irght) == 0 && (t.flip & hm) ? 1 : 2;
     if (g == 2) {
       const uint32_t f = (uint32_t)(t.flip & e->irght);
       size_t q = std::find(lo.begin(), lo.end(), f) - lo.begin();

@@ -33,7 +33,41 @@ static void block_sizes() {
     printf("cls_wanted_%d %d\n", k, hphi_cls_wanted(&e, k));
 }
 
+// terms whose flip leaves the high half: the engine's group against the class
+// layout's, for hops, a density product in the high half and a density-assisted hop
+static void high_terms() {
+  const int n = 6;
+  std::vector<int> idx;
+  std::vector<double> t;
+  for (int i = 0; i < n; i++)
+    for (int s = 0; s < 2; s++) {
+      const int j = (i + 1) % n, a[8] = {i, s, j, s, j, s, i, s};
+      idx.insert(idx.end(), a, a + 8);
+      for (int q = 0; q < 2; q++) t.push_back(1.0), t.push_back(0.0);
+    }
+  const int ia[] = {4, 0, 4, 0, 5, 1, 5, 1, 5, 0, 5, 0, 0, 0, 1, 0, 1, 0, 0, 0, 5, 0, 5, 0};
+  const double iv[] = {0.7, 0.0, 0.2, 0.1, 0.2, -0.1};
+  hphi_model_desc d{};
+  d.model = HPHI_MODEL_HUBBARD, d.nsite = n, d.nup = 3, d.ndown = 3;
+  d.n_transfer = (int)idx.size() / 4, d.transfer_idx = idx.data(), d.transfer_t = t.data();
+  d.n_interall = 3, d.interall_idx = ia, d.interall_V = iv;
+  hphi_engine e;
+  std::vector<char> up;
+  if (!plan(d, e, up)) return;
+  e.hi_split = 1;
+  const ClsTerm *T = (const ClsTerm *)up.data();
+  int differ = 0, high = 0;
+  for (int i = 0; i < e.cls_args.n_low + e.cls_args.nt; i++) {
+    if (T[i].src < 0) continue;
+    const bool here = i >= e.cls_args.n_low && i < e.cls_args.n_low + e.cls_args.n_high;
+    differ += here != (T[i].src >= e.n_low && T[i].src < e.n_low + e.n_high);
+    high += here;
+  }
+  printf("hi_wanted %d\nhigh_terms %d\nhigh_filed_differently %d\n", hphi_hi_wanted(&e), high, differ);
+}
+
 int main() {
   block_sizes();
+  high_terms();
   return 0;
 }

@@ -27,3 +27,9 @@ def plans(tmp_path_factory):
 @pytest.mark.parametrize("k", [1, 2, 4, 8, 16, 0, -1, 3, 32, 64, 65, 128, 1024, 1028])
 def test_class_kernel_serves_its_block_sizes_only(plans, k):
     assert int(plans[f"cls_wanted_{k}"]) == (k in (1, 2, 4, 8, 16))
+
+
+def test_high_group_is_the_one_the_high_half_pass_applies(plans):
+    """The class kernel skips its own high group when the second pass runs; that pass applies the engine's."""
+    assert int(plans["hi_wanted"]) == 1 and int(plans["high_terms"]) > 0
+    assert int(plans["high_filed_differently"]) == 0
