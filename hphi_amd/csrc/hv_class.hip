@@ -423,10 +423,18 @@ int hphi_cls_wanted(const hphi_engine *e, int k) {
   return e->use_blk && (e->cls == 1 || !(e->bk_tpb || e->bk_wgs_per_cu || e->bk_cpl[slot]));
 }
 
-// Sums bit-equal to the gather kernels': no group holds both kinds of
-// predicate, whose terms stand in another order here.
+// Sums bit-equal to the gather kernels': real couplings (a complex product is
+// three roundings there, two fused steps here), no group with both kinds of
+// predicate, whose terms stand in another order here, and no term filed under
+// mixed here and under low there (a flip within the low half with a mask or
+// sign that reaches into the high one).
 int hphi_cls_same_order(const hphi_engine *e) {
   const ClsArgs &A = e->cls_args;
+  if (!e->c2_realc) return 0;
+  for (int t = 0; t < e->n_low; t++) {
+    const GTerm &x = e->h_terms_dev[t];
+    if ((x.flip | x.tmask | x.sgn) & ~e->irght) return 0;
+  }
   return (A.n_lowp == 0 || A.n_lowp == A.n_low) && (A.n_mixp == 0 || A.n_mixp == A.n_mixed);
 }
 

@@ -33,9 +33,9 @@ static void block_sizes() {
     printf("cls_wanted_%d %d\n", k, hphi_cls_wanted(&e, k));
 }
 
-// terms whose flip leaves the high half: the engine's group against the class
-// layout's, for hops, a density product in the high half and a density-assisted hop
-static void high_terms() {
+// Hubbard ring of 6 sites with hops re + i im and the InterAll entries ia, planned
+static bool ring(double re, double im, const std::vector<int> &ia, const std::vector<double> &iv, hphi_engine &e,
+                 std::vector<char> &up) {
   const int n = 6;
   std::vector<int> idx;
   std::vector<double> t;
@@ -43,17 +43,25 @@ static void high_terms() {
     for (int s = 0; s < 2; s++) {
       const int j = (i + 1) % n, a[8] = {i, s, j, s, j, s, i, s};
       idx.insert(idx.end(), a, a + 8);
-      for (int q = 0; q < 2; q++) t.push_back(1.0), t.push_back(0.0);
+      for (int q = 0; q < 2; q++) t.push_back(re), t.push_back(q ? -im : im);
     }
-  const int ia[] = {4, 0, 4, 0, 5, 1, 5, 1, 5, 0, 5, 0, 0, 0, 1, 0, 1, 0, 0, 0, 5, 0, 5, 0};
-  const double iv[] = {0.7, 0.0, 0.2, 0.1, 0.2, -0.1};
   hphi_model_desc d{};
   d.model = HPHI_MODEL_HUBBARD, d.nsite = n, d.nup = 3, d.ndown = 3;
   d.n_transfer = (int)idx.size() / 4, d.transfer_idx = idx.data(), d.transfer_t = t.data();
-  d.n_interall = 3, d.interall_idx = ia, d.interall_V = iv;
+  d.n_interall = (int)iv.size() / 2, d.interall_idx = ia.data(), d.interall_V = iv.data();
+  return plan(d, e, up);
+}
+static const std::vector<int> NN_HIGH = {4, 0, 4, 0, 5, 1, 5, 1};  // n n on two sites of the high half
+static const std::vector<int> ASSISTED = {5, 0, 5, 0, 0, 0, 1, 0, 1, 0, 0, 0, 5, 0, 5, 0};  // n in the high half, hop in the low one
+
+// terms whose flip leaves the high half: the engine's group against the class
+// layout's, for hops, a density product in the high half and a density-assisted hop
+static void high_terms() {
+  std::vector<int> ia = NN_HIGH;
+  ia.insert(ia.end(), ASSISTED.begin(), ASSISTED.end());
   hphi_engine e;
   std::vector<char> up;
-  if (!plan(d, e, up)) return;
+  if (!ring(1.0, 0.0, ia, {0.7, 0.0, 0.2, 0.1, 0.2, -0.1}, e, up)) return;
   e.hi_split = 1;
   const ClsTerm *T = (const ClsTerm *)up.data();
   int differ = 0, high = 0;
@@ -66,8 +74,20 @@ static void high_terms() {
   printf("hi_wanted %d\nhigh_terms %d\nhigh_filed_differently %d\n", hphi_hi_wanted(&e), high, differ);
 }
 
+// may LOBPCG's H·v, which needs the gather kernels' order of summation, run by classes?
+static void same_order() {
+  std::vector<char> up;
+  hphi_engine real, cplx, nn, assisted;
+  if (ring(1.0, 0.0, {}, {}, real, up)) printf("same_order_real_hops %d\n", hphi_cls_same_order(&real));
+  if (ring(1.0, 0.3, {}, {}, cplx, up)) printf("same_order_complex_hops %d\n", hphi_cls_same_order(&cplx));
+  if (ring(0.0, 0.0, NN_HIGH, {0.7, 0.0}, nn, up)) printf("same_order_nn_high %d\n", hphi_cls_same_order(&nn));
+  if (ring(0.0, 0.0, ASSISTED, {0.2, 0.0, 0.2, 0.0}, assisted, up))
+    printf("same_order_assisted %d\n", hphi_cls_same_order(&assisted));
+}
+
 int main() {
   block_sizes();
   high_terms();
+  same_order();
   return 0;
 }

@@ -33,3 +33,8 @@ def test_high_group_is_the_one_the_high_half_pass_applies(plans):
     """The class kernel skips its own high group when the second pass runs; that pass applies the engine's."""
     assert int(plans["hi_wanted"]) == 1 and int(plans["high_terms"]) > 0
     assert int(plans["high_filed_differently"]) == 0
+
+
+@pytest.mark.parametrize("name,same", [("real_hops", 1), ("complex_hops", 0), ("nn_high", 0), ("assisted", 0)])
+def test_lobpcg_runs_by_classes_only_in_the_gather_order(plans, name, same):
+    assert int(plans[f"same_order_{name}"]) == same
