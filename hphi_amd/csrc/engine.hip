@@ -1445,7 +1445,11 @@ static int wait_prdct(hphi_engine *e, int k, double *prdct) {
 static int hv_call(hphi_engine *e, int k, HvArgs &A, double *prdct) {
   int g = 0;
   (void)hv_path(e, k, &g);
-  if (g * k > HV_HOST_PARTIALS || (k == 1 && hphi_hi_split_on(e))) {
+  // the two-pass H·v (and the build of its tables, which allocates) only where
+  // the launch below would take it: with the engine's own partial sums
+  const int split = k == 1 && A.partial == (double2 *)e->d_partial ? hphi_hi_split_on(e) : 0;
+  if (split < 0) return -1;
+  if (g * k > HV_HOST_PARTIALS || split) {
     if (hv_launch_args(e, k, A, (double2 *)e->hd_prdct)) return -1;
     return wait_prdct(e, k, prdct);
   }
@@ -1489,7 +1493,8 @@ extern "C" int hphi_mltply_block_dev(hphi_engine *e, int k, double *V0, const do
 
 // ------------------------------------------------- allocation-free H·v ----
 // hphi_mltply_block_dev_noalloc keeps the per-workgroup partial sums of prdct
-// in this fixed array rather than in the engine's buffers.  Every device holds its own copy; host code never passes the
+// in this fixed array where they are more than the engine's pinned buffer takes
+// (HV_HOST_PARTIALS).  Every device holds its own copy; host code never passes the
 // array's name to a kernel (on the host it is only a stand-in), but the
 // device address hipGetSymbolAddress returned for that device, recorded
 // once per device when an engine is created there.

@@ -168,13 +168,14 @@ int hphi_mltply_block_dev(hphi_engine *e, int k, double *V0, const double *V1, d
  * bit for bit).  No counterpart in the reference: it is for callers that
  * cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  It calls no hipMalloc/hipFree:
- * the prdct partial sums live in a fixed per-device array of 2^18 + 16
- * complex128 (4 MiB, held until the process ends), so a launch of g
- * workgroups needs g*k <= 2^18 (every default and tuned shape on <= 256 CUs
+ * up to 256 prdct partial sums go to the engine's pinned host buffer, as in
+ * every call; more live in a fixed per-device array of 2^18 complex128 (4 MiB,
+ * held until the process ends), so a launch of g workgroups needs g*k <= 2^18 (every default and tuned shape on <= 256 CUs
  * with <= 64 workgroups per CU); larger launches are rejected with an error.
  * hphi_sz and hphi_diagonalcalc must have run on the engine (no lazy build),
- * and the engine's device must be current.  Calls that overlap on one device
- * share that array and race. */
+ * and the engine's device must be current.  It always runs in one pass
+ * ("hi_split" does not apply).  Calls that overlap on one device share that
+ * array and race. */
 int hphi_mltply_block_dev_noalloc(hphi_engine *e, int k, double *V0, const double *V1, double *prdct);
 
 /* ---- device memory and vector helpers for host drivers ----------------- */
