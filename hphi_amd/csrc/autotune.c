@@ -40,6 +40,7 @@ int hphi_autotune(hphi_engine *e, int k, double *v0, const double *v1, int reps,
                   size_t report_len) {
   if (!e || !v0 || !v1) return hphi_set_error("hphi_autotune: NULL argument");
   if (hphi_block_size_ok("hphi_autotune", k)) return -1;
+  if (hphi_diagonalcalc(e, NULL)) return -1; /* tables and plans: which kernels there are to choose from */
   if (reps < 1) reps = 2;
   cand_t cands[96];
   int n = 0, c2 = 0, blk = 0, lds_ok = 0, crank_ok = 0, gc = 0, cls = 0;

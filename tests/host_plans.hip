@@ -85,7 +85,49 @@ static void same_order() {
     printf("same_order_assisted %d\n", hphi_cls_same_order(&assisted));
 }
 
+// The autotuner's device calls, in place of the library's: building makes the
+// class layout of a fresh engine available, and a timed call costs what `cost` says.
+static void *layout;
+static double (*cost)(const hphi_engine *e, int k);
+extern "C" int hphi_diagonalcalc(hphi_engine *e, double *) {
+  e->d_cls = layout;
+  return 0;
+}
+extern "C" int hphi_time_mltply_dev(hphi_engine *e, int k, double *, const double *, int, int, double *ms) {
+  *ms = cost(e, k);
+  return 0;
+}
+
+static bool has(const char *report, const char *a) { return strstr(report, a) != nullptr; }
+
+// a chain of 20 sites that no call has built yet
+static bool fresh(hphi_engine &e, std::vector<char> &up) {
+  static std::vector<int> ij;
+  static std::vector<double> J;
+  ij.clear(), J.clear();
+  for (int i = 0; i < 20; i++) ij.push_back(i), ij.push_back((i + 1) % 20), J.push_back(1.0);
+  hphi_model_desc d{};
+  d.model = HPHI_MODEL_SPIN, d.nsite = 20, d.nup = 10;
+  d.n_exchange = 20, d.exchange_ij = ij.data(), d.exchange_J = J.data();
+  if (!plan(d, e, up)) return false;
+  layout = e.d_cls;
+  e.d_cls = nullptr;
+  return true;
+}
+
+static void autotune_fresh() {
+  cost = [](const hphi_engine *, int) { return 1.0; };
+  for (int k : {1, 8}) {
+    hphi_engine e;
+    std::vector<char> up, rep(8192);
+    double v = 0;
+    if (fresh(e, up) && hphi_autotune(&e, k, &v, &v, 1, rep.data(), rep.size()) == 0)
+      printf("autotune_fresh_%d %d\n", k, has(rep.data(), "cls"));
+  }
+}
+
 int main() {
+  autotune_fresh();
   block_sizes();
   high_terms();
   same_order();

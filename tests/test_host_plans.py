@@ -38,3 +38,8 @@ def test_high_group_is_the_one_the_high_half_pass_applies(plans):
 @pytest.mark.parametrize("name,same", [("real_hops", 1), ("complex_hops", 0), ("nn_high", 0), ("assisted", 0)])
 def test_lobpcg_runs_by_classes_only_in_the_gather_order(plans, name, same):
     assert int(plans[f"same_order_{name}"]) == same
+
+
+@pytest.mark.parametrize("k", [1, 8])
+def test_autotuner_offers_the_class_kernel_on_a_fresh_engine(plans, k):
+    assert int(plans[f"autotune_fresh_{k}"]) == 1
