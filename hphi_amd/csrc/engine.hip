@@ -1016,11 +1016,26 @@ extern "C" int hphi_engine_info(const hphi_engine *e, uint64_t *dim, uint64_t *s
 
 extern "C" uint64_t hphi_engine_device_bytes(const hphi_engine *e) { return e ? e->bytes : 0; }
 
+// knob name "<stem><k>": the place of k, -1 if it is another knob's name
+static int knob_slot(const std::string &k, const char *stem) {
+  const size_t n = strlen(stem);
+  if (k.compare(0, n, stem) || k.size() == n) return -1;
+  const int slot = hphi_block_slot(atoi(k.c_str() + n));
+  return slot >= 0 && k.substr(n) == std::to_string(1 << slot) ? slot : -1;
+}
+
+// Shapes set by hand, for the autotuner: it puts them back after its sweep, so
+// that the shapes it leaves for one block size take no kernel away from another.
+extern "C" int hphi_tune_hand(const hphi_engine *e) { return e->hand; }
+extern "C" void hphi_tune_hand_restore(hphi_engine *e, int hand) { e->hand = hand; }
+
 extern "C" int hphi_engine_tune(hphi_engine *e, const char *knob, int value) {
   if (!e || !knob) return hphi_set_error("hphi_engine_tune: NULL argument");
   std::string k(knob);
+  const auto by_hand = [&](int bit) { e->hand = value ? e->hand | bit : e->hand & ~bit; };
+  int slot;
   if (k == "tpb" || k == "wgs_per_cu" || k == "lds21" || k == "c2_crank" || k == "c2_unroll" || k == "xcd_map")
-    e->c2_tuned = 1;
+    e->hand |= HAND_C2;
   if (k == "tpb") {
     if (value != 256 && value != 512 && value != 1024) return hphi_set_error("tpb must be 256, 512 or 1024");
     e->c2_tpb = value;
@@ -1066,12 +1081,25 @@ extern "C" int hphi_engine_tune(hphi_engine *e, const char *knob, int value) {
     e->grid_per_cu = value;
   } else if (k == "use_blk") {
     e->use_blk = value ? 1 : 0;
+    for (int &x : e->use_blk_k) x = -2;
+  } else if ((slot = knob_slot(k, "use_blk_k")) >= 1) {
+    if (value < -2 || value > 1 || value == -1) return hphi_set_error("%s must be -2, 0 or 1", knob);
+    e->use_blk_k[slot] = value;
   } else if (k == "cls") {
     if (value < -1 || value > 1) return hphi_set_error("cls must be -1, 0 or 1");
     e->cls = value;
+    for (int &x : e->cls_k) x = -2;
+  } else if ((slot = knob_slot(k, "cls_k")) >= 0) {
+    if (value < -2 || value > 1) return hphi_set_error("%s must be -2, -1, 0 or 1", knob);
+    e->cls_k[slot] = value;
+  } else if ((slot = knob_slot(k, "cls_blocks_k")) >= 0) {
+    if (value != -2 && value != 0 && value != 1 && value != 2 && value != 4)
+      return hphi_set_error("%s must be -2, 0, 1, 2 or 4", knob);
+    e->cls_blocks_k[slot] = value;
   } else if (k == "cls_blocks") {
     if (value != 0 && value != 1 && value != 2 && value != 4) return hphi_set_error("cls_blocks must be 0, 1, 2 or 4");
     e->cls_blocks = value;
+    for (int &x : e->cls_blocks_k) x = -2;
   } else if (k == "cls_order") {
     if (value < -1 || value > 1) return hphi_set_error("cls_order must be -1, 0 or 1");
     e->cls_order = value;
@@ -1081,20 +1109,28 @@ extern "C" int hphi_engine_tune(hphi_engine *e, const char *knob, int value) {
   } else if (k == "gc_tile") {
     if (value < -1 || value > 1) return hphi_set_error("gc_tile must be -1, 0 or 1");
     e->gc_tile = value;
+    for (int &x : e->gc_tile_k) x = -2;
+  } else if ((slot = knob_slot(k, "gc_tile_k")) >= 0) {
+    if (value < -2 || value > 1) return hphi_set_error("%s must be -2, -1, 0 or 1", knob);
+    e->gc_tile_k[slot] = value;
   } else if (k == "lb_mfma") {
     e->lb_mfma = value ? 1 : 0;
   } else if (k == "blk_tpb") {
     if (value != 0 && value != 256 && value != 1024) return hphi_set_error("blk_tpb must be 0, 256 or 1024");
     e->bk_tpb = value;
+    by_hand(HAND_BLK_TPB);
   } else if (k == "blk_wgs_per_cu") {
     if (value < 0 || value > 64) return hphi_set_error("blk_wgs_per_cu out of range");
     e->bk_wgs_per_cu = value;
+    by_hand(HAND_BLK_WGS);
   } else if (k.rfind("blk_cpl", 0) == 0) {
-    int kk = atoi(k.c_str() + 7), slot = kk == 2 ? 0 : kk == 4 ? 1 : kk == 8 ? 2 : kk == 16 ? 3 : -1;
-    if (slot < 0) return hphi_set_error("unknown tuning knob %s", knob);
+    const int kk = atoi(k.c_str() + 7);
+    slot = hphi_block_slot(kk);
+    if (slot < 1) return hphi_set_error("unknown tuning knob %s", knob);
     if (value != 0 && !hphi_blk_cpl_ok(kk, value))
       return hphi_set_error("%s: %d columns per lane not available", knob, value);
-    e->bk_cpl[slot] = value;
+    e->bk_cpl[slot - 1] = value;
+    by_hand(HAND_BLK_CPL(slot));
   } else {
     return hphi_set_error("unknown tuning knob %s", knob);
   }
@@ -1104,6 +1140,7 @@ extern "C" int hphi_engine_tune(hphi_engine *e, const char *knob, int value) {
 extern "C" int hphi_engine_get_tune(const hphi_engine *e, const char *knob, int *value) {
   if (!e || !knob || !value) return hphi_set_error("hphi_engine_get_tune: NULL argument");
   std::string k(knob);
+  int slot, cb, cpl;
   if (k == "tpb") *value = e->c2_tpb;
   else if (k == "wgs_per_cu") *value = e->c2_wgs_per_cu;
   else if (k == "lds21") *value = e->c2_lds21;
@@ -1117,17 +1154,23 @@ extern "C" int hphi_engine_get_tune(const hphi_engine *e, const char *knob, int 
   else if (k == "use_c2") *value = e->use_c2 && e->c2_ok;
   else if (k == "grid_per_cu") *value = e->grid_per_cu;
   else if (k == "use_blk") *value = e->use_blk && hphi_blk_ok(e);
+  else if ((slot = knob_slot(k, "use_blk_k")) >= 1) *value = hphi_use_blk(e, slot) && hphi_blk_ok(e);
   else if (k == "cls") *value = hphi_cls_wanted(e, 1);
-  else if (k == "cls_blocks") *value = hphi_cls_blocks(e);
+  else if ((slot = knob_slot(k, "cls_k")) >= 0) *value = hphi_cls_wanted(e, 1 << slot);
+  else if (k == "cls_blocks" || (slot = knob_slot(k, "cls_blocks_k")) >= 0) {
+    hphi_cls_shape(e, k == "cls_blocks" ? 1 : 1 << slot, &cb, &cpl);
+    *value = cb;
+  }
   else if (k == "cls_order") *value = e->cls_args.groups[0] != nullptr;
   else if (k == "cls_wgs_per_cu") *value = e->cls_wgs_per_cu;
   else if (k == "gc_tile") *value = hphi_gc_wanted(e, 1) || hphi_gc_wanted(e, 2) || hphi_gc_wanted(e, 4) ||
                                     hphi_gc_wanted(e, 8) || hphi_gc_wanted(e, 16);
+  else if ((slot = knob_slot(k, "gc_tile_k")) >= 0) *value = hphi_gc_wanted(e, 1 << slot);
   else if (k == "lb_mfma") *value = e->lb_mfma;
   else if (k == "blk_tpb" || k == "blk_wgs_per_cu" || k.rfind("blk_cpl", 0) == 0) {
     int kk = k.rfind("blk_cpl", 0) == 0 ? atoi(k.c_str() + 7) : 16;
     if (kk != 2 && kk != 4 && kk != 8 && kk != 16) return hphi_set_error("unknown tuning knob %s", knob);
-    int cpl, tpb, wpc;
+    int tpb, wpc;
     hphi_blk_shape(e, kk, &cpl, &tpb, &wpc);
     *value = k == "blk_tpb" ? tpb : k == "blk_wgs_per_cu" ? wpc : cpl;
   } else return hphi_set_error("unknown tuning knob %s", knob);
@@ -1344,7 +1387,7 @@ static int hv_path(const hphi_engine *e, int k, int *grid, int gather = 0) {
     *grid = hphi_gc_partials(e, k);
     return HV_PATH_GC;
   }
-  if (k > 1 && e->use_blk && hphi_blk_ok(e)) {
+  if (hphi_block_slot(k) > 0 && hphi_use_blk(e, hphi_block_slot(k)) && hphi_blk_ok(e)) {
     *grid = hphi_blk_grid(e, k);
     return HV_PATH_BLK;
   }

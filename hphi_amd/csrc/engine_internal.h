@@ -203,6 +203,18 @@ struct GcPlan {
   GcPass pass[GC_MAXPASS];
 };
 
+// launch shapes set by hand: of k_hv_canon; of k_hv_blk for every block size; its
+// columns per lane of one (slot 1..4: k = 2, 4, 8, 16)
+#define HAND_C2 1
+#define HAND_BLK_TPB 2
+#define HAND_BLK_WGS 4
+#define HAND_BLK_CPL(slot) (4 << (slot))
+
+// place of a block size in per-size arrays; -1: no kernel for it
+static inline int hphi_block_slot(int k) {
+  return k == 1 ? 0 : k == 2 ? 1 : k == 4 ? 2 : k == 8 ? 3 : k == 16 ? 4 : -1;
+}
+
 struct hphi_engine {
   int model = 0, nsite = 0, nup = 0, ndown = 0, nbits = 0, nlow = 0;
   uint64_t dim = 0, sdim = 0, size21 = 0, size22 = 0, irght = 0, ilft = 0, ihfbit = 0;
@@ -258,14 +270,23 @@ struct hphi_engine {
   // canonical H·v by classes: -1 unless a shape of k_hv_canon is set, 0 off, 1 on where the sector allows it
   int cls = -1, cls_blocks = 0, cls_order = -1;
   int cls_wgs_per_cu = 256;  // by class: 8x4 J1-J2 77.3 ms at 64, 75.1 at 256; 7x4 3.67, 3.37; no effect below
-  int c2_tuned = 0;  // a shape of k_hv_canon was set by hand
+  // launch shapes set by hand (HAND_*), which keep k_hv_canon or k_hv_blk where the knobs above are -1
+  int hand = 0;
   void *d_cls = nullptr;
   ClsArgs cls_args{};
   // grand-canonical H·v in LDS tiles: -1 by size, 0 off, 1 also with a hand-set block shape
   int gc_tile = -1;
+  // the same for one block size (1, 2, 4, 8, 16), the autotuner's choice; -2: as for the engine
+  int cls_k[5] = {-2, -2, -2, -2, -2}, cls_blocks_k[5] = {-2, -2, -2, -2, -2}, gc_tile_k[5] = {-2, -2, -2, -2, -2};
+  int use_blk_k[5] = {-2, -2, -2, -2, -2};
   GcPlan gc_plan[5];  // block sizes 1, 2, 4, 8, 16
   GcTerm *d_gcterms = nullptr;
 };
+
+// may blocks of the size in this place leave the generic kernel?
+static inline int hphi_use_blk(const hphi_engine *e, int slot) {
+  return e->use_blk_k[slot] != -2 ? e->use_blk_k[slot] : e->use_blk;
+}
 
 extern "C" int hphi_set_error(const char *fmt, ...);
 extern "C" int hphi_block_size_ok(const char *entry, int k);
@@ -304,7 +325,6 @@ int hphi_cls_upload(const hphi_engine *e, ClsArgs &A, char *dev, const void *up,
 void hphi_cls_units(ClsArgs &A, int cb, int rpt);
 int hphi_cls_wanted(const hphi_engine *e, int k);
 int hphi_cls_same_order(const hphi_engine *e);
-int hphi_cls_blocks(const hphi_engine *e);
 int hphi_cls_grid(const hphi_engine *e, int k);
 void hphi_cls_shape(const hphi_engine *e, int k, int *cb, int *cpl);
 int hphi_hv_launch_cls(hphi_engine *e, const HvArgs &H, int k, int g, int skip_high);

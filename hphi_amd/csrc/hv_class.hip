@@ -390,8 +390,7 @@ static bool cls_possible(const hphi_engine *e) {
 // lookup costs more (8.5e5: 43.0, 37.8, 34.4).  Beyond the caches: one, whose rank
 // tiles follow closest on each other in a block (Spin 4.0e7: 3,070, 3,197, 3,527; 6.0e8:
 // 69,733, 72,963 with two; Hubbard 1.7e8: 11,393, 11,407, 11,573).
-int hphi_cls_blocks(const hphi_engine *e) {
-  if (e->cls_blocks > 0) return e->cls_blocks;
+static int cls_blocks(const hphi_engine *e) {
   const uint64_t d = e->dim;
   if (d >= (uint64_t)1 << 24) return 1;
   if (e->model == HPHI_MODEL_HUBBARD) return d < ((uint64_t)1 << 17) ? 1 : d < ((uint64_t)1 << 19) ? 2 : 4;
@@ -406,21 +405,23 @@ int hphi_cls_blocks(const hphi_engine *e) {
 // 13.0, 17.6 us with one, two, four), then two (2.7e6: 1,384, 1,338, 1,364), four
 // beyond the caches (4.0e7, k = 4: 15,032, 14,865, 14,658).
 void hphi_cls_shape(const hphi_engine *e, int k, int *cb, int *cpl) {
-  *cb = hphi_cls_blocks(e);
+  const int slot = hphi_block_slot(k), own = slot < 0 ? -2 : e->cls_blocks_k[slot];
+  const int set = own != -2 ? own : e->cls_blocks;
+  *cb = set > 0 ? set : cls_blocks(e);
   *cpl = 1;
   if (k == 1) return;
   const uint64_t n = e->dim * (uint64_t)k;
-  if (e->cls_blocks == 0) *cb = n < ((uint64_t)1 << 18) ? 1 : e->dim < ((uint64_t)1 << 24) ? 2 : 4;
+  if (set == 0) *cb = n < ((uint64_t)1 << 18) ? 1 : e->dim < ((uint64_t)1 << 24) ? 2 : 4;
   if (e->model == HPHI_MODEL_HUBBARD && n >= ((uint64_t)1 << 18)) *cpl = 2;
 }
 
 // a launch shape of the other kernel for k columns set by hand keeps that kernel
 int hphi_cls_wanted(const hphi_engine *e, int k) {
-  if (!e->d_cls || !e->c2_crank || e->cls == 0) return 0;
-  if (k == 1) return e->use_c2 && (e->cls == 1 || !e->c2_tuned);
-  const int slot = k == 2 ? 0 : k == 4 ? 1 : k == 8 ? 2 : k == 16 ? 3 : -1;
-  if (slot < 0) return 0;
-  return e->use_blk && (e->cls == 1 || !(e->bk_tpb || e->bk_wgs_per_cu || e->bk_cpl[slot]));
+  const int slot = hphi_block_slot(k);
+  if (slot < 0 || !e->d_cls) return 0;
+  const int on = e->cls_k[slot] != -2 ? e->cls_k[slot] : e->cls;
+  if (on == 0 || !(k == 1 ? e->use_c2 : hphi_use_blk(e, slot))) return 0;
+  return on == 1 || !(e->hand & (k == 1 ? HAND_C2 : HAND_BLK_TPB | HAND_BLK_WGS | HAND_BLK_CPL(slot)));
 }
 
 // Sums bit-equal to the gather kernels': real couplings (a complex product is

@@ -399,14 +399,14 @@ static uint32_t gc_pick(const std::vector<GcSrc> &terms, const std::vector<char>
 
 static int gc_kc(int k) { return k >= 4 ? 4 : k; }
 
-static int gc_slot(int k) { return k == 1 ? 0 : k == 2 ? 1 : k == 4 ? 2 : k == 8 ? 3 : k == 16 ? 4 : -1; }
-
 int hphi_gc_wanted(const hphi_engine *e, int k) {
-  const int sl = gc_slot(k);
-  if (sl < 0 || !hphi_model_gc(e->model) || e->gc_tile == 0) return 0;
+  const int sl = hphi_block_slot(k);
+  if (sl < 0 || !hphi_model_gc(e->model)) return 0;
+  const int on = e->gc_tile_k[sl] != -2 ? e->gc_tile_k[sl] : e->gc_tile;
+  if (on == 0) return 0;
   // a block-kernel shape set by hand keeps that kernel
-  if (e->gc_tile < 0 && k > 1 && (e->bk_tpb || e->bk_wgs_per_cu || e->bk_cpl[sl - 1])) return 0;
-  if (k > 1 && !e->use_blk) return 0;
+  if (on < 0 && k > 1 && (e->hand & (HAND_BLK_TPB | HAND_BLK_WGS | HAND_BLK_CPL(sl)))) return 0;
+  if (k > 1 && !hphi_use_blk(e, sl)) return 0;
   return e->gc_plan[sl].npass > 0;
 }
 
@@ -421,7 +421,7 @@ int hphi_gc_plan_build(hphi_engine *e) {
   for (int k = 1; k <= 16; k *= 2) {
     const int kc = gc_kc(k);
     const int s = __builtin_ctz(GC_TPB * GC_E / kc);
-    GcPlan &P = e->gc_plan[gc_slot(k)];
+    GcPlan &P = e->gc_plan[hphi_block_slot(k)];
     P = GcPlan{};
     if (n < s + 3 || (e->gc_tile != 1 && ((uint64_t)1 << (n - s)) * (uint64_t)(k / kc) < GC_MIN_TILES)) continue;
     const int keep = kc == 1 ? 3 : kc == 2 ? 2 : 0;  // runs of 128 bytes, 64 with KC = 4
@@ -540,7 +540,7 @@ int hphi_gc_plan_build(hphi_engine *e) {
 // workgroups of one pass: two per CU (their tiles fill the LDS), whole column
 // groups on every XCD
 static int gc_grid(const hphi_engine *e, int k) {
-  const GcPlan &P = e->gc_plan[gc_slot(k)];
+  const GcPlan &P = e->gc_plan[hphi_block_slot(k)];
   const int ncg = k / gc_kc(k);
   const uint64_t per_xcd = std::max<uint64_t>((((uint64_t)1 << P.pass[0].nob) + 7) / 8, 1) * (uint64_t)ncg;
   const uint64_t want = (uint64_t)std::max(e->num_cu, 8) * 2 / 8;
@@ -548,7 +548,7 @@ static int gc_grid(const hphi_engine *e, int k) {
   return (int)(8 * g);
 }
 
-int hphi_gc_partials(const hphi_engine *e, int k) { return gc_grid(e, k) * e->gc_plan[gc_slot(k)].npass; }
+int hphi_gc_partials(const hphi_engine *e, int k) { return gc_grid(e, k) * e->gc_plan[hphi_block_slot(k)].npass; }
 
 template <int KC>
 static int gc_launch(hphi_engine *e, const GcArgs &G, int g, bool first) {
@@ -571,7 +571,7 @@ static int gc_launch(hphi_engine *e, const GcArgs &G, int g, bool first) {
 
 // every pass in stream order; partials at A.partial[0 .. *grid * k)
 int hphi_hv_launch_gc(hphi_engine *e, const HvArgs &A, int k, int *grid) {
-  const GcPlan &P = e->gc_plan[gc_slot(k)];
+  const GcPlan &P = e->gc_plan[hphi_block_slot(k)];
   const int g = gc_grid(e, k), kc = gc_kc(k);
   for (int p = 0; p < P.npass; p++) {
     const GcPass &Q = P.pass[p];

@@ -125,12 +125,18 @@ int hphi_engine_info(const hphi_engine *e, uint64_t *dim, uint64_t *size21, uint
  *   least 256 tiles, unless a block-kernel knob is set; 1: every sector with 8
  *   tiles, set before the diagonal is built; read back: whether the engine has
  *   tiles in use);
+ *   "cls_k1|2|4|8|16", "cls_blocks_k...", "gc_tile_k...", "use_blk_k2...": the same for calls of one
+ *   block size, -2 as for the engine (the autotuner's choice; setting the
+ *   engine's knob clears them); read back: whether that block size runs so;
  *   LOBPCG: "lb_mfma" 0|1 (block-8 Gram matrices on the FP64 matrix cores). */
 int hphi_engine_tune(hphi_engine *e, const char *knob, int value);
 int hphi_engine_get_tune(const hphi_engine *e, const char *knob, int *value);
 /* Times every candidate launch shape on the caller's device vectors (k = block
- * size; v0 accumulates, re-initialise it afterwards) and keeps the fastest;
- * one line per candidate goes to `report` when non-NULL. */
+ * size; v0 accumulates, re-initialise it afterwards) and keeps the fastest for
+ * that block size, and the fastest shape of the gather kernels for callers that
+ * need their order of summation; other block sizes keep their kernel.  Builds
+ * tables and diagonal on first use.  One line per candidate goes to `report`
+ * when non-NULL. */
 int hphi_autotune(hphi_engine *e, int k, double *v0, const double *v1, int reps, char *report,
                   size_t report_len);
 /* Host only (no device work): dim of the sector and the number of nonzero

@@ -2,6 +2,7 @@
 // line per check for tests/test_host_plans.py.
 #include <cstdio>
 #include <cstring>
+#include <string>
 #include <vector>
 
 #include "engine_internal.h"
@@ -90,7 +91,10 @@ static void same_order() {
 static void *layout;
 static double (*cost)(const hphi_engine *e, int k);
 extern "C" int hphi_diagonalcalc(hphi_engine *e, double *) {
-  e->d_cls = layout;
+  if (hphi_model_gc(e->model))
+    for (GcPlan &P : e->gc_plan) P.npass = 1;
+  else
+    e->d_cls = layout;
   return 0;
 }
 extern "C" int hphi_time_mltply_dev(hphi_engine *e, int k, double *, const double *, int, int, double *ms) {
@@ -126,8 +130,80 @@ static void autotune_fresh() {
   }
 }
 
+static int knob(const hphi_engine *e, const char *name, int k) {
+  int v = -1;
+  if (hphi_engine_get_tune(e, (std::string(name) + "_k" + std::to_string(k)).c_str(), &v)) hphi_engine_get_tune(e, name, &v);
+  return v;
+}
+static bool generic(const hphi_engine *e, int k) { return !(k == 1 ? e->use_c2 : knob(e, "use_blk", k)); }
+
+// "<name> <class kernel or tiles in use>,<blocks per wave or 0>..." for k = 1, 2, 4, 8, 16
+static void state(const char *name, const hphi_engine &e) {
+  printf("%s", name);
+  for (int k = 1; k <= 16; k *= 2) {
+    int cb = 0, cpl = 0;
+    if (!hphi_model_gc(e.model)) hphi_cls_shape(&e, k, &cb, &cpl);
+    printf(" %d,%d", hphi_cls_wanted(&e, k) || hphi_gc_wanted(&e, k), cb);
+  }
+  printf("\n");
+}
+
+// what the autotuner leaves for every block size, by who wins the sweep for one of them
+static void autotune_sizes() {
+  struct Run {
+    const char *name;
+    int k;
+    double (*cost)(const hphi_engine *e, int k);
+  };
+  const Run spin[] = {
+      {"tuned_none", 0, nullptr},
+      {"tuned_1_canon", 1, [](const hphi_engine *e, int k) { return hphi_cls_wanted(e, k) ? 2.0 : generic(e, k) ? 3.0 : 1.0; }},
+      {"tuned_1_lds", 1, [](const hphi_engine *e, int k) { return hphi_cls_wanted(e, k) || generic(e, k) ? 2.0 : 1.0 + e->c2_crank; }},
+      {"tuned_1_class4", 1, [](const hphi_engine *e, int k) {
+         int cb, cpl;
+         hphi_cls_shape(e, k, &cb, &cpl);
+         return hphi_cls_wanted(e, k) && cb == 4 ? 1.0 : e->c2_tpb == 512 ? 2.0 : 3.0;
+       }},
+      {"tuned_1_generic", 1, [](const hphi_engine *e, int k) { return generic(e, k) ? 1.0 : 2.0; }},
+      {"tuned_8_block", 8, [](const hphi_engine *e, int k) { return hphi_cls_wanted(e, k) || generic(e, k) ? 2.0 : 1.0; }},
+      {"tuned_8_generic", 8, [](const hphi_engine *e, int k) { return generic(e, k) ? 1.0 : 2.0; }}};
+  double v = 0;
+  for (const Run &r : spin) {
+    hphi_engine e;
+    std::vector<char> up;
+    if (!fresh(e, up)) return;
+    hphi_diagonalcalc(&e, nullptr);
+    cost = r.cost;
+    if (r.k && hphi_autotune(&e, r.k, &v, &v, 1, nullptr, 0)) continue;
+    state(r.name, e);
+    if (!strcmp(r.name, "tuned_1_class4")) printf("tuned_1_class4_tpb %d\n", e.c2_tpb);  // under it: the best gather shape
+  }
+  const Run gc[] = {
+      {"gc_none", 0, nullptr},
+      {"gc_1_generic", 1, [](const hphi_engine *e, int k) { return hphi_gc_wanted(e, k) ? 2.0 : 1.0; }},
+      {"gc_2_block", 2, [](const hphi_engine *e, int k) { return hphi_gc_wanted(e, k) || generic(e, k) ? 2.0 : 1.0; }},
+      {"gc_8_generic", 8, [](const hphi_engine *e, int k) { return generic(e, k) ? 1.0 : 2.0; }}};
+  for (const Run &r : gc) {
+    hphi_engine e;
+    e.model = HPHI_MODEL_SPINGC;
+    hphi_diagonalcalc(&e, nullptr);
+    cost = r.cost;
+    if (r.k && hphi_autotune(&e, r.k, &v, &v, 1, nullptr, 0)) continue;
+    state(r.name, e);
+  }
+  // a shape set by hand stays one
+  hphi_engine e;
+  std::vector<char> up;
+  if (!fresh(e, up)) return;
+  hphi_diagonalcalc(&e, nullptr);
+  hphi_engine_tune(&e, "blk_tpb", 256);
+  cost = [](const hphi_engine *, int) { return 1.0; };
+  if (!hphi_autotune(&e, 1, &v, &v, 1, nullptr, 0)) state("tuned_1_by_hand", e);
+}
+
 int main() {
   autotune_fresh();
+  autotune_sizes();
   block_sizes();
   high_terms();
   same_order();

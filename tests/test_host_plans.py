@@ -43,3 +43,28 @@ def test_lobpcg_runs_by_classes_only_in_the_gather_order(plans, name, same):
 @pytest.mark.parametrize("k", [1, 8])
 def test_autotuner_offers_the_class_kernel_on_a_fresh_engine(plans, k):
     assert int(plans[f"autotune_fresh_{k}"]) == 1
+
+
+@pytest.mark.parametrize("run,k,on", [("tuned_1_canon", 1, 0), ("tuned_1_lds", 1, 0), ("tuned_1_class4", 1, 1),
+                                      ("tuned_1_generic", 1, 0), ("tuned_8_block", 8, 0), ("tuned_8_generic", 8, 0),
+                                      ("gc_1_generic", 1, 0), ("gc_2_block", 2, 0), ("gc_8_generic", 8, 0)])
+def test_autotuning_one_block_size_leaves_the_others(plans, run, k, on):
+    """Whichever kernel wins for k columns, the other block sizes keep theirs and their shape."""
+    before, after = plans[run.split("_")[0] + "_none"].split(), plans[run].split()
+    assert len(before) == len(after) == 5
+    for i in range(5):
+        if 1 << i == k:
+            assert after[i].startswith(f"{on},")
+        else:
+            assert after[i] == before[i] and before[i].startswith("1,")
+
+
+def test_autotuning_leaves_the_best_gather_shape_under_the_class_kernel(plans):
+    assert plans["tuned_1_class4"].split()[0] == "1,4"
+    assert int(plans["tuned_1_class4_tpb"]) == 512
+
+
+def test_shapes_set_by_hand_stay_so(plans):
+    """k = 1 is the class kernel's; a workgroup size of the block kernel set by hand keeps that kernel for blocks."""
+    got = [x.split(",")[0] for x in plans["tuned_1_by_hand"].split()]
+    assert got == ["1", "0", "0", "0", "0"]
