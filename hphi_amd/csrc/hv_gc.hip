@@ -529,9 +529,12 @@ int hphi_gc_plan_build(hphi_engine *e) {
     for (GcPlan &P : e->gc_plan) P.npass = 0;
     return 0;
   }
-  (void)hipFree(e->d_gcterms);
-  e->d_gcterms = nullptr;
-  HIPCHK(hipMalloc(&e->d_gcterms, sizeof(GcTerm) * all.size()));
+  if (hipMalloc((void **)&e->d_gcterms, sizeof(GcTerm) * all.size()) != hipSuccess) {
+    (void)hipGetLastError();
+    e->d_gcterms = nullptr;
+    for (GcPlan &P : e->gc_plan) P.npass = 0;  // no room: the gather kernels serve this engine
+    return 0;
+  }
   HIPCHK(hipMemcpy(e->d_gcterms, all.data(), sizeof(GcTerm) * all.size(), hipMemcpyHostToDevice));
   e->bytes += sizeof(GcTerm) * all.size();
   return 0;

@@ -201,7 +201,24 @@ static void autotune_sizes() {
   if (!hphi_autotune(&e, 1, &v, &v, 1, nullptr, 0)) state("tuned_1_by_hand", e);
 }
 
+// a device without room: hipMalloc fails in here
+extern "C" hipError_t hipMalloc(void **, size_t) { return hipErrorOutOfMemory; }
+
+static void tiles_without_memory() {
+  std::vector<int> ij;
+  std::vector<double> J(20, 1.0);
+  for (int i = 0; i < 20; i++) ij.push_back(i), ij.push_back((i + 1) % 20);
+  hphi_model_desc d{};
+  d.model = HPHI_MODEL_SPINGC, d.nsite = 20;
+  d.n_exchange = 20, d.exchange_ij = ij.data(), d.exchange_J = J.data();
+  hphi_engine e;
+  if (hphi_engine_prepare(&d, &e)) return;
+  const int rc = hphi_gc_plan_build(&e);
+  printf("tiles_without_memory %d %d\n", rc, hphi_gc_wanted(&e, 1) || hphi_gc_wanted(&e, 16));
+}
+
 int main() {
+  tiles_without_memory();
   autotune_fresh();
   autotune_sizes();
   block_sizes();

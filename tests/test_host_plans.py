@@ -68,3 +68,8 @@ def test_shapes_set_by_hand_stay_so(plans):
     """k = 1 is the class kernel's; a workgroup size of the block kernel set by hand keeps that kernel for blocks."""
     got = [x.split(",")[0] for x in plans["tuned_1_by_hand"].split()]
     assert got == ["1", "0", "0", "0", "0"]
+
+
+def test_tiles_without_room_for_their_terms_leave_the_gather_kernels(plans):
+    """Neither an error nor tiles."""
+    assert plans["tiles_without_memory"].split() == ["0", "0"]
