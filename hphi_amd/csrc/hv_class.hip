@@ -415,13 +415,47 @@ void hphi_cls_shape(const hphi_engine *e, int k, int *cb, int *cpl) {
   if (e->model == HPHI_MODEL_HUBBARD && n >= ((uint64_t)1 << 18)) *cpl = 2;
 }
 
+// Where the gather kernels are as fast or faster, by two things.
+//
+// Row offsets: one KB of LDS per low-half flip of the mixed terms.  Exchange and
+// hops have 16 at most; four-orbital InterAll entries of 16 Hubbard sites up to 72.
+// Up to 26, four workgroups share a CU; up to 36, three, which pays where the tiles
+// are full; beyond, two.  Microseconds, k_hv_canon / this kernel for k = 1, k_hv_blk /
+// this one for k = 8:
+//   16 sites, 4 + 4 electrons (3.3e6)   24 flips 299 / 207, 1370 / 1029; 36 378 / 314, 1679 / 1449;
+//                                       40 406 / 465, 1782 / 2036
+//   14 sites, 7 + 7 (1.2e7)             36 1411 / 868, 6389 / 5092; 40 1510 / 1221, 6794 / 7075
+//   13 sites, 4 + 4 (5.1e5, fill 0.70)  34 91 / 101, 274 / 330
+//
+// Fill of the tiles: a class of few ranks leaves lanes of its tiles idle.  Below 2^17
+// states the device has room for the idle ones, from 2^19 on no sector is that
+// dilute; between them (k = 1 unless noted):
+//   Spin of 30, 32 sites, 5 up (fill 0.34, 0.35)     23.4 / 25.5, 27.3 / 30.3; k = 2 32.6 / 27.8
+//   24, 28 sites, 6 up (fill 0.49, 0.53)             19.9 / 17.5, 35.9 / 32.7
+//   Hubbard 16 sites, 3 + 3 (0.42)                   26.1 / 28.7; k = 2 31.7 / 44.4, k = 4 93 / 75
+//   Hubbard 7x2, 3 + 4 (0.55)                        33.2 / 38.1
+//   Hubbard 16 sites, 2 + 5 (0.61)                   41.0 / 35.4; k = 2 50.3 / 48.4
+//   Hubbard 5x3, 3 + 3 (0.41), k = 4                 57.5 / 67.0; 143,325 states (0.44) 49.1 / 42.3
+static bool cls_pays(const hphi_engine *e, int k) {
+  const ClsArgs &A = e->cls_args;
+  if (A.nlo > 36) return false;
+  const bool hub = e->model == HPHI_MODEL_HUBBARD;
+  if (A.nlo <= 26 && (e->dim < (uint64_t)1 << 17 || e->dim >= (uint64_t)1 << 19 || k > (hub ? 4 : 1))) return true;
+  uint64_t lanes = 0;
+  for (int c = 0; c < A.ncls; c++) lanes += (uint64_t)A.nblk[c] * ((A.size[c] + 63) / 64 * 64);
+  const double fill = (double)e->dim / (double)lanes;
+  if (A.nlo > 26) return fill >= 0.75;
+  if (k == 4) return fill >= 0.45 || e->dim < (uint64_t)3 << 16 || e->dim >= (uint64_t)1 << 18;
+  return fill >= (hub ? 0.56 : 0.45);
+}
+
 // a launch shape of the other kernel for k columns set by hand keeps that kernel
 int hphi_cls_wanted(const hphi_engine *e, int k) {
   const int slot = hphi_block_slot(k);
   if (slot < 0 || !e->d_cls) return 0;
   const int on = e->cls_k[slot] != -2 ? e->cls_k[slot] : e->cls;
   if (on == 0 || !(k == 1 ? e->use_c2 : hphi_use_blk(e, slot))) return 0;
-  return on == 1 || !(e->hand & (k == 1 ? HAND_C2 : HAND_BLK_TPB | HAND_BLK_WGS | HAND_BLK_CPL(slot)));
+  return on == 1 || (cls_pays(e, k) && !(e->hand & (k == 1 ? HAND_C2 : HAND_BLK_TPB | HAND_BLK_WGS | HAND_BLK_CPL(slot))));
 }
 
 // Sums bit-equal to the gather kernels': real couplings (a complex product is

@@ -115,7 +115,7 @@ int hphi_engine_info(const hphi_engine *e, uint64_t *dim, uint64_t *size21, uint
  *   "hi_p1_wgs_per_cu" 1..256 (first pass), "hi_fuse_copy" 0|1;
  *   block kernel (k > 1): "use_blk" 0|1, "blk_cpl2|4|8|16" columns per lane
  *   (1, 4 or k; 0 = default), "blk_tpb" 0|256|1024, "blk_wgs_per_cu" 0..64;
- *   canonical H·v by classes: "cls" -1|0|1 (-1: unless one of tpb, wgs_per_cu,
+ *   canonical H·v by classes: "cls" -1|0|1 (-1: where it is the faster one, unless one of tpb, wgs_per_cu,
  *   lds21, c2_crank, c2_unroll or xcd_map is set, for k > 1 one of blk_tpb,
  *   blk_wgs_per_cu or blk_cpl of this k; read back: whether it is in use for
  *   k = 1), "cls_blocks" 0|1|2|4 (blocks per wave, 0 by size), "cls_wgs_per_cu" 1..256,

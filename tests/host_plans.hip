@@ -86,6 +86,58 @@ static void same_order() {
     printf("same_order_assisted %d\n", hphi_cls_same_order(&assisted));
 }
 
+// Which kernel by default: a J1-J2 ring, and a Hubbard chain with `pairs` InterAll
+// entries that move two electrons, one within each half
+static void by_default(const char *name, hphi_model_desc &d) {
+  hphi_engine e;
+  std::vector<char> up;
+  if (!plan(d, e, up)) return;
+  printf("default_%s", name);
+  for (int k = 1; k <= 16; k *= 2) printf(" %d", hphi_cls_wanted(&e, k));
+  e.cls = 1;
+  printf(" %d %d\n", hphi_cls_wanted(&e, 1), e.cls_args.nlo);
+}
+static void ring_default(int n, int nup) {
+  std::vector<int> ij;
+  for (int q = 1; q <= 2; q++)
+    for (int i = 0; i < n; i++) ij.push_back(i), ij.push_back((i + q) % n);
+  std::vector<double> J(2 * n, 1.0);
+  hphi_model_desc d{};
+  d.model = HPHI_MODEL_SPIN, d.nsite = n, d.nup = nup;
+  d.n_exchange = 2 * n, d.exchange_ij = ij.data(), d.exchange_J = J.data();
+  by_default(("spin_" + std::to_string(n) + "_" + std::to_string(nup)).c_str(), d);
+}
+static void hubbard_default(int n, int u, int w, int pairs) {
+  std::vector<int> idx, ia;
+  std::vector<double> t, iv;
+  for (int i = 0; i < n; i++)
+    for (int s = 0; s < 2; s++) {
+      const int j = (i + 1) % n, a[8] = {i, s, j, s, j, s, i, s};
+      idx.insert(idx.end(), a, a + 8);
+      t.insert(t.end(), {1.0, 0.0, 1.0, 0.0});
+    }
+  for (int s = 0; s < 2; s++)
+    for (int i = 0; i < n / 2; i++)
+      for (int j = i + 1; j < n / 2 && pairs > 0; j++, pairs--) {
+        const int k = n / 2 + i, l = n / 2 + j, a[16] = {i, s, j, s, k, s, l, s, l, s, k, s, j, s, i, s};
+        ia.insert(ia.end(), a, a + 16);
+        iv.insert(iv.end(), {0.1, 0.0, 0.1, 0.0});
+      }
+  hphi_model_desc d{};
+  d.model = HPHI_MODEL_HUBBARD, d.nsite = n, d.nup = u, d.ndown = w;
+  d.n_transfer = (int)idx.size() / 4, d.transfer_idx = idx.data(), d.transfer_t = t.data();
+  d.n_interall = (int)iv.size() / 2, d.interall_idx = ia.data(), d.interall_V = iv.data();
+  by_default(("hubbard_" + std::to_string(n) + "_" + std::to_string(u) + "_" + std::to_string(w) + "_" +
+              std::to_string(iv.size() / 4)).c_str(), d);
+}
+static void defaults() {
+  ring_default(20, 2), ring_default(28, 5), ring_default(30, 5), ring_default(32, 27), ring_default(24, 6);
+  ring_default(32, 6), ring_default(24, 12);
+  hubbard_default(8, 1, 1, 0), hubbard_default(14, 3, 3, 0), hubbard_default(16, 3, 3, 0), hubbard_default(15, 3, 3, 0);
+  hubbard_default(16, 2, 5, 0), hubbard_default(12, 6, 6, 0), hubbard_default(12, 6, 6, 30), hubbard_default(16, 4, 4, 20);
+  hubbard_default(16, 4, 4, 32), hubbard_default(16, 4, 4, 36), hubbard_default(12, 3, 3, 30);
+}
+
 // The autotuner's device calls, in place of the library's: building makes the
 // class layout of a fresh engine available, and a timed call costs what `cost` says.
 static void *layout;
@@ -218,6 +270,7 @@ static void tiles_without_memory() {
 }
 
 int main() {
+  defaults();
   tiles_without_memory();
   autotune_fresh();
   autotune_sizes();

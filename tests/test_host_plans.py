@@ -73,3 +73,24 @@ def test_shapes_set_by_hand_stay_so(plans):
 def test_tiles_without_room_for_their_terms_leave_the_gather_kernels(plans):
     """Neither an error nor tiles."""
     assert plans["tiles_without_memory"].split() == ["0", "0"]
+
+
+# k = 1, 2, 4, 8, 16: by classes or not; forced for k = 1; at most this many low-half flips
+DEFAULTS = {
+    "spin_20_2": "1 1 1 1 1", "spin_24_12": "1 1 1 1 1", "spin_24_6": "1 1 1 1 1", "spin_32_6": "1 1 1 1 1",
+    "spin_28_5": "1 1 1 1 1",                                  # as dilute, but fewer than 2^17 states
+    "spin_30_5": "0 1 1 1 1", "spin_32_27": "0 1 1 1 1",       # dilute: single columns
+    "hubbard_8_1_1_0": "1 1 1 1 1", "hubbard_12_6_6_0": "1 1 1 1 1", "hubbard_16_2_5_0": "1 1 1 1 1",
+    "hubbard_14_3_3_0": "0 0 1 1 1", "hubbard_16_3_3_0": "0 0 1 1 1",
+    "hubbard_15_3_3_0": "0 0 0 1 1",
+    "hubbard_12_6_6_30": "1 1 1 1 1", "hubbard_16_4_4_20": "1 1 1 1 1", "hubbard_16_4_4_32": "1 1 1 1 1",
+    "hubbard_12_3_3_30": "0 0 0 0 0",                          # three workgroups per CU, dilute
+    "hubbard_16_4_4_36": "0 0 0 0 0",                          # two workgroups per CU
+}
+
+
+@pytest.mark.parametrize("name", DEFAULTS)
+def test_default_kernel_of_canonical_sectors(plans, name):
+    *wanted, forced, nlo = plans["default_" + name].split()
+    assert " ".join(wanted) == DEFAULTS[name], nlo
+    assert forced == "1"
