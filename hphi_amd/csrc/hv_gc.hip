@@ -391,10 +391,10 @@ static uint32_t gc_pick(const std::vector<GcSrc> &terms, const std::vector<char>
 }
 
 // Which grand-canonical engines take this path: 32-bit states, two-bit parity
-// predicates, and tiles enough to fill the device, two per CU.  Per H·v, block
+// predicates, and tiles enough to give every CU one.  Per H·v, block
 // kernel / tiles: 64 tiles (9x2 strip, k = 1) 32.3 / 31.9 us, 128 (9x2, k = 2)
 // 48.9 / 47.1 and (HubbardGC 9, k = 2) 28.6 / 37.6, 256 (9x2, k = 4) 72 / 60 and
-// (HubbardGC 9, k = 4) 44.1 / 44.4, 256 (10x2, k = 1) 115 / 57.
+// (HubbardGC 9, k = 4) 44.1 / 44.4, 256 (10x2, k = 1) 115 / 57.  gc_pays says which of them.
 #define GC_MIN_TILES 256
 
 static int gc_kc(int k) { return k >= 4 ? 4 : k; }
@@ -410,6 +410,37 @@ int hphi_gc_wanted(const hphi_engine *e, int k) {
   return e->gc_plan[sl].npass > 0;
 }
 
+// Where the tiles are the faster ones, by default, among sectors with tiles
+// enough.  W: the gathers an amplitude needs in the block kernel, wrem: those
+// the first pass still makes.  Two things cost what the tiles save; per H·v,
+// block kernel / tiles:
+//  * terms of no case of gc_parity (a test per element) and gathered ones.  With
+//    fewer than 512 tiles, one per workgroup, up to 0.3 of the terms (a ring of 18
+//    sites, k = 4, with 10 InterAll pairs, 0.53: 58 / 71 us; 20 sites, k = 1, 5 pairs,
+//    0.33: 57 / 60; HubbardGC 10, k = 1, 0.05: 50 / 48); with more, k = 2 two thirds (20
+//    sites, 0.88: 202 / 215, 0.68: 111 / 111; HubbardGC 11, 0.69: 318 / 330), k = 4 half, and a
+//    quarter where there are three passes (21 sites, 0.78: 431 / 458; HubbardGC 11, 0.67: 585 / 667,
+//    three passes at 0.35: 689 / 799; 20 sites, 0.50: 163 / 149); any share for k = 1
+//    (22 sites, 0.67: 294 / 209) and for k >= 8, where the block kernel's rows no
+//    longer share cache lines (20 sites, 0.92: 1897 / 1169).
+//  * blocks of 512 MB on, k >= 8, with few terms, of which some are gathered:
+//    HubbardGC 11 (W 11, wrem 2) k = 16 1937 / 2247, a ring of 24 sites (12, 3) k = 8
+//    3885 / 4542; HubbardGC 11 with 20 more pairs (13, 4) k = 16 3594 / 3120; the ring of
+//    25 in three passes (12.5, 0) k = 8 9406 / 8958; HubbardGC 10 (10, 0, 256 MB) 487 / 434.
+static bool gc_pays(const hphi_engine *e, int k, const GcPlan &P, double W, double wrem) {
+  int fast = 0, slow = 0;
+  for (int q = 0; q < P.npass; q++) {
+    fast += P.pass[q].nloc - P.pass[q].nother;
+    slow += P.pass[q].nother + P.pass[q].nrem;
+  }
+  const double share = (double)slow / std::max(fast + slow, 1);
+  const uint64_t tiles = ((uint64_t)1 << P.pass[0].nob) * (uint64_t)(k / gc_kc(k));
+  if (k <= 4 && tiles < 512) return share <= 0.3;
+  if (k == 2) return share <= 2.0 / 3.0;
+  if (k == 4) return share <= (P.npass >= 3 ? 0.25 : 0.5);
+  return k < 8 || e->dim * (uint64_t)k < (uint64_t)1 << 25 || W >= 13.0 || wrem < 2.0;
+}
+
 // The passes of every block size, and their term tables on the device; called
 // once the engine's diagonal is built, so that launches allocate nothing.
 int hphi_gc_plan_build(hphi_engine *e) {
@@ -418,6 +449,8 @@ int hphi_gc_plan_build(hphi_engine *e) {
   if (!gc_sources(e, terms)) return 0;
   const int n = e->nbits, nt = (int)terms.size();
   std::vector<GcTerm> all;
+  double W = 0.0;
+  for (const GcSrc &t : terms) W += gc_weight(t) / GC_COST_GATHER;
   for (int k = 1; k <= 16; k *= 2) {
     const int kc = gc_kc(k);
     const int s = __builtin_ctz(GC_TPB * GC_E / kc);
@@ -438,7 +471,10 @@ int hphi_gc_plan_build(hphi_engine *e) {
     // a term that several passes cover goes to the one with the fewest terms
     // (the first pass also gathers and reads the diagonal: it counts those)
     int nrem = 0;
-    for (int t = 0; t < nt; t++) nrem += open[t];
+    double wrem = 0.0;
+    for (int t = 0; t < nt; t++)
+      if (open[t]) nrem++, wrem += gc_weight(terms[t]) / GC_COST_GATHER;
+    const size_t first = all.size();
     std::vector<int> pass(nt, -1);
     int load[GC_MAXPASS] = {4 * nrem + 4};
     for (int many = 0; many < 2; many++)
@@ -513,6 +549,10 @@ int hphi_gc_plan_build(hphi_engine *e) {
           }
         Q.nrem = nrem;
       }
+    }
+    if (e->gc_tile != 1 && !gc_pays(e, k, P, W, wrem)) {
+      P = GcPlan{};
+      all.resize(first);
     }
   }
   for (GcTerm &g : all) {

@@ -121,8 +121,8 @@ int hphi_engine_info(const hphi_engine *e, uint64_t *dim, uint64_t *size21, uint
  *   k = 1), "cls_blocks" 0|1|2|4 (blocks per wave, 0 by size), "cls_wgs_per_cu" 1..256,
  *   "cls_order" -1|0|1 (units by class, or by index dealt to the XCDs one by one; -1:
  *   by index from 2^24 states on; set before the tables are built);
- *   grand-canonical H·v in LDS tiles: "gc_tile" -1|0|1 (-1: sectors of at
- *   least 256 tiles, unless a block-kernel knob is set; 1: every sector with 8
+ *   grand-canonical H·v in LDS tiles: "gc_tile" -1|0|1 (-1: where they are the
+ *   faster ones, from 256 tiles on, unless a block-kernel knob is set; 1: every sector with 8
  *   tiles, set before the diagonal is built; read back: whether the engine has
  *   tiles in use);
  *   "cls_k1|2|4|8|16", "cls_blocks_k...", "gc_tile_k...", "use_blk_k2...": the same for calls of one

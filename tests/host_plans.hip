@@ -1,6 +1,7 @@
 // Host-side plans of the H·v kernels, without a device: prints one "name value"
 // line per check for tests/test_host_plans.py.
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <string>
 #include <vector>
@@ -253,8 +254,16 @@ static void autotune_sizes() {
   if (!hphi_autotune(&e, 1, &v, &v, 1, nullptr, 0)) state("tuned_1_by_hand", e);
 }
 
-// a device without room: hipMalloc fails in here
-extern "C" hipError_t hipMalloc(void **, size_t) { return hipErrorOutOfMemory; }
+// device memory, with room or without
+static bool room = false;
+extern "C" hipError_t hipMalloc(void **p, size_t n) {
+  *p = room ? malloc(n) : nullptr;
+  return *p ? hipSuccess : hipErrorOutOfMemory;
+}
+extern "C" hipError_t hipMemcpy(void *to, const void *from, size_t n, hipMemcpyKind) {
+  memcpy(to, from, n);
+  return hipSuccess;
+}
 
 static void tiles_without_memory() {
   std::vector<int> ij;
@@ -269,7 +278,51 @@ static void tiles_without_memory() {
   printf("tiles_without_memory %d %d\n", rc, hphi_gc_wanted(&e, 1) || hphi_gc_wanted(&e, 16));
 }
 
+// Which block sizes of a grand-canonical ring run in tiles by default: SpinGC with
+// bonds to `far` neighbours and `pairs` InterAll terms, a projector times a flip; HubbardGC with hops
+static void gc_default(const char *name, int n, int far, int pairs, bool hubbard) {
+  std::vector<int> ij, ia, idx;
+  std::vector<double> J, iv, t;
+  for (int q = 1; q <= far; q++)
+    for (int i = 0; i < n; i++) ij.push_back(i), ij.push_back((i + q) % n), J.push_back(1.0 / q);
+  for (int q = 0; q < pairs; q++) {
+    const int a = q % n, b = (q + 1 + q / n) % n;
+    const int e[16] = {a, 1, a, 0, b, 1, b, 1, b, 1, b, 1, a, 0, a, 1};
+    ia.insert(ia.end(), e, e + 16);
+    iv.insert(iv.end(), {0.1, 0.05, 0.1, -0.05});
+  }
+  for (int i = 0; i < n && hubbard; i++)
+    for (int s = 0; s < 2; s++) {
+      const int j = (i + 1) % n, a[8] = {i, s, j, s, j, s, i, s};
+      idx.insert(idx.end(), a, a + 8);
+      t.insert(t.end(), {1.0, 0.0, 1.0, 0.0});
+    }
+  hphi_model_desc d{};
+  d.model = hubbard ? HPHI_MODEL_HUBBARDGC : HPHI_MODEL_SPINGC, d.nsite = n;
+  d.n_exchange = hubbard ? 0 : (int)J.size(), d.exchange_ij = ij.data(), d.exchange_J = J.data();
+  d.n_interall = (int)iv.size() / 2, d.interall_idx = ia.data(), d.interall_V = iv.data();
+  d.n_transfer = (int)idx.size() / 4, d.transfer_idx = idx.data(), d.transfer_t = t.data();
+  printf("gc_%s", name);
+  for (int forced = 0; forced < 2; forced++) {
+    hphi_engine e;
+    if (hphi_engine_prepare(&d, &e)) break;
+    if (forced) e.gc_tile = 1;
+    room = true;
+    hphi_gc_plan_build(&e);
+    room = false;
+    for (int k = 1; k <= 16; k *= 2) printf(" %d", hphi_gc_wanted(&e, k));
+    free(e.d_gcterms);
+  }
+  printf("\n");
+}
+static void gc_defaults() {
+  gc_default("j1j2_18", 18, 2, 0, false), gc_default("j1j2_22", 22, 2, 0, false), gc_default("ring_24", 24, 1, 0, false);
+  gc_default("pairs_18", 18, 1, 10, false), gc_default("pairs_20", 20, 1, 30, false), gc_default("pairs_22", 22, 1, 30, false);
+  gc_default("hubbard_10", 10, 0, 0, true), gc_default("hubbard_11", 11, 0, 0, true);
+}
+
 int main() {
+  gc_defaults();
   defaults();
   tiles_without_memory();
   autotune_fresh();

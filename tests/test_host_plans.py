@@ -94,3 +94,20 @@ def test_default_kernel_of_canonical_sectors(plans, name):
     *wanted, forced, nlo = plans["default_" + name].split()
     assert " ".join(wanted) == DEFAULTS[name], nlo
     assert forced == "1"
+
+
+# k = 1, 2, 4, 8, 16: in tiles or not
+GC_DEFAULTS = {
+    "j1j2_18": "0 0 1 1 1", "j1j2_22": "1 1 1 1 1", "hubbard_10": "1 1 1 1 1",
+    "pairs_18": "0 0 0 1 1",    # 256 tiles for k = 4, half of the terms of no case
+    "pairs_20": "0 0 0 1 1",    # three quarters
+    "pairs_22": "1 0 0 1 1",    # the same, 1,024 tiles for k = 1
+    "ring_24": "1 1 1 0 0", "hubbard_11": "1 1 1 0 0",  # few terms, blocks of 512 MB
+}
+
+
+@pytest.mark.parametrize("name", GC_DEFAULTS)
+def test_default_kernel_of_grand_canonical_sectors(plans, name):
+    got = plans["gc_" + name].split()
+    assert " ".join(got[:5]) == GC_DEFAULTS[name]
+    assert all(f >= w for w, f in zip(got[:5], got[5:])) and "1" in got[5:]
