@@ -810,7 +810,7 @@ def main():
             "speedup_vs_sequential": round(p0["solves_per_s"] / sv["sequential_solves_per_s"], 3),
             "rate_per_s": 120.0, "p50_s": round(p1["p50_s"], 3), "p99_s": round(p1["p99_s"], 3),
             "converged": [p0["converged"], p1["converged"]],
-            "slab_hv": {"kernel": "k_sl_cls", "achieved_gbs": p0["hv_gbs"], "frac": p0["hv_frac"],
+            "slab_hv": {"kernel": "k_sl_hv", "achieved_gbs": p0["hv_gbs"], "frac": p0["hv_frac"],
                         "launches": p0["hv_launches"],
                         "note": "algorithmic bytes (per slab 8 dim, per running column 56 dim + 16 per "
                                 "off-diagonal element) over HIP-event time of the slab H·v launches"},

@@ -32,7 +32,8 @@ EXPORTED = [
     "hphi_read_def", "hphi_model_desc_free", "hphi_tridiag_lowest",
     "hphi_lanczos_good_eigenvalues", "hphi_lanczos_converged",
     "hphi_server_create", "hphi_server_destroy", "hphi_server_submit", "hphi_server_tick",
-    "hphi_server_results", "hphi_server_now", "hphi_server_stats", "hphi_lobpcg", "hphi_herm_eig",
+    "hphi_server_results", "hphi_server_now", "hphi_server_stats", "hphi_server_tune",
+    "hphi_lobpcg", "hphi_herm_eig",
     "hphi_lanczos_eigenvector", "hphi_vec_lanczos_update_acc", "hphi_expec_energy_flct", "hphi_expec_cisajs",
     "hphi_expec_cisajscktalt", "hphi_write_vec_file", "hphi_read_vec_file", "hphi_write_restart_vecs",
     "hphi_read_restart_vecs", "hphi_write_tmcomponents", "hphi_read_tmcomponents", "hphi_write_energy",
@@ -181,6 +182,7 @@ def lib():
         L.hphi_server_now.argtypes = [_vp]
         L.hphi_server_now.restype = C.c_double
         L.hphi_server_stats.argtypes = [_vp, _f64p]
+        L.hphi_server_tune.argtypes = [_vp, C.c_char_p, C.c_int]
         L.hphi_lanczos_eigenvector.argtypes = [_vp, C.POINTER(LanczosParams), C.c_int, _vp,
                                                C.POINTER(LanczosResult)]
         L.hphi_vec_lanczos_update_acc.argtypes = [_vp, _vp, _vp, _vp, C.c_double, C.c_double, C.c_double]
@@ -594,6 +596,10 @@ class Server:
         check(lib().hphi_server_submit(self.h, C.byref(d), seed, t_arrival, C.byref(i)))
         del keep
         return i.value
+
+    def tune(self, **knobs) -> None:
+        for k, v in knobs.items():
+            check(lib().hphi_server_tune(self.h, k.encode(), int(v)))
 
     def tick(self):
         a, w = C.c_int(), C.c_int()

@@ -9,7 +9,7 @@
 // decodes the state's bits, predicates, Jordan-Wigner signs and target
 // indices once and applies them to every running column of its slab, so up
 // to SL_K jobs pay for one index decode and read one 64-byte row per term;
-// slabs whose sector has a class layout run by classes (k_sl_cls).
+// large sectors with a class layout run by classes (hphi_slab_cls_pays).
 //
 // A tick
 //   1. admits waiting jobs: first, free columns of running slabs go to arrived
@@ -361,22 +361,16 @@ __device__ __forceinline__ void sl_hv_state(CSlab S, uint64_t j, const uint16_t 
   }
 }
 
-// pass 2 over one chunk of SL_TPW tiles of one slab: Q_c <- cc_c Q_c + s_c (H w)_c
-// for the running columns; <w_c|H w_c> per chunk
-__global__ __launch_bounds__(SV_TPB) void k_sl_hv(const SlabDev *slabs, const uint64_t *prefix, int ns,
-                                                  const double *js, double2 *partial) {
-  extern __shared__ uint4 s21v[];
+// pass 2 by states, one chunk of SL_TPW tiles of a slab: Q_c <- cc_c Q_c + s_c (H w)_c
+// for the running columns; <w_c|H w_c> per wave and column into red.  s21v: list_2_1 in LDS
+__device__ __forceinline__ void sl_by_state(CSlab S, uint64_t chunk, const uint4 *s21v, const double *js,
+                                            double2 (*red)[SL_K]) {
   const uint16_t *s21 = (const uint16_t *)s21v;
-  int sb;
-  const uint64_t chunk = sl_chunk8((CU64)prefix, ns, &sb);
-  CSlab S = (CSlab)slabs + sb;
-  const uint32_t n8 = (uint32_t)((S->size21 + 7) / 8);  // 16-byte rows of the packed table
-  for (uint32_t i = threadIdx.x; i < n8; i += SV_TPB) s21v[i] = S->l21p[i];
   __syncthreads();
   double pre[SL_K], pim[SL_K];
 #pragma unroll
   for (int c = 0; c < SL_K; c++) pre[c] = pim[c] = 0.0;
-  const uint64_t t0 = (chunk - ((CU64)prefix)[sb]) * SL_TPW;
+  const uint64_t t0 = chunk * SL_TPW;
   const int full = (1 << SL_K) - 1;
   const bool real = ((S->realc | ~S->mask) & full) == full;  // every running column has real couplings
   const uint64_t dim = S->dim;
@@ -386,8 +380,6 @@ __global__ __launch_bounds__(SV_TPB) void k_sl_hv(const SlabDev *slabs, const ui
     if (real) sl_hv_state<true>(S, j, s21, js, pre, pim);
     else sl_hv_state<false>(S, j, s21, js, pre, pim);
   }
-  // per-column prdct partials: [blk][SL_K] double2
-  __shared__ double2 red[SV_TPB / 64][SL_K];
 #pragma unroll
   for (int c = 0; c < SL_K; c++) {
     for (int off = 32; off > 0; off >>= 1) {
@@ -398,15 +390,6 @@ __global__ __launch_bounds__(SV_TPB) void k_sl_hv(const SlabDev *slabs, const ui
   if ((threadIdx.x & 63) == 0)
 #pragma unroll
     for (int c = 0; c < SL_K; c++) red[threadIdx.x >> 6][c] = make_double2(pre[c], pim[c]);
-  __syncthreads();
-  if (threadIdx.x < SL_K) {
-    double2 s = red[0][threadIdx.x];
-    for (int w = 1; w < SV_TPB / 64; w++) {
-      s.x += red[w][threadIdx.x].x;
-      s.y += red[w][threadIdx.x].y;
-    }
-    partial[chunk * SL_K + threadIdx.x] = s;
-  }
 }
 
 // ---- pass 2 by classes (the layout of hv_class.hip): a wave takes 64 / SL_K ranks
@@ -415,10 +398,11 @@ __global__ __launch_bounds__(SV_TPB) void k_sl_hv(const SlabDev *slabs, const ui
 // high-half and mixed targets from the slab's table, couplings from LDS.
 //
 // A burst of 40 jobs (24-site sectors and smaller), microseconds per launch:
-// k_sl_hv 1,126; this kernel with an eighth of the launch per XCD 1,023 (XCDs
+// by states 1,126; by classes with an eighth of the launch per XCD 1,023 (XCDs
 // with the heavier slabs last), an eighth of every slab 803, units dealt so that
 // workgroups running together stay neighbours 733.  It misses L2 for 4.0 GB per
 // launch, 5.5 TB/s, the rate of a large copy; one or four blocks per wave cost 8 %.
+#define SL_LDS (40 << 10)         // of one workgroup, for four per CU
 #define SC_B 2                    // blocks per wave
 #define SC_RPT (64 / SL_K)        // ranks per tile
 #define SC_W (SV_TPB / 64)        // waves per workgroup
@@ -598,29 +582,19 @@ __device__ __forceinline__ void sc_coef(CSlab S, CCls C, double *sco) {
   }
 }
 
-// dynamic LDS: list_2_1 (n21 16-byte rows), row offsets (nla uint32), couplings
-__global__ __launch_bounds__(SV_TPB) void k_sl_cls(const SlabDev *slabs, const uint64_t *prefix, int ns,
-                                                   const double *js, double2 *partial, uint32_t n21, uint32_t nla) {
-  extern __shared__ uint4 s21v[];
+// pass 2 by classes, workgroup i of the slab's 8 m; LDS: list_2_1, row offsets, couplings
+__device__ __forceinline__ void sl_by_class(CSlab S, CCls C, uint32_t i, uint32_t m, const uint4 *s21v, uint32_t *sla,
+                                            double *sco, const double *js, double2 (*red)[SL_K]) {
   const uint16_t *s21 = (const uint16_t *)s21v;
-  uint32_t *sla = (uint32_t *)(s21v + n21);
-  double *sco = (double *)(sla + nla);
-  int sb;
-  const uint64_t chunk = sl_chunk8((CU64)prefix, ns, &sb);
-  CSlab S = (CSlab)slabs + sb;
-  const CCls C = (CCls)S->cls;
   const int full = (1 << SL_K) - 1;
   const bool real = ((S->realc | ~S->mask) & full) == full;  // every running column has real couplings
-  const uint32_t n8 = (uint32_t)((S->size21 + 7) / 8);
-  for (uint32_t i = threadIdx.x; i < n8; i += SV_TPB) s21v[i] = S->l21p[i];
   if (real) sc_coef<true>(S, C, sco);
   else sc_coef<false>(S, C, sco);
   __syncthreads();
   // an eighth of the units per XCD, dealt to groups of SC_G workgroups, whose
   // waves take every (4 x group)-th unit: workgroups that run together work on
   // neighbouring units, whose gathers meet in L2
-  const uint32_t m = (uint32_t)(((CU64)prefix)[sb + 1] - ((CU64)prefix)[sb]) / 8;
-  const uint32_t i = (uint32_t)(chunk - ((CU64)prefix)[sb]), x = i / m, g0 = i % m / SC_G * SC_G;
+  const uint32_t x = i / m, g0 = i % m / SC_G * SC_G;
   const uint32_t gn = g0 + SC_G < m ? SC_G : m - g0;
   const uint64_t X0 = (uint64_t)C->units * x / 8, XN = (uint64_t)C->units * (x + 1) / 8 - X0;
   const uint32_t u0 = (uint32_t)(X0 + XN * g0 / m) + (i % m - g0) * SC_W, u1 = (uint32_t)(X0 + XN * (g0 + gn) / m);
@@ -632,12 +606,33 @@ __global__ __launch_bounds__(SV_TPB) void k_sl_cls(const SlabDev *slabs, const u
     if (real) sc_units<true, false>(S, C, u0, u1, gn * SC_W, s21, sla, sco, js, &pre, &pim);
     else sc_units<false, false>(S, C, u0, u1, gn * SC_W, s21, sla, sco, js, &pre, &pim);
   }
-  __shared__ double2 red[SC_W][SL_K];
   for (int off = 32; off >= SL_K; off >>= 1) {
     pre += __shfl_xor(pre, off, 64);
     pim += __shfl_xor(pim, off, 64);
   }
   if ((threadIdx.x & 63) < SL_K) red[threadIdx.x >> 6][threadIdx.x & 63] = make_double2(pre, pim);
+}
+
+// Pass 2 of all slabs: by classes or by states, the slab decides.  One kernel for
+// both, so that slabs of either kind fill the device together (as two launches, one
+// after the other, a burst of 40 jobs takes 2 % longer); either path's registers
+// allow 16 waves per CU, four workgroups, and so do 40 KB of LDS.  Dynamic LDS:
+// list_2_1; by classes the row offsets (nla uint32) from the n21-th 16 bytes on, then the couplings.
+__global__ __launch_bounds__(SV_TPB) void k_sl_hv(const SlabDev *slabs, const uint64_t *prefix, int ns,
+                                                  const double *js, double2 *partial, uint32_t n21, uint32_t nla) {
+  extern __shared__ uint4 s21v[];
+  __shared__ double2 red[SC_W][SL_K];
+  int sb;
+  const uint64_t chunk = sl_chunk8((CU64)prefix, ns, &sb);
+  CSlab S = (CSlab)slabs + sb;
+  const uint32_t n8 = (uint32_t)((S->size21 + 7) / 8);  // 16-byte rows of the packed table
+  for (uint32_t i = threadIdx.x; i < n8; i += SV_TPB) s21v[i] = S->l21p[i];
+  const uint64_t at = ((CU64)prefix)[sb];
+  if (S->cls)
+    sl_by_class(S, (CCls)S->cls, (uint32_t)(chunk - at), (uint32_t)(((CU64)prefix)[sb + 1] - at) / 8, s21v,
+                (uint32_t *)(s21v + n21), (double *)((uint32_t *)(s21v + n21) + nla), js, red);
+  else
+    sl_by_state(S, chunk - at, s21v, js, red);
   __syncthreads();
   if (threadIdx.x < SL_K) {
     double2 s = red[0][threadIdx.x];
@@ -871,6 +866,46 @@ __global__ void k_sl_start(double2 *R, double2 *Q, int col, uint64_t dim, uint64
 }
 
 // ==================================================================== host
+// Which slabs run by classes (mode -1; 1: every one the layout fits).  By classes
+// a wave covers 16 ranks of two blocks with four lanes per state that all test the
+// term, where by states a lane tests it for its state's columns at once; it pays
+// where the gathers, not those tests, are the time.  Microseconds per launch, by
+// states / by classes, one slab and four:
+//   Spin   20 sites, 10 up (184,756)       43 / 48     120 / 106 (rings of 40 to 64 terms from 5 x 2^15
+//          23 sites, 7 up (245,157)        47 / 50     159 / 136  states on: the fuller launches count)
+//          24 sites, 6 up (134,596)        43 / 50     118 / 101
+//          20 sites, 190 terms (184,756)  140 / 171    452 / 437
+//          22 sites, 8 up (319,770)        67 / 56     196 / 160
+//          4x4 J1-J2 (12,870)              34 / 43     45 / 46
+//          6x4, 6 up (134,596)             73 / 101    194 / 208
+//          6x4, 7 up (346,104)            141 / 109    413 / 353
+//          6x4, 12 up (2.7e6)             870 / 673
+//   Hubbard 12 sites, 3 + 3 (48,400)       19 / 33     31 / 42
+//          5 + 6 (731,808)                 89 / 91     261 / 250 (three slabs, as below)
+//          6 + 6 (853,776)                104 / 97     306 / 301
+//          13 sites, 6 + 6 (2.9e6)        386 / 347   1085 / 980
+//          12 sites, 6 + 6, with 4 four-orbital InterAll pairs (a term acts on 0.39 of the
+//          states, not half): 117 / 120, 341 / 353; complex hops (0.25) 140 / 139, 384 / 380
+// LDS: four workgroups per CU.  All-to-all exchange on 26 sites, 7 up (657,800; 325
+// terms, 42 KB): 664 / 663, 1829 / 2032; on 24 (735,471; 276 terms, 30 KB) 634 / 530, 1785 / 1413.
+bool hphi_slab_cls_pays(const hphi_engine &h) {
+  const bool hub = h.model == HPHI_MODEL_HUBBARD;
+  double share = 0.0;
+  size_t n = 0;
+  std::vector<uint64_t> lo;  // low-half flips of the mixed terms
+  for (const GTerm &t : h.h_terms_dev) {
+    if (t.kind == P_EQ && t.tmask == 0 && t.tval != 0) continue;
+    n++;
+    share += t.kind != P_EQ ? 0.5 : 1.0 / (double)((uint64_t)1 << __builtin_popcountll(t.tmask));
+    const uint64_t all = t.flip | t.tmask | t.sgn, f = t.flip & h.irght;
+    if ((all & h.irght) && (all & ~h.irght) && std::find(lo.begin(), lo.end(), f) == lo.end()) lo.push_back(f);
+  }
+  if (h.dim < (hub ? (uint64_t)3 << 18 : n <= 64 ? (uint64_t)5 << 15 : (uint64_t)1 << 18)) return false;
+  const size_t lds = 2 * h.size21 + sizeof(uint32_t) * SC_W * SC_RPT * lo.size() + 16 * SL_K * (n + 14) +  // padding
+                     sizeof(double2) * SC_W * SL_K;
+  return lds <= SL_LDS && (!hub || share >= 0.4 * (double)n);
+}
+
 namespace {
 
 struct Arena {
@@ -1020,7 +1055,7 @@ struct Slab {
   double *hist = nullptr;   // [SL_K][2][max_iter + 2]
   std::vector<double2> coef_host;
   ClsArgs cls{};             // class layout (plan with device addresses)
-  ClsArgs *d_cls = nullptr;  // its copy on the device; null: k_sl_hv serves the slab
+  ClsArgs *d_cls = nullptr;  // its copy on the device; null: by states
   uint64_t hv_chunks = 0;    // workgroups of its H·v
   uint64_t nnz = 0;  // off-diagonal elements of one column's H (hphi_term_nnz)
   Job *col[SL_K] = {};
@@ -1044,9 +1079,9 @@ size_t slab_footprint(const hphi_engine &h, int max_iter, bool cls) {
 // slab within the arena and list_2_1 (32 KB), row offsets (16 KB) and couplings
 // (64 KB) fit LDS; the answer depends on the structure and the arena alone, so
 // every slab of a structure runs the same kernel.
-bool slab_cls(const hphi_engine &h, int max_iter, size_t arena) {
-  return h.size21 <= 16384 && h.h_terms_dev.size() + 5 * 7 <= 1024 && hphi_cls_bytes_bound(&h) &&
-         slab_footprint(h, max_iter, true) <= arena;
+bool slab_cls(const hphi_engine &h, int max_iter, size_t arena, int mode) {
+  return mode != 0 && (mode == 1 || hphi_slab_cls_pays(h)) && h.size21 <= 16384 && h.h_terms_dev.size() + 5 * 7 <= 1024 &&
+         hphi_cls_bytes_bound(&h) && slab_footprint(h, max_iter, true) <= arena;
 }
 
 double mono_now() {
@@ -1084,6 +1119,7 @@ struct hphi_server {
   double st_hv_s = 0, st_hv_bytes = 0;
   uint64_t st_hv_launches = 0;
   uint64_t st_moves = 0;  // columns moved between slabs (compact)
+  int cls = -1;           // slabs by classes: -1 where it is the faster one, 0 none, 1 every one the layout fits
 };
 
 extern "C" double hphi_server_now(const hphi_server *s) { return s ? mono_now() - s->t0 : 0.0; }
@@ -1174,7 +1210,7 @@ extern "C" int hphi_server_submit(hphi_server *s, const hphi_model_desc *d, uint
   j->shash = structure_hash(j->h);
   for (const GTerm &t : j->h.h_terms_dev)
     if (t.cim != 0.0) j->realc = 0;
-  j->cls = slab_cls(j->h, s->p.max_iter, s->arena.size);
+  j->cls = slab_cls(j->h, s->p.max_iter, s->arena.size, s->cls);
   const size_t fp = slab_footprint(j->h, s->p.max_iter, j->cls);
   if (fp > s->arena.size) {
     delete j;
@@ -1257,7 +1293,7 @@ static int slab_create(hphi_server *s, const Job *j, size_t off, size_t bytes, S
   if (!rc && cls) {
     b->cls = plan;
     hphi_cls_units(b->cls, SC_B, SC_RPT);
-    // SC_UPW units per wave, fewer while that leaves CUs idle; no more workgroups than k_sl_hv has
+    // SC_UPW units per wave, fewer while that leaves CUs idle; no more workgroups than by states
     const uint64_t w = (b->cls.units + SC_W - 1) / SC_W;
     b->hv_chunks = std::min<uint64_t>(b->hv_chunks, std::max<uint64_t>(w / SC_UPW, std::min<uint64_t>(w, 256)));
     b->d_cls = (ClsArgs *)p, p += al256(sizeof(ClsArgs));
@@ -1579,12 +1615,14 @@ extern "C" int hphi_server_tick(hphi_server *s, int *n_active, int *n_waiting) {
     }
     if (tiles > s->max_tiles) return hphi_set_error("too many tiles in flight");
     const size_t lds = 16 * (size_t)((max21 + 7) / 8);  // list_2_1 as uint16 (rank + 2 < 2^16 for <= 16 low bits)
-    if (lds > 65536)
-      (void)hipFuncSetAttribute((const void *)k_sl_hv, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     const uint32_t n21 = (uint32_t)((maxk21 + 7) / 8), nla = (uint32_t)((maxla + 3) / 4 * 4);
     const size_t ldsk = 16 * (size_t)n21 + 4 * (size_t)nla + maxco;
-    if (ldsk > 65536)
-      (void)hipFuncSetAttribute((const void *)k_sl_cls, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldsk);
+    // one launch of pass 2, unless list_2_1 of a slab without class layout would
+    // leave the others fewer workgroups per CU
+    const size_t ldsm = std::max(lds, ldsk);
+    const bool split = ldsm > SL_LDS;
+    if (ldsm > 65536)
+      (void)hipFuncSetAttribute((const void *)k_sl_hv, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldsm);
     HIPCHK(hipMemcpyAsync(s->d_slabs, sd.data(), sizeof(SlabDev) * sd.size(), hipMemcpyHostToDevice, s->stream));
     HIPCHK(hipMemcpyAsync(s->d_cols, cd.data(), sizeof(ColDev) * cd.size(), hipMemcpyHostToDevice, s->stream));
     HIPCHK(hipMemcpyAsync(s->d_prefix, prefix.data(), sizeof(uint64_t) * prefix.size(), hipMemcpyHostToDevice,
@@ -1604,12 +1642,11 @@ extern "C" int hphi_server_tick(hphi_server *s, int *n_active, int *n_waiting) {
       HIPCHK(hipEventRecord(s->ev_hv[2 * st], s->stream));
       const uint64_t *dpv = s->d_prefix + s_pv0[st], *pvh = prefix.data() + s_pv0[st];
       const int nk = s_nk[st];
-      if (nk)
-        hipLaunchKernelGGL(k_sl_cls, dim3((unsigned)pvh[nk]), dim3(SV_TPB), ldsk, s->stream, dsl, dpv,
-                           nk, (const double *)s->d_js, (double2 *)s->d_part, n21, nla);
-      if (ns > nk)
-        hipLaunchKernelGGL(k_sl_hv, dim3((unsigned)(pvh[ns] - pvh[nk])), dim3(SV_TPB), lds, s->stream,
-                           dsl + nk, dpv + nk, ns - nk, (const double *)s->d_js, (double2 *)s->d_part);
+      for (int a = 0, b; a < ns; a = b) {  // slabs a .. b-1
+        b = split && a < nk ? nk : ns;
+        hipLaunchKernelGGL(k_sl_hv, dim3((unsigned)(pvh[b] - pvh[a])), dim3(SV_TPB), !split ? ldsm : a < nk ? ldsk : lds,
+                           s->stream, dsl + a, dpv + a, b - a, (const double *)s->d_js, (double2 *)s->d_part, n21, nla);
+      }
       HIPCHK(hipEventRecord(s->ev_hv[2 * st + 1], s->stream));
       hipLaunchKernelGGL(k_sl_alpha, dim3(nc), dim3(CS_TPB), 0, s->stream, dcl, dpv, (const double2 *)s->d_part,
                          s->d_js, out);
@@ -1699,6 +1736,14 @@ extern "C" int hphi_server_tick(hphi_server *s, int *n_active, int *n_waiting) {
   }
   if (n_active) *n_active = (int)s->active.size();
   if (n_waiting) *n_waiting = (int)s->waiting.size();
+  return 0;
+}
+
+extern "C" int hphi_server_tune(hphi_server *s, const char *knob, int value) {
+  if (!s || !knob) return hphi_set_error("hphi_server_tune: NULL argument");
+  if (strcmp(knob, "cls")) return hphi_set_error("unknown tuning knob %s", knob);
+  if (value < -1 || value > 1) return hphi_set_error("cls must be -1, 0 or 1");
+  s->cls = value;
   return 0;
 }
 

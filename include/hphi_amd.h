@@ -482,6 +482,9 @@ double hphi_server_now(const hphi_server *s);
  * element), their number; jobs moved between slabs of one structure to pack
  * their running columns into fewer slabs */
 int hphi_server_stats(const hphi_server *s, double *out);
+/* Knob of jobs submitted from here on: "cls" -1|0|1, slabs by classes (-1: where
+ * that is the faster kernel; 1: wherever the layout fits). */
+int hphi_server_tune(hphi_server *s, const char *knob, int value);
 
 /* k lowest eigenvalues (ascending) of the symmetric tridiagonal matrix with
  * diagonal a[0..n) and off-diagonal b[0..n-1), by Sturm bisection (host only;

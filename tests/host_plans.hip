@@ -10,6 +10,7 @@
 #include "hphi_amd.h"
 
 int hphi_engine_prepare(const hphi_model_desc *d, hphi_engine *e);
+bool hphi_slab_cls_pays(const hphi_engine &h);
 
 // a canonical engine as hphi_engine_create leaves it, with its class layout planned
 static bool plan(const hphi_model_desc &d, hphi_engine &e, std::vector<char> &up) {
@@ -95,6 +96,7 @@ static void by_default(const char *name, hphi_model_desc &d) {
   if (!plan(d, e, up)) return;
   printf("default_%s", name);
   for (int k = 1; k <= 16; k *= 2) printf(" %d", hphi_cls_wanted(&e, k));
+  printf(" %d", hphi_slab_cls_pays(e));
   e.cls = 1;
   printf(" %d %d\n", hphi_cls_wanted(&e, 1), e.cls_args.nlo);
 }
@@ -107,6 +109,17 @@ static void ring_default(int n, int nup) {
   d.model = HPHI_MODEL_SPIN, d.nsite = n, d.nup = nup;
   d.n_exchange = 2 * n, d.exchange_ij = ij.data(), d.exchange_J = J.data();
   by_default(("spin_" + std::to_string(n) + "_" + std::to_string(nup)).c_str(), d);
+}
+// all-to-all exchange: many terms, whose couplings take LDS in a served slab
+static void all_to_all_default(int n, int nup) {
+  std::vector<int> ij;
+  for (int i = 0; i < n; i++)
+    for (int j = i + 1; j < n; j++) ij.push_back(i), ij.push_back(j);
+  std::vector<double> J(ij.size() / 2, 1.0);
+  hphi_model_desc d{};
+  d.model = HPHI_MODEL_SPIN, d.nsite = n, d.nup = nup;
+  d.n_exchange = (int)J.size(), d.exchange_ij = ij.data(), d.exchange_J = J.data();
+  by_default(("all_" + std::to_string(n) + "_" + std::to_string(nup)).c_str(), d);
 }
 static void hubbard_default(int n, int u, int w, int pairs) {
   std::vector<int> idx, ia;
@@ -132,6 +145,8 @@ static void hubbard_default(int n, int u, int w, int pairs) {
               std::to_string(iv.size() / 4)).c_str(), d);
 }
 static void defaults() {
+  all_to_all_default(24, 8), all_to_all_default(26, 7);
+  ring_default(22, 8), ring_default(20, 10), all_to_all_default(20, 10), hubbard_default(12, 5, 6, 0), hubbard_default(12, 6, 6, 4);
   ring_default(20, 2), ring_default(28, 5), ring_default(30, 5), ring_default(32, 27), ring_default(24, 6);
   ring_default(32, 6), ring_default(24, 12);
   hubbard_default(8, 1, 1, 0), hubbard_default(14, 3, 3, 0), hubbard_default(16, 3, 3, 0), hubbard_default(15, 3, 3, 0);

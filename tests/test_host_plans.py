@@ -91,7 +91,7 @@ DEFAULTS = {
 
 @pytest.mark.parametrize("name", DEFAULTS)
 def test_default_kernel_of_canonical_sectors(plans, name):
-    *wanted, forced, nlo = plans["default_" + name].split()
+    *wanted, slab, forced, nlo = plans["default_" + name].split()
     assert " ".join(wanted) == DEFAULTS[name], nlo
     assert forced == "1"
 
@@ -111,3 +111,11 @@ def test_default_kernel_of_grand_canonical_sectors(plans, name):
     got = plans["gc_" + name].split()
     assert " ".join(got[:5]) == GC_DEFAULTS[name]
     assert all(f >= w for w, f in zip(got[:5], got[5:])) and "1" in got[5:]
+
+
+@pytest.mark.parametrize("name,on", [("spin_24_6", 0), ("spin_20_10", 1), ("spin_22_8", 1), ("all_20_10", 0), ("spin_24_12", 1),
+                                     ("hubbard_12_5_6_0", 0), ("hubbard_12_6_6_0", 1), ("hubbard_12_6_6_4", 0),
+                                     ("hubbard_14_3_3_0", 0), ("all_24_8", 1), ("all_26_7", 0)])
+def test_served_slabs_by_classes(plans, name, on):
+    """By size, by the share of the states that a term acts on (Hubbard) and by LDS."""
+    assert int(plans["default_" + name].split()[5]) == on
