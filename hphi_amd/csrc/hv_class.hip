@@ -436,10 +436,16 @@ void hphi_cls_shape(const hphi_engine *e, int k, int *cb, int *cpl) {
 //   Hubbard 7x2, 3 + 4 (0.55)                        33.2 / 38.1
 //   Hubbard 16 sites, 2 + 5 (0.61)                   41.0 / 35.4; k = 2 50.3 / 48.4
 //   Hubbard 5x3, 3 + 3 (0.41), k = 4                 57.5 / 67.0; 143,325 states (0.44) 49.1 / 42.3
+//
+// Hubbard sectors of a few workgroups: a chain of latencies either way, and the
+// gather kernels' is the shorter (k_hv_canon has one rank lookup less in front of a
+// term).  225 states: 11.5 / 12.5, k = 2 10.3 / 12.1, k = 4 12.4 / 11.5; 36: k = 4 9.8 / 10.8;
+// 784: 11.6 / 12.7, k = 2 12.8 / 12.5; 3,136: 11.9 / 12.3; 4,900: 12.0 / 11.7.
 static bool cls_pays(const hphi_engine *e, int k) {
   const ClsArgs &A = e->cls_args;
   if (A.nlo > 36) return false;
   const bool hub = e->model == HPHI_MODEL_HUBBARD;
+  if (hub && k <= 4 && e->dim < (k == 1 ? 4096u : k == 2 ? 512u : 128u)) return false;
   if (A.nlo <= 26 && (e->dim < (uint64_t)1 << 17 || e->dim >= (uint64_t)1 << 19 || k > (hub ? 4 : 1))) return true;
   uint64_t lanes = 0;
   for (int c = 0; c < A.ncls; c++) lanes += (uint64_t)A.nblk[c] * ((A.size[c] + 63) / 64 * 64);

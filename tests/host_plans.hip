@@ -149,6 +149,7 @@ static void defaults() {
   ring_default(22, 8), ring_default(20, 10), all_to_all_default(20, 10), hubbard_default(12, 5, 6, 0), hubbard_default(12, 6, 6, 4);
   ring_default(20, 2), ring_default(28, 5), ring_default(30, 5), ring_default(32, 27), ring_default(24, 6);
   ring_default(32, 6), ring_default(24, 12);
+  hubbard_default(4, 1, 1, 0), hubbard_default(6, 2, 2, 0), hubbard_default(8, 3, 3, 0), hubbard_default(8, 4, 4, 0);
   hubbard_default(8, 1, 1, 0), hubbard_default(14, 3, 3, 0), hubbard_default(16, 3, 3, 0), hubbard_default(15, 3, 3, 0);
   hubbard_default(16, 2, 5, 0), hubbard_default(12, 6, 6, 0), hubbard_default(12, 6, 6, 30), hubbard_default(16, 4, 4, 20);
   hubbard_default(16, 4, 4, 32), hubbard_default(16, 4, 4, 36), hubbard_default(12, 3, 3, 30);

@@ -80,7 +80,9 @@ DEFAULTS = {
     "spin_20_2": "1 1 1 1 1", "spin_24_12": "1 1 1 1 1", "spin_24_6": "1 1 1 1 1", "spin_32_6": "1 1 1 1 1",
     "spin_28_5": "1 1 1 1 1",                                  # as dilute, but fewer than 2^17 states
     "spin_30_5": "0 1 1 1 1", "spin_32_27": "0 1 1 1 1",       # dilute: single columns
-    "hubbard_8_1_1_0": "1 1 1 1 1", "hubbard_12_6_6_0": "1 1 1 1 1", "hubbard_16_2_5_0": "1 1 1 1 1",
+    "hubbard_4_1_1_0": "0 0 0 1 1", "hubbard_8_1_1_0": "0 0 0 1 1", "hubbard_6_2_2_0": "0 0 1 1 1",  # a few workgroups
+    "hubbard_8_3_3_0": "0 1 1 1 1", "hubbard_8_4_4_0": "1 1 1 1 1",
+    "hubbard_12_6_6_0": "1 1 1 1 1", "hubbard_16_2_5_0": "1 1 1 1 1",
     "hubbard_14_3_3_0": "0 0 1 1 1", "hubbard_16_3_3_0": "0 0 1 1 1",
     "hubbard_15_3_3_0": "0 0 0 1 1",
     "hubbard_12_6_6_30": "1 1 1 1 1", "hubbard_16_4_4_20": "1 1 1 1 1", "hubbard_16_4_4_32": "1 1 1 1 1",
