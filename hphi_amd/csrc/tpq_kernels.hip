@@ -142,10 +142,12 @@ __global__ __launch_bounds__(TQ_TPB) void k_tpq_fused(double2 *v1, const double2
 // One workgroup's sums of the m columns of partial[nblk][m] (m a power of two,
 // at most 128) into sh[0..m), in fixed order.  Latency-bound: one thread per
 // column took 297 us for 1024 x 128 sums; TQ_FIN threads with eight loads in
-// flight each take 55 us (1 MB through one CU).
+// flight each take 55 us (1 MB through one CU).  Up to 1,024 sums two waves
+// (tq_fin): sixteen, to start and to join, make a step of 64 states 20.0 us, two 18.9.
 #define TQ_FIN 1024
+static int tq_fin(int nblk, int m) { return nblk * m <= 1024 ? 128 : TQ_FIN; }
 __device__ __forceinline__ void tq_colsums(const double *__restrict__ partial, int nblk, int m, double *sh) {
-  const int q = threadIdx.x % m, ns = TQ_FIN / m;
+  const int q = threadIdx.x % m, ns = blockDim.x / m;
   double a[8] = {};
   for (int b = threadIdx.x / m; b < nblk; b += 8 * ns) {
 #pragma unroll
@@ -154,7 +156,7 @@ __device__ __forceinline__ void tq_colsums(const double *__restrict__ partial, i
   }
   sh[threadIdx.x] = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
   __syncthreads();
-  for (int st = TQ_FIN / 2; st >= m; st >>= 1) {
+  for (int st = blockDim.x / 2; st >= m; st >>= 1) {
     if (threadIdx.x < st) sh[threadIdx.x] += sh[threadIdx.x + st];
     __syncthreads();
   }
@@ -297,7 +299,7 @@ static int tpq_enqueue_step(hphi_engine *e, const TpqPlan &P) {
                      dim, P.k, P.sj, P.sc, (const double *)P.state, P.lv, 1.0 / P.Ns, P.obs_kind, e->nsite,
                      hphi_model_gc(e->model) ? (const uint64_t *)nullptr : (const uint64_t *)e->d_list1,
                      P.part);
-  hipLaunchKernelGGL(k_tpq_finalize, dim3(1), dim3(TQ_FIN), 0, e->stream, (const double *)P.part, P.g, P.k,
+  hipLaunchKernelGGL(k_tpq_finalize, dim3(1), dim3(tq_fin(P.g, P.k * TQ_NRED)), 0, e->stream, (const double *)P.part, P.g, P.k,
                      (const double2 *)(P.layout == 1 ? e->d_prdct : e->d_coef), P.state, P.lv, P.Ns, P.obs_kind,
                      e->nsite, P.sz_const, P.out, P.steps, P.row0);
   HIPCHK(hipGetLastError());
@@ -390,7 +392,7 @@ static int tpq_run(hphi_engine *e, const hphi_tpq_params *p, const double *W0, i
                          p->init_kind);
     hipLaunchKernelGGL(k_tpq_colnorm, dim3(P.g), dim3(TQ_TPB), 0, e->stream, (const double2 *)P.V1, dim, k, P.sj,
                        P.sc, P.part);
-    hipLaunchKernelGGL(k_tpq_start, dim3(1), dim3(TQ_FIN), 0, e->stream, (const double *)P.part, P.g, k, P.state);
+    hipLaunchKernelGGL(k_tpq_start, dim3(1), dim3(tq_fin(P.g, k)), 0, e->stream, (const double *)P.part, P.g, k, P.state);
     if (step0 > 0) {  // resumed: the given vector is step step0 - 1's, its row is not kept
       hipLaunchKernelGGL(k_tpq_set_step, dim3(1), dim3(1), 0, e->stream, P.state, (double)(step0 - 1));
       P.row0 = step0;
@@ -667,14 +669,14 @@ static int ctpq_run(hphi_engine *e, const hphi_ctpq_params *p, const double *W0,
       // normalise A into P (global_norm; step 0: global_1st_norm)
       hipLaunchKernelGGL(k_tpq_colnorm, dim3(g), dim3(TQ_TPB), 0, e->stream, (const double2 *)A, dim, k, (uint64_t)k,
                          (uint64_t)1, part);
-      hipLaunchKernelGGL(k_ct_norms, dim3(1), dim3(TQ_FIN), 0, e->stream, (const double *)part, g, k, state);
+      hipLaunchKernelGGL(k_ct_norms, dim3(1), dim3(tq_fin(g, k)), 0, e->stream, (const double *)part, g, k, state);
       hipLaunchKernelGGL(k_ct_scale, dim3(gs), dim3(256), 0, e->stream, P, (const double2 *)A, dim, k,
                          (const double *)state);
       // measure: Hp = H P (its prdct is E), <H^2> and the moments (expec_energy_flct)
       if (hphi_hv_launch_ex(e, k, (double *)Hp, (const double *)P, 1)) { rc = -1; break; }
       hipLaunchKernelGGL(k_ct_moments, dim3(g), dim3(TQ_TPB), 0, e->stream, (const double2 *)P, (const double2 *)Hp,
                          dim, k, obs_kind, e->nsite, list1, part);
-      hipLaunchKernelGGL(k_ct_finalize, dim3(1), dim3(TQ_FIN), 0, e->stream, (const double *)part, g, k,
+      hipLaunchKernelGGL(k_ct_finalize, dim3(1), dim3(tq_fin(g, k * TQ_NRED)), 0, e->stream, (const double *)part, g, k,
                          (const double2 *)e->d_prdct, (const double *)state, s, dtau, obs_kind, e->nsite, sz_const,
                          out, step0);
       if (hipGetLastError() != hipSuccess) { rc = hphi_set_error("hphi_ctpq: launch failed"); break; }
