@@ -340,8 +340,10 @@ static bool gc_sources(const hphi_engine *e, std::vector<GcSrc> &out) {
 // terms: grown from every starting bit, each time by the bit that completes
 // the most weight, and among equals the one that shares most with open terms.
 // One- and two-bit flips go through a weight matrix (their gains are updated
-// as bits join: a few thousand operations per set, 0.05 ms for all the plans of
-// a 22-site strip); wider flips are looked up.
+// as bits join); wider ones count once per flip, for the bit that completes them.
+// All plans of a 22-site strip: 0.15 ms of one core; of HubbardGC 10 with 200
+// four-orbital pairs: 1.26 ms with every term looked up for every bit and every block
+// size's plan made anew, 0.15 so.
 static uint32_t gc_pick(const std::vector<GcSrc> &terms, const std::vector<char> &open, int n, int s, int keep,
                         double *weight) {
   double one[32] = {}, two[32][32] = {}, touch[32] = {};
@@ -356,6 +358,12 @@ static uint32_t gc_pick(const std::vector<GcSrc> &terms, const std::vector<char>
     else if (nb == 2) two[a][31 - __builtin_clz(f)] += w, two[31 - __builtin_clz(f)][a] += w;
     else if (nb > 2) wide.emplace_back(f, w);
   }
+  std::sort(wide.begin(), wide.end());  // terms of one flip count together (the weights are powers of two: exact)
+  size_t nw = 0;
+  for (const auto &f : wide)
+    if (nw > 0 && wide[nw - 1].first == f.first) wide[nw - 1].second += f.second;
+    else wide[nw++] = f;
+  wide.resize(nw);
   uint32_t best = 0;
   double bw = -1.0;
   for (int start = 0; start < n; start++) {
@@ -372,14 +380,14 @@ static uint32_t gc_pick(const std::vector<GcSrc> &terms, const std::vector<char>
     if (__builtin_popcount(S) > s) continue;
     while (__builtin_popcount(S) < s) {
       int bb = -1;
-      double bs = -1.0;
-      for (int b = 0; b < n; b++) {
-        if ((S >> b) & 1) continue;
-        double sc = gain[b] + touch[b];
-        for (const auto &f : wide)
-          if (((f.first >> b) & 1) && (f.first & ~(S | (1u << b))) == 0) sc += f.second;
-        if (sc > bs) bs = sc, bb = b;
+      double bs = -1.0, sc[32];
+      for (int b = 0; b < n; b++) sc[b] = gain[b] + touch[b];
+      for (const auto &f : wide) {
+        const uint32_t missing = f.first & ~S;
+        if (missing && !(missing & (missing - 1))) sc[__builtin_ctz(missing)] += f.second;
       }
+      for (int b = 0; b < n; b++)
+        if (!((S >> b) & 1) && sc[b] > bs) bs = sc[b], bb = b;
       add(bb);
     }
     for (const auto &f : wide)
@@ -449,7 +457,9 @@ int hphi_gc_plan_build(hphi_engine *e) {
   if (!gc_sources(e, terms)) return 0;
   const int n = e->nbits, nt = (int)terms.size();
   std::vector<GcTerm> all;
-  double W = 0.0;
+  GcPlan made;  // the last plan made, its columns per tile and what it gathers
+  int made_kc = 0;
+  double W = 0.0, made_wrem = 0.0;
   for (const GcSrc &t : terms) W += gc_weight(t) / GC_COST_GATHER;
   for (int k = 1; k <= 16; k *= 2) {
     const int kc = gc_kc(k);
@@ -457,6 +467,11 @@ int hphi_gc_plan_build(hphi_engine *e) {
     GcPlan &P = e->gc_plan[hphi_block_slot(k)];
     P = GcPlan{};
     if (n < s + 3 || (e->gc_tile != 1 && ((uint64_t)1 << (n - s)) * (uint64_t)(k / kc) < GC_MIN_TILES)) continue;
+    if (made_kc == kc) {  // the same tiles, more of them
+      P = made;
+      if (e->gc_tile != 1 && !gc_pays(e, k, P, W, made_wrem)) P = GcPlan{};
+      continue;
+    }
     const int keep = kc == 1 ? 3 : kc == 2 ? 2 : 0;  // runs of 128 bytes, 64 with KC = 4
     std::vector<char> open(nt, 1);
     uint32_t S[GC_MAXPASS];
@@ -474,7 +489,6 @@ int hphi_gc_plan_build(hphi_engine *e) {
     double wrem = 0.0;
     for (int t = 0; t < nt; t++)
       if (open[t]) nrem++, wrem += gc_weight(terms[t]) / GC_COST_GATHER;
-    const size_t first = all.size();
     std::vector<int> pass(nt, -1);
     int load[GC_MAXPASS] = {4 * nrem + 4};
     for (int many = 0; many < 2; many++)
@@ -550,10 +564,10 @@ int hphi_gc_plan_build(hphi_engine *e) {
         Q.nrem = nrem;
       }
     }
-    if (e->gc_tile != 1 && !gc_pays(e, k, P, W, wrem)) {
-      P = GcPlan{};
-      all.resize(first);
-    }
+    made = P;
+    made_kc = kc;
+    made_wrem = wrem;
+    if (e->gc_tile != 1 && !gc_pays(e, k, P, W, wrem)) P = GcPlan{};
   }
   for (GcTerm &g : all) {
     const GTerm &t = terms[g.src].t;
@@ -565,10 +579,7 @@ int hphi_gc_plan_build(hphi_engine *e) {
     g.cre = t.cre;
     g.cim = t.cim;
   }
-  if (all.empty()) {
-    for (GcPlan &P : e->gc_plan) P.npass = 0;
-    return 0;
-  }
+  if (std::all_of(e->gc_plan, e->gc_plan + 5, [](const GcPlan &P) { return P.npass == 0; })) return 0;
   if (hipMalloc((void **)&e->d_gcterms, sizeof(GcTerm) * all.size()) != hipSuccess) {
     (void)hipGetLastError();
     e->d_gcterms = nullptr;
