@@ -973,7 +973,6 @@ extern "C" void hphi_engine_destroy(hphi_engine *e) {
   (void)hipFree(e->d_l21);
   (void)hipFree(e->d_l22);
   (void)hipFree(e->d_hb);
-  (void)hipFree(e->d_blkpos);
   (void)hipFree(e->d_hitgt);
   (void)hipFree(e->d_v1t);
   (void)hipFree(e->d_tofs);

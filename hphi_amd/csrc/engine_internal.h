@@ -262,7 +262,6 @@ struct hphi_engine {
   int hi_fuse_copy = 1;   // the first pass writes the tile-major copy (0: a copy kernel does)
   int hi_p1_wgs_per_cu = 256;  // workgroups per CU of that first pass (8x4 J1-J2: 90.4 ms at 256, 93.6 at 48)
   uint32_t *d_hb = nullptr;      // blocks of each class (hi_plan)
-  uint32_t *d_blkpos = nullptr;  // position of every block within its class (~0u: empty block)
   uint32_t *d_hitgt = nullptr;  // targets of the high-half pass
   double2 *d_v1t = nullptr;      // tile-major copy of v1, hi_plan.base[ncls] elements
   ulonglong2 *d_tofs = nullptr;  // per block: its first tile-major element, and the stride between its tiles

@@ -525,22 +525,22 @@ int hphi_hi_split_on(hphi_engine *e) {
   }
   P.wgp[P.ncls] = w;
   P.base[P.ncls] = base;
+  uint32_t *blkpos = nullptr;  // position of every block within its class (~0u: empty block)
   if (hipMalloc(&e->d_hb, sizeof(uint32_t) * hb.size()) != hipSuccess ||
-      hipMalloc(&e->d_blkpos, sizeof(uint32_t) * nb) != hipSuccess ||
+      hipMalloc(&blkpos, sizeof(uint32_t) * nb) != hipSuccess ||
       hipMalloc(&e->d_hitgt, sizeof(uint32_t) * hb.size() * std::max(e->n_high, 1)) != hipSuccess ||
       hipMalloc(&e->d_v1t, sizeof(double2) * base) != hipSuccess ||
       hipMalloc(&e->d_tofs, sizeof(ulonglong2) * nb) != hipSuccess ||
       hipMemcpy(e->d_tofs, tofs.data(), sizeof(ulonglong2) * nb, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(e->d_hb, hb.data(), sizeof(uint32_t) * hb.size(), hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(e->d_blkpos, pos.data(), sizeof(uint32_t) * nb, hipMemcpyHostToDevice) != hipSuccess) {
+      hipMemcpy(blkpos, pos.data(), sizeof(uint32_t) * nb, hipMemcpyHostToDevice) != hipSuccess) {
     (void)hipGetLastError();
     (void)hipFree(e->d_hb);
-    (void)hipFree(e->d_blkpos);
+    (void)hipFree(blkpos);
     (void)hipFree(e->d_hitgt);
     (void)hipFree(e->d_v1t);
     (void)hipFree(e->d_tofs);
     e->d_hb = nullptr;
-    e->d_blkpos = nullptr;
     e->d_hitgt = nullptr;
     e->d_v1t = nullptr;
     e->d_tofs = nullptr;
@@ -548,10 +548,11 @@ int hphi_hi_split_on(hphi_engine *e) {
     return 0;
   }
   hipLaunchKernelGGL(k_hi_targets, dim3((unsigned)((hb.size() * e->n_high + 255) / 256)), dim3(256), 0, e->stream,
-                     (const uint32_t *)e->d_hb, (const uint32_t *)e->d_blkpos, (const GTerm *)e->d_terms + e->n_low,
+                     (const uint32_t *)e->d_hb, (const uint32_t *)blkpos, (const GTerm *)e->d_terms + e->n_low,
                      (uint32_t)hb.size(), e->n_high, e->nlow, e->d_hitgt);
   HIPCHK(hipGetLastError());
-  e->bytes += sizeof(uint32_t) * (hb.size() * (1 + (size_t)e->n_high) + nb) + sizeof(double2) * base + sizeof(ulonglong2) * nb;
+  HIPCHK(hipFree(blkpos));  // waits for its only reader
+  e->bytes += sizeof(uint32_t) * (hb.size() * (1 + (size_t)e->n_high)) + sizeof(double2) * base + sizeof(ulonglong2) * nb;
   e->hi_plan = P;
   e->hi_ok = 1;
   return 1;

@@ -747,11 +747,11 @@ static int cls_launch(hphi_engine *e, const HvArgs &H, const ClsArgs &A, int g) 
   const size_t lds = sizeof(uint32_t) * CL_TPB * std::max(A.nlo, 1);
   const bool hub = e->model == HPHI_MODEL_HUBBARD;
 #define CL_GO(R, RK) hipLaunchKernelGGL((k_hv_cls<K, CPL, CB, R, RK>), dim3(g), dim3(CL_TPB), lds, e->stream, H, A)
-  if (e->c2_realc) {
-    if (hub) CL_GO(true, 3);
-    else CL_GO(true, 2);
-  } else {
-    if (hub) CL_GO(false, 3);
+  if (hub) {
+    if (e->c2_realc) CL_GO(true, 3);
+    else CL_GO(false, 3);
+  } else if constexpr (CPL == 1) {  // two columns per lane: Hubbard alone (hphi_cls_shape)
+    if (e->c2_realc) CL_GO(true, 2);
     else CL_GO(false, 2);
   }
 #undef CL_GO
