@@ -355,7 +355,7 @@ ISSUE_COUNTERS = ("SQ_INSTS_VALU", "SQ_INSTS_VMEM_RD", "SQ_INSTS_LDS", "SQ_INSTS
 
 def reduce_issue(directory: str, out: str, cmd: str, cfg: int = 2):
     """Issue-side counters of the plain H·v (one rocprofv3 --pmc pass of
-    --pmc-probe with the SQ counters of ISSUE_COUNTERS): mean per dispatch, per
+    --pmc-probe with the SQ counters of ISSUE_COUNTERS): mean per H·v, per
     64-state tile (one wave's worth of states), and the VALU issue time a tile
     needs (4 cycles per wave64 instruction on a 16-lane SIMD) against the
     cycles a tile may take at the measured launch time."""
@@ -363,13 +363,15 @@ def reduce_issue(directory: str, out: str, cmd: str, cfg: int = 2):
 
     spec = L.baseline_config(cfg)
     dim = spec.dim
-    vals = {c: _pmc_means(directory, c).get("k_hv_cls") for c in ISSUE_COUNTERS}
+    means = {c: _pmc_means(directory, c) for c in ISSUE_COUNTERS}
+    used = [k for k in HV_KERNELS if k in means["SQ_WAVES"]]
+    vals = {c: sum(m[k] for k in used) for c, m in means.items()}
     tiles = dim / 64.0
-    lines = [f"# issue counters of one plain H·v launch (k_hv_cls), {PMC_WORKLOADS[cfg][1]}",
+    lines = [f"# issue counters of one plain H·v ({' + '.join(used)}), {PMC_WORKLOADS[cfg][1]}",
              f"# command: {cmd}"]
     for c in ISSUE_COUNTERS:
         v = vals[c]
-        lines.append(f"{c}: {v:.6e} per dispatch" + (f", {v / tiles:.1f} per 64-state tile" if v else ""))
+        lines.append(f"{c}: {v:.6e} per H·v" + (f", {v / tiles:.1f} per 64-state tile" if v else ""))
     hv_ms = _probe_hv_ms(directory)
     if vals["SQ_INSTS_VALU"] and hv_ms:
         simds = 1024

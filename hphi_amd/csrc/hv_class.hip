@@ -619,16 +619,19 @@ int hphi_cls_upload(const hphi_engine *e, ClsArgs &A, char *dev, const void *up,
   return 0;
 }
 
-// The order of the units.  A vector that the 256 MB memory-side cache holds: class
-// after class, an XCD the next eighth of them after the other, so that each XCD's
-// gathers stay near its own part and meet in its L2 (2.7e6 states 151 us; with the
-// order below 175).  Beyond (2^24 states) gathers that miss L2 would miss that
-// cache too, at the 5.5 TB/s of HBM: groups follow the first index of their first
-// block and are dealt to the XCDs one by one, to the one with the fewest slots, so
-// that all XCDs work in one neighbourhood of the vector instead of eight.  Class
-// after class / by index, an eighth per XCD / dealt one by one / four by four:
-// 8x4 75.3, 72.7, 69.7, 70.5 ms; 7x4 3,380, 3,254, 3,070, 3,071 us, k = 4 16,455, 16,431,
-// 14,658; 4x4 Hubbard 12,880, 13,667 (one block per wave), 11,400, 11,634.
+// The order of the units.  Class after class, an XCD the next eighth of them after
+// the other: each XCD's gathers stay near its own part and meet in its L2, and
+// what misses finds the 256 MB memory-side cache.  From 2^24 states on: groups follow
+// the first index of their first block and are dealt to the XCDs one by one, to the
+// one with the fewest slots, so that all XCDs work in one neighbourhood of the
+// vector instead of eight and gathers that miss L2 have a chance in that cache.
+// By class / by index, k = 1: rings of 24, 25, 26, 27 sites (2.7e6 to 2.0e7 states)
+// 90 / 104, 157 / 190, 382 / 410, 870 / 875 us; Hubbard 14 sites, 6 + 6 (9.0e6) 261 / 274, 7x2
+// (1.2e7) 463 / 520; 7x4 (4.0e7) 3,380 / 3,070; 4x4 Hubbard (1.7e8) 12,880 / 11,400; 8x4 75,300 /
+// 69,700 (with an eighth per XCD by index 72,700, 13,667 on 4x4 Hubbard; dealt four by four
+// 70,500, 11,634).  Blocks cross over earlier, at some 600 MB: ring of 25, k = 4 763 / 777, k = 8
+// 1,595 / 1,550, k = 16 4,084 / 3,667; 7x2 k = 4 1,992 / 1,979, k = 8 4,463 / 4,079; an
+// engine keeps one order, the single column's.
 static int cls_by_index(const hphi_engine *e) {
   if (e->cls_order >= 0) return e->cls_order;
   return e->dim >= (uint64_t)1 << 24;

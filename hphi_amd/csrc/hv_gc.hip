@@ -20,11 +20,13 @@
 // amplitude against 37 on the 11x2 strip at k = 16).
 //
 // 11x2 triangular strip, k = 16 (6.7e7 amplitudes): 6.45 ms in the block kernel,
-// 2.50 ms here in three passes (0.8 ms each: 48 bytes per amplitude at 3.9 TB/s,
-// where a device copy reaches 4.4); k = 1: 442 -> 146 us; HubbardGC ring of 11
-// sites with complex spin flips, k = 2: 308 -> 255 us.  Reading the next tile's
-// rows while the terms run (spills), and tiles of 1024 threads with 4 elements
-// each, were no faster (2.98 and 3.16 ms).
+// 2.67 ms here in three passes (0.61 ms for 32 bytes per amplitude, 3.6 TB/s, then
+// 1.03 ms each for 48 bytes, 3.2 TB/s; a device copy of that size reaches 4.4, a
+// read-modify-write stream 5.5); k = 1: 442 -> 146 us; HubbardGC ring of 11 sites
+// with complex spin flips, k = 2: 308 -> 262 us (95 and 2 x 84: 4.6 and 4.8 TB/s of a
+// vector that the memory-side cache holds).  Reading the next tile's rows while the
+// terms run (spills), and tiles of 1024 threads with 4 elements each, were no faster
+// (2.98 and 3.16 ms, this form 2.50 beside them).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

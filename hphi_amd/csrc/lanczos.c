@@ -211,13 +211,6 @@ static int lanczos_core(hphi_engine *e, const hphi_lanczos_params *p, hphi_lancz
     goto done;
   }
 loop:
-  /* Steps run on the device from check to check (at most LZ_BATCH), with alpha,
-   * beta and the scale factors there: one wait per batch instead of two per step.
-   * Where a step is short against a check (LZ_AHEAD states), the next batch is
-   * queued before the wait, and its steps go unused when the run ends here.
-   * 184,756 states, a check every 5 steps: LZ_OLD us per step with the waits, LZ_ONE
-   * with one per batch, LZ_NEW with a batch ahead.  A run that returns its state
-   * (out) queues single steps, so that the buffers hold the last one's vectors. */
   /* Steps run on the device from check to check (LZ_BATCH at most) with alpha,
    * beta and the scale factors there, one wait per batch instead of two per step.
    * Where a step is short against a check (up to LZ_AHEAD states) the next batch
