@@ -575,6 +575,10 @@ bool hphi_cls_plan(const hphi_engine *e, ClsArgs &A, std::vector<char> &up) {
   std::vector<ClsTerm> terms;
   for (auto &g : grp) terms.insert(terms.end(), g.begin(), g.end());
   A.np = (uint32_t)at.size();
+  // the target table, 4 bytes per block and term: a vector's bytes or 128 MB at most (8x4 J1-J2 takes
+  // 27 MB; thousands of density-assisted hops on 16 sites would take gigabytes), rows addressed in 32 bits
+  const uint64_t entries = (uint64_t)A.np * (uint64_t)A.nt;
+  if (entries > 0xffffffffull || 4 * entries > std::max<uint64_t>(16 * e->dim, (uint64_t)128 << 20)) return false;
   const size_t tb = sizeof(ClsTerm) * terms.size();
   up.resize(tb + 8 * (size_t)A.np);
   std::copy(terms.begin(), terms.end(), (ClsTerm *)up.data());

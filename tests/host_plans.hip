@@ -155,6 +155,37 @@ static void defaults() {
   hubbard_default(16, 4, 4, 32), hubbard_default(16, 4, 4, 36), hubbard_default(12, 3, 3, 30);
 }
 
+// n sites, u + w electrons, `extra` more terms on a ring of hops: each hop assisted by
+// the densities of other orbitals; is there a class layout?
+static void many_terms(int n, int u, int w, int extra) {
+  std::vector<int> ia, idx;
+  std::vector<double> iv, t;
+  for (int i = 0; i < n; i++)
+    for (int s = 0; s < 2; s++) {
+      const int j = (i + 1) % n, a[8] = {i, s, j, s, j, s, i, s};
+      idx.insert(idx.end(), a, a + 8);
+      t.insert(t.end(), {1.0, 0.0, 1.0, 0.0});
+    }
+  for (int i = 0; i < n; i++)
+    for (int j = 0; j < n; j++)
+      for (int m = 0; m < n; m++)
+        for (int s = 0; s < 4 && extra > 0; s++) {
+          if (i == j || m == i || m == j || i > j) continue;
+          const int a[16] = {m, s / 2, m, s / 2, i, s % 2, j, s % 2, j, s % 2, i, s % 2, m, s / 2, m, s / 2};
+          ia.insert(ia.end(), a, a + 16);
+          iv.insert(iv.end(), {0.1, 0.0, 0.1, 0.0});
+          extra -= 2;
+        }
+  hphi_model_desc d{};
+  d.model = HPHI_MODEL_HUBBARD, d.nsite = n, d.nup = u, d.ndown = w;
+  d.n_transfer = (int)idx.size() / 4, d.transfer_idx = idx.data(), d.transfer_t = t.data();
+  d.n_interall = (int)iv.size() / 2, d.interall_idx = ia.data(), d.interall_V = iv.data();
+  hphi_engine e;
+  std::vector<char> up;
+  const bool ok = plan(d, e, up);
+  printf("many_terms_%d_%d_%d %d\n", n, u, (int)iv.size() / 2, ok);
+}
+
 // The autotuner's device calls, in place of the library's: building makes the
 // class layout of a fresh engine available, and a timed call costs what `cost` says.
 static void *layout;
@@ -340,6 +371,7 @@ static void gc_defaults() {
 int main() {
   gc_defaults();
   defaults();
+  many_terms(16, 3, 3, 200), many_terms(16, 3, 3, 6000), many_terms(16, 8, 8, 6000);
   tiles_without_memory();
   autotune_fresh();
   autotune_sizes();

@@ -121,3 +121,10 @@ def test_default_kernel_of_grand_canonical_sectors(plans, name):
 def test_served_slabs_by_classes(plans, name, on):
     """By size, by the share of the states that a term acts on (Hubbard) and by LDS."""
     assert int(plans["default_" + name].split()[5]) == on
+
+
+@pytest.mark.parametrize("name,ok", [("16_3_200", 1), ("16_3_6000", 0), ("16_8_6000", 1)])
+def test_class_layout_keeps_its_target_table_to_a_vector(plans, name, ok):
+    """6,000 density-assisted hops on 8,650 blocks: 200 MB of targets for a vector of 5 MB, so none;
+    with 8 + 8 electrons the vector is 2.6 GB."""
+    assert int(plans["many_terms_" + name]) == ok
