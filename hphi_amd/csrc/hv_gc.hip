@@ -30,6 +30,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <map>
 #include <utility>
 #include <vector>
 
@@ -309,23 +310,23 @@ static double gc_weight(const GcSrc &s) {
 // conjugate couplings) act where the two bits differ, and the imaginary part
 // changes sign with the first one's bit: a parity term with its own sign mask.
 static bool gc_sources(const hphi_engine *e, std::vector<GcSrc> &out) {
+  std::map<uint64_t, std::vector<size_t>> open;  // value terms of one or two bits without their partner, by flip
   for (const GTerm &t : e->h_terms_dev) {
     if (t.kind == P_EQ && t.tmask == 0 && t.tval != 0) continue;  // padding
     if (t.kind != P_EQ && __builtin_popcountll(t.tmask) != 2) return false;
     const int nb = __builtin_popcountll(t.tmask);
     bool merged = false;
-    if (t.kind == P_EQ && t.flip == t.tmask && (nb == 1 || (nb == 2 && __builtin_popcountll(t.tval) == 1)))
-      for (GcSrc &s : out) {
-        GTerm &u = s.t;
-        if (u.kind != P_EQ || u.flip != t.flip || u.tmask != t.tmask || u.tval != (t.tval ^ t.tmask) || u.sgn != t.sgn ||
-            u.cre != t.cre)
-          continue;
+    if (t.kind == P_EQ && t.flip == t.tmask && (nb == 1 || (nb == 2 && __builtin_popcountll(t.tval) == 1))) {
+      std::vector<size_t> &same = open[t.flip];
+      for (size_t i : same) {
+        GTerm &u = out[i].t;
+        if (u.kind != P_EQ || u.tval != (t.tval ^ t.tmask) || u.sgn != t.sgn || u.cre != t.cre) continue;
         if (nb == 1 && u.cim == t.cim) {
           u.kind = P_SAME;
           u.tmask = u.tval = 0;
           merged = true;
         } else if (nb == 2 && u.cim == -t.cim) {
-          s.sgi = (uint32_t)(u.sgn ^ u.tval);
+          out[i].sgi = (uint32_t)(u.sgn ^ u.tval);
           u.kind = P_DIFF;
           u.tval = 0;
           u.cim = -u.cim;
@@ -333,6 +334,8 @@ static bool gc_sources(const hphi_engine *e, std::vector<GcSrc> &out) {
         }
         if (merged) break;
       }
+      if (!merged) same.push_back(out.size());
+    }
     if (!merged) out.push_back(GcSrc{t, (uint32_t)t.sgn});
   }
   return true;
