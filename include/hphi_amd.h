@@ -115,19 +115,21 @@ int hphi_engine_info(const hphi_engine *e, uint64_t *dim, uint64_t *size21, uint
  *   "hi_p1_wgs_per_cu" 1..256 (first pass), "hi_fuse_copy" 0|1;
  *   block kernel (k > 1): "use_blk" 0|1, "blk_cpl2|4|8|16" columns per lane
  *   (1, 4 or k; 0 = default), "blk_tpb" 0|256|1024, "blk_wgs_per_cu" 0..64;
- *   canonical H·v by classes: "cls" -1|0|1 (-1: where it is the faster one, unless one of tpb, wgs_per_cu,
- *   lds21, c2_crank, c2_unroll or xcd_map is set, for k > 1 one of blk_tpb,
- *   blk_wgs_per_cu or blk_cpl of this k; read back: whether it is in use for
- *   k = 1), "cls_blocks" 0|1|2|4 (blocks per wave, 0 by size), "cls_wgs_per_cu" 1..256,
- *   "cls_order" -1|0|1 (units by class, or by index dealt to the XCDs one by one; -1:
- *   by index from 2^24 states on; set before the tables are built);
+ *   canonical H·v by classes: "cls" -1|0|1 (-1: where it is the faster one, unless
+ *   one of tpb, wgs_per_cu, lds21, c2_crank, c2_unroll or xcd_map is set, for
+ *   k > 1 one of blk_tpb, blk_wgs_per_cu or blk_cpl of this k; read back: whether
+ *   it is in use for k = 1), "cls_blocks" 0|1|2|4 (blocks per wave, 0 by size),
+ *   "cls_wgs_per_cu" 1..256, "cls_order" -1|0|1 (units by class, or by index
+ *   dealt to the XCDs one by one; -1: by index from 2^24 states on; set before
+ *   the tables are built);
  *   grand-canonical H·v in LDS tiles: "gc_tile" -1|0|1 (-1: where they are the
- *   faster ones, from 256 tiles on, unless a block-kernel knob is set; 1: every sector with 8
- *   tiles, set before the diagonal is built; read back: whether the engine has
- *   tiles in use);
- *   "cls_k1|2|4|8|16", "cls_blocks_k...", "gc_tile_k...", "use_blk_k2...": the same for calls of one
- *   block size, -2 as for the engine (the autotuner's choice; setting the
- *   engine's knob clears them); read back: whether that block size runs so;
+ *   faster ones, from 256 tiles on, unless a block-kernel knob is set; 1: every
+ *   sector with 8 tiles, set before the diagonal is built; read back: whether the
+ *   engine has tiles in use);
+ *   "cls_k1|2|4|8|16", "cls_blocks_k...", "gc_tile_k...", "use_blk_k2...": the
+ *   same for calls of one block size, -2 as for the engine (the autotuner's
+ *   choice; setting the engine's knob clears them); read back: whether that
+ *   block size runs so;
  *   LOBPCG: "lb_mfma" 0|1 (block-8 Gram matrices on the FP64 matrix cores). */
 int hphi_engine_tune(hphi_engine *e, const char *knob, int value);
 int hphi_engine_get_tune(const hphi_engine *e, const char *knob, int *value);
@@ -176,8 +178,9 @@ int hphi_mltply_block_dev(hphi_engine *e, int k, double *V0, const double *V1, d
  * loops, harnesses that forbid hipMalloc).  It calls no hipMalloc/hipFree:
  * up to 256 prdct partial sums go to the engine's pinned host buffer, as in
  * every call; more live in a fixed per-device array of 2^18 complex128 (4 MiB,
- * held until the process ends), so a launch of g workgroups needs g*k <= 2^18 (every default and tuned shape on <= 256 CUs
- * with <= 64 workgroups per CU); larger launches are rejected with an error.
+ * held until the process ends), so a launch of g workgroups needs g*k <= 2^18
+ * (every default and tuned shape on <= 256 CUs with <= 64 workgroups per CU);
+ * larger launches are rejected with an error.
  * hphi_sz and hphi_diagonalcalc must have run on the engine (no lazy build),
  * and the engine's device must be current.  It always runs in one pass
  * ("hi_split" does not apply).  Calls that overlap on one device share that
